@@ -148,6 +148,43 @@ def test_pack_unpack_round_trip(gpu, torch_mod, M, K):
     assert np.array_equal(back[:, : nb * 64], mant[:, : nb * 64])
 
 
+@pytest.mark.parametrize("M,K,offset", [(1, 64, 0), (65, 192, 0), (64, 256, 1), (127, 320, 7), (200, 1000, 3)])
+def test_pack_layout_bytes(gpu, torch_mod, M, K, offset):
+    """The GPU planes byte for byte against a numpy transpose, from sources at
+    any byte address (offset) with a ragged K, and back to such addresses."""
+    qk, torch = gpu, torch_mod
+    nb, nt = K // 64, (M + 63) // 64
+    nb4 = (nb + 3) // 4
+    mant, exps = qk.synth_planes(M, K, 50 + M, 0, 255)
+    say("pack layout", M, K, offset)
+    src = torch.empty(M * K + 16, dtype=torch.int8, device="cuda")[offset:offset + M * K]
+    src.copy_(torch.from_numpy(mant.reshape(-1)))
+    esrc = torch.empty(M * nb + 16, dtype=torch.uint8, device="cuda")[offset:offset + M * nb]
+    esrc.copy_(torch.from_numpy(np.ascontiguousarray(exps[:, :nb]).reshape(-1)))
+    dm = qk.DeviceMatrix.empty(M, K)
+    qk.check(qk.load().bfp8_dev_pack(dm.mant.data_ptr(), dm.exps.data_ptr(), src.data_ptr(), esrc.data_ptr(), M, K,
+                                     qk._stream()))
+    m = np.zeros((nt * 64, nb * 64), np.int8)
+    m[:M] = mant[:, :nb * 64]
+    want = m.reshape(nt, 64, nb, 4, 4, 4).transpose(0, 2, 5, 1, 3, 4).reshape(-1)  # [t][b][q][r][d][p]
+    e = np.zeros((nt * 64, nb4 * 4), np.uint8)
+    e[:M, :nb] = exps[:, :nb]
+    want_e = e.reshape(nt, 64, nb4, 4).transpose(0, 2, 1, 3).reshape(-1)
+    assert np.array_equal(dm.mant.cpu().numpy().reshape(-1).view(np.int8)[:want.size], want)
+    assert np.array_equal(dm.exps.cpu().numpy().reshape(-1).view(np.uint8)[:want_e.size], want_e)
+    back = torch.full((M * K + 16,), 5, dtype=torch.int8, device="cuda")
+    eback = torch.full((M * nb + 16,), 5, dtype=torch.uint8, device="cuda")
+    qk.check(qk.load().bfp8_dev_unpack(back[offset:].data_ptr(), eback[offset:].data_ptr(), dm.mant.data_ptr(),
+                                       dm.exps.data_ptr(), M, K, qk._stream()))
+    full = np.full(M * K + 16, 5, np.int8)
+    rows = full[offset:offset + M * K].reshape(M, K)
+    rows[:, :nb * 64] = mant[:, :nb * 64]
+    assert np.array_equal(back.cpu().numpy(), full)
+    efull = np.full(M * nb + 16, 5, np.uint8)
+    efull[offset:offset + M * nb] = np.ascontiguousarray(exps[:, :nb]).reshape(-1)
+    assert np.array_equal(eback.cpu().numpy(), efull)
+
+
 def test_gpu_synth_matches_host_synth(gpu, torch_mod):
     qk, torch = gpu, torch_mod
     M, K = 1000, 1024
