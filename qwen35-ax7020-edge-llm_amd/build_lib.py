@@ -11,7 +11,7 @@ Translation units:
   csrc/runtime_ftz.hip       decode runtime kernels (norms, conv, GDN, swiglu), f32 flush-to-zero
   csrc/fused_gemv.hip        the forward's GEMVs with their activation prologue, f32 flush-to-zero
   csrc/sweep.hip             a whole plan in one launch (a tile queue, LDS-quantized activations, in-launch top-k)
-  csrc/batch_mfma.hip        the batched GEMV (8..16 vectors) on the matrix cores, f32 flush-to-zero
+  csrc/batch_mfma.hip        the batched GEMV (up to 16 vectors) on the matrix cores, f32 flush-to-zero
   csrc/qwen_kernels_api.cpp  C ABI host code (include/qwen_kernels.h)
   csrc/qwen_runtime_api.cpp  C ABI of the runtime kernels and the forward loop
   csrc/qwen_weights.cpp      manifest-driven weight-image loader

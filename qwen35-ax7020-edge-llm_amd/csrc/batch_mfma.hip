@@ -1,4 +1,4 @@
-// batch_mfma.hip -- the batched BFP8 GEMV (8..16 activation vectors against
+// batch_mfma.hip -- the batched BFP8 GEMV (up to 16 activation vectors against
 // one weight matrix, weights read once) on the matrix cores, f32 flush-to-zero
 // like the reference's Advanced SIMD epilogue.
 //
@@ -29,17 +29,12 @@
 // and takes the two products otherwise; e < 8 (es = 0) and zero, infinite or
 // NaN scales give the same result either way.
 //
-// Work split: wavefront (s, g) takes a 64-row tile's 32-row half s and the
-// residues of group g (kRes residues per wavefront), keeping fs_q of its
-// residues; the wavefronts of a half combine their fs_q into y at the end
-// through LDS.  GEMVs with many tiles and K <= 1024: a workgroup per four
-// tiles, all 4 residues per wavefront (bfp8_gemv_batch_cu_kernel); with
-// larger K, a workgroup per tile, 2 residues per wavefront.  GEMVs with few
-// tiles: a workgroup per half, 1 residue per wavefront, every weight load of
-// a chunk in flight at once, and (more than 8 vectors) a workgroup per half
-// of the vectors too, so that more wavefronts, each with a shorter epilogue
-// chain, run on more CUs; with K <= 1024 each residue's blocks are split
-// over four wavefronts besides (bfp8_gemv_batch_split_kernel).
+// Work split: GEMVs with many tiles and K <= 1024, a workgroup per four tiles,
+// a wavefront per 32-row half with all 4 residues (bfp8_gemv_batch_cu_kernel);
+// with larger K, a workgroup per tile, a wavefront per half and two residues
+// (bfp8_gemv_batch_mfma_kernel); otherwise a workgroup of 16 wavefronts per half
+// and group of vectors, a wavefront per residue and quarter of the blocks
+// (bfp8_gemv_batch_span_kernel).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -56,9 +51,9 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kMfVec = 16;   // vectors (the MFMA's rows are vector x part)
 constexpr int kMfGroup = 2;  // blocks per weight-load group
 
-// CH: blocks of split activations staged in LDS at a time (16: the whole K of
-// the configured shapes in one staging; 8: half the LDS and the staging
-// registers, for the kernel whose occupancy they limit).
+// CH: blocks of split activations staged in LDS at a time (16: the whole K in
+// one staging; 8: half the LDS and the staging registers, for the kernel whose
+// occupancy they limit).
 template <int CH>
 struct MfLds {
     // A operands: [block][residue][k half][part][vector], 8 bytes each: the
@@ -66,8 +61,8 @@ struct MfLds {
     uint64_t xa[CH][4][64];
     float xs[CH][kMfVec];      // [block][vector] block scales
     int lo[CH], hi[CH];        // per block: e range of the one-product epilogue
-    // the end's exchange: 3 residue groups x 2 halves x 8 values x 64 lanes at most
-    static_assert(CH * 4 * 64 * sizeof(uint64_t) >= 3 * 2 * 8 * 64 * sizeof(float),
+    // the end's exchange: 2 halves x 2 residues x 8 values x 64 lanes
+    static_assert(CH * 4 * 64 * sizeof(uint64_t) >= 2 * 2 * 8 * 64 * sizeof(float),
                   "the fs exchange fits in the staging area");
 };
 
@@ -147,41 +142,34 @@ __device__ __forceinline__ void mf_stage_store(MfLds<CH>& L, const MfStaged<NT, 
     if (kSync) __syncthreads();
 }
 
+constexpr int kMfRes = 2;    // residues per wavefront of the workgroup-per-tile kernel
+constexpr int kMfDepth = 2;  // its weight-load groups in flight per wavefront
+constexpr int kMfChunk = 8;  // its blocks per staging
+
 // A lane's result slots: register i of the MFMA result (and i + 8, the low
-// parts) is vector 8(i/4) + 4*kh + i%4 of the lane's row; every vector: slots
-// i = 0..7; vector half kVH: slots i = 4 kVH .. 4 kVH + 3.
-template <int kVH>
-struct MfSlots {
-    static constexpr int n = kVH < 0 ? 8 : 4;
-    static constexpr int i0 = kVH < 0 ? 0 : 4 * kVH;
-};
-
-template <int kRes, int kVH>
+// parts) is vector 8(i/4) + 4*kh + i%4 of the lane's row, i = 0..7.
 struct MfState {
-    float fs[kRes][MfSlots<kVH>::n];  // [residue of the group][slot]
+    float fs[kMfRes][8];  // [residue of the group][slot]
 };
 
-template <int kRes>
 struct MfLoads {
-    uint64_t w[kMfGroup][kRes];  // [block][residue of the group]
+    uint64_t w[kMfGroup][kMfRes];  // [block][residue of the group]
     uint32_t e;
 };
 
 // One block: an MFMA per residue of the group and the epilogue.
-template <int kRes, int kVH, int CH>
-__device__ __forceinline__ void mf_block(MfState<kRes, kVH>& st, const MfLds<CH>& L, const uint64_t (&w)[kRes], uint32_t e,
+__device__ __forceinline__ void mf_block(MfState& st, const MfLds<kMfChunk>& L, const uint64_t (&w)[kMfRes], uint32_t e,
                                          int u, int q0, int lane) {
-    constexpr int NS = MfSlots<kVH>::n, I0 = MfSlots<kVH>::i0;
-    i32x16 d[kRes];
+    i32x16 d[kMfRes];
     const i32x16 zero = {};
 #pragma unroll
-    for (int r = 0; r < kRes; ++r)
+    for (int r = 0; r < kMfRes; ++r)
         d[r] = __builtin_amdgcn_mfma_i32_32x32x16_i8((long)L.xa[u][q0 + r][lane], (long)w[r], zero, 0, 0, 0);
     const int kh = lane >> 5;
-    float xs[NS];
+    float xs[8];
 #pragma unroll
-    for (int h = 0; h < NS / 4; ++h) {  // slots 4h..4h+3: vectors 8 (I0 / 4 + h) + 4 kh ..
-        const f32x4 x4 = *reinterpret_cast<const f32x4*>(&L.xs[u][8 * (I0 / 4 + h) + 4 * kh]);
+    for (int h = 0; h < 2; ++h) {  // slots 4h..4h+3: vectors 8h + 4 kh ..
+        const f32x4 x4 = *reinterpret_cast<const f32x4*>(&L.xs[u][8 * h + 4 * kh]);
 #pragma unroll
         for (int m = 0; m < 4; ++m) xs[4 * h + m] = x4[m];
     }
@@ -189,22 +177,22 @@ __device__ __forceinline__ void mf_block(MfState<kRes, kVH>& st, const MfLds<CH>
     const int lo = L.lo[u], hi = L.hi[u];
     const bool one_product = (e < 8u) | ((uint32_t)((int)e - lo) <= (uint32_t)(hi - lo));
     if (__builtin_amdgcn_ballot_w64(!one_product) == 0) {
-        float c[NS];
+        float c[8];
 #pragma unroll
-        for (int k = 0; k < NS; ++k) c[k] = es * xs[k];
+        for (int k = 0; k < 8; ++k) c[k] = es * xs[k];
 #pragma unroll
-        for (int r = 0; r < kRes; ++r)
+        for (int r = 0; r < kMfRes; ++r)
 #pragma unroll
-            for (int k = 0; k < NS; ++k) {
-                const int S = (int)((uint32_t)d[r][I0 + k] << 8) + d[r][I0 + k + 8];
+            for (int k = 0; k < 8; ++k) {
+                const int S = (int)((uint32_t)d[r][k] << 8) + d[r][k + 8];
                 st.fs[r][k] = st.fs[r][k] + (float)S * c[k];
             }
     } else {
 #pragma unroll
-        for (int r = 0; r < kRes; ++r)
+        for (int r = 0; r < kMfRes; ++r)
 #pragma unroll
-            for (int k = 0; k < NS; ++k) {
-                const int S = (int)((uint32_t)d[r][I0 + k] << 8) + d[r][I0 + k + 8];
+            for (int k = 0; k < 8; ++k) {
+                const int S = (int)((uint32_t)d[r][k] << 8) + d[r][k + 8];
                 const float t1 = (float)S * es;
                 st.fs[r][k] = st.fs[r][k] + t1 * xs[k];
             }
@@ -216,13 +204,12 @@ __device__ __forceinline__ void mf_block(MfState<kRes, kVH>& st, const MfLds<CH>
 // per dword).  The whole offset goes in the per-lane offset, which the buffer
 // range check covers: groups past the tile read zeros without touching memory.
 static_assert(4 % kMfGroup == 0, "a group's exponents share one dword");
-template <int kRes>
-__device__ __forceinline__ void mf_issue(MfLoads<kRes>& ld, __amdgpu_buffer_rsrc_t wrs, __amdgpu_buffer_rsrc_t ers, int wv,
+__device__ __forceinline__ void mf_issue(MfLoads& ld, __amdgpu_buffer_rsrc_t wrs, __amdgpu_buffer_rsrc_t ers, int wv,
                                          int ev, int gi) {
 #pragma unroll
     for (int uu = 0; uu < kMfGroup; ++uu)
 #pragma unroll
-        for (int r = 0; r < kRes; ++r) {
+        for (int r = 0; r < kMfRes; ++r) {
             const u32x2 v = __builtin_bit_cast(
                 u32x2, __builtin_amdgcn_raw_buffer_load_b64(wrs, wv + (gi * kMfGroup + uu) * 4096 + r * 1024, 0,
                                                             kNonTemporal));
@@ -231,94 +218,82 @@ __device__ __forceinline__ void mf_issue(MfLoads<kRes>& ld, __amdgpu_buffer_rsrc
     ld.e = load_e(ers, ev + (gi * kMfGroup / 4) * 256, 0);
 }
 
-template <int kRes, int NT, int kVH, int CH>
-__device__ __forceinline__ void mf_group(MfState<kRes, kVH>& st, MfLds<CH>& L, const MfLoads<kRes>& ld, int gi, int nb,
+constexpr int kMfThreads = 256;
+
+__device__ __forceinline__ void mf_group(MfState& st, MfLds<kMfChunk>& L, const MfLoads& ld, int gi, int nb,
                                          const uint32_t* __restrict__ xsplit, const float* __restrict__ xscale, int B,
                                          int q0, int lane) {
     const int b0 = gi * kMfGroup;
-    if (b0 % CH == 0 && b0 > 0) {  // the first chunk is staged before the loop
+    if (b0 % kMfChunk == 0 && b0 > 0) {  // the first chunk is staged before the loop
         __syncthreads();  // every wavefront is done with the previous chunk
-        MfStaged<NT, CH> S;
-        mf_stage_load<NT, kVH, CH>(S, xsplit, xscale, nb, B, b0, min(CH, nb - b0));
-        mf_stage_store<NT, CH>(L, S);
+        MfStaged<kMfThreads, kMfChunk> S;
+        mf_stage_load<kMfThreads, -1, kMfChunk>(S, xsplit, xscale, nb, B, b0, min(kMfChunk, nb - b0));
+        mf_stage_store<kMfThreads, kMfChunk>(L, S);
     }
 #pragma unroll
     for (int uu = 0; uu < kMfGroup; ++uu) {
         if (b0 + uu >= nb) break;
-        mf_block<kRes, kVH, CH>(st, L, ld.w[uu], (ld.e >> (8 * ((b0 + uu) & 3))) & 0xffu, (b0 + uu) % CH, q0, lane);
+        mf_block(st, L, ld.w[uu], (ld.e >> (8 * ((b0 + uu) & 3))) & 0xffu, (b0 + uu) % kMfChunk, q0, lane);
     }
 }
 
-// The work of one workgroup: tile t, its 32-row half s (kHalves == 1) or both
-// (kHalves == 2, wavefront w takes half w & 1), the residues of group grp,
-// the vectors of kVH (every vector, or one half of them).
-// kDepth: weight-load groups in flight per wavefront (2: one group computed
-// while the next loads; CH / kMfGroup: a chunk's every weight load issued at
-// once, for GEMVs with too few tiles to fill the memory system otherwise).
-template <int kRes, int kHalves, int kDepth, int kVH, int CH>
-__device__ __forceinline__ void mf_body(MfLds<CH>& L, float* __restrict__ Y, const uint32_t* __restrict__ xsplit,
+// The work of one wavefront: tile t, its 32-row half s, the residues of group
+// grp (two of them), all vectors.
+__device__ __forceinline__ void mf_body(MfLds<kMfChunk>& L, float* __restrict__ Y, const uint32_t* __restrict__ xsplit,
                                         const float* __restrict__ xscale, const uint8_t* __restrict__ mant,
                                         const uint8_t* __restrict__ exps, int M, int K, int B, int t, int s, int grp) {
-    constexpr int NS = MfSlots<kVH>::n, I0 = MfSlots<kVH>::i0;
     const int lane = threadIdx.x & 63;
-    const int q0 = grp * kRes;
+    const int q0 = grp * kMfRes;
     const int col = lane & 31, kh = lane >> 5;
     const int nb = K >> 6, nb4 = (nb + 3) >> 2;
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(mant + (size_t)t * nb * 4096u, (uint32_t)nb * 4096u);
     const __amdgpu_buffer_rsrc_t ers = make_rsrc(exps + (size_t)t * nb4 * 256u, (uint32_t)nb4 * 256u);
     const int wv = q0 * 1024 + (32 * s + col) * 16 + kh * 8;
     const int ev = (32 * s + col) * 4;
-    MfState<kRes, kVH> st;
+    MfState st;
 #pragma unroll
-    for (int r = 0; r < kRes; ++r)
+    for (int r = 0; r < kMfRes; ++r)
 #pragma unroll
-        for (int k = 0; k < NS; ++k) st.fs[r][k] = 0.0f;
+        for (int k = 0; k < 8; ++k) st.fs[r][k] = 0.0f;
     const int ng = (nb + kMfGroup - 1) / kMfGroup;
     // the first chunk's activation loads go out first, then the first
     // weight groups: the staging then waits for its own loads only (a
     // wavefront's loads complete in the order issued)
-    constexpr int NT = 64 * kHalves * (4 / kRes);
-    MfStaged<NT, CH> S0;
-    mf_stage_load<NT, kVH, CH>(S0, xsplit, xscale, nb, B, 0, min(CH, nb));
-    MfLoads<kRes> ld[kDepth];
+    MfStaged<kMfThreads, kMfChunk> S0;
+    mf_stage_load<kMfThreads, -1, kMfChunk>(S0, xsplit, xscale, nb, B, 0, min(kMfChunk, nb));
+    MfLoads ld[kMfDepth];
 #pragma unroll
-    for (int d = 0; d < kDepth; ++d) mf_issue<kRes>(ld[d], wrs, ers, wv, ev, d);
-    mf_stage_store<NT, CH>(L, S0);
-    for (int gi = 0; gi < ng; gi += kDepth) {
-        // kDepth load sets in turn: set d holds group gi + d, then gi + d + kDepth
+    for (int d = 0; d < kMfDepth; ++d) mf_issue(ld[d], wrs, ers, wv, ev, d);
+    mf_stage_store<kMfThreads, kMfChunk>(L, S0);
+    for (int gi = 0; gi < ng; gi += kMfDepth) {
+        // kMfDepth load sets in turn: set d holds group gi + d, then gi + d + kMfDepth
 #pragma unroll
-        for (int d = 0; d < kDepth; ++d) {
-            if (gi + d < ng) mf_group<kRes, NT, kVH, CH>(st, L, ld[d], gi + d, nb, xsplit, xscale, B, q0, lane);
-            mf_issue<kRes>(ld[d], wrs, ers, wv, ev, gi + d + kDepth);
+        for (int d = 0; d < kMfDepth; ++d) {
+            if (gi + d < ng) mf_group(st, L, ld[d], gi + d, nb, xsplit, xscale, B, q0, lane);
+            mf_issue(ld[d], wrs, ers, wv, ev, gi + d + kMfDepth);
         }
     }
-    float (&fs)[kRes][NS] = st.fs;
+    float (&fs)[kMfRes][8] = st.fs;
 
-    // y = (fs_0 + fs_2) + (fs_1 + fs_3): the other residue groups of the half
-    // hand their sums to group 0 through the (no longer needed) staging area
+    // y = (fs_0 + fs_2) + (fs_1 + fs_3): the second residue group of the half
+    // hands its sums to the first through the (no longer needed) staging area
     __syncthreads();
-    float* xch = reinterpret_cast<float*>(&L.xa[0][0][0]);  // [group - 1][half][residue][slot][lane]
+    float* xch = reinterpret_cast<float*>(&L.xa[0][0][0]);  // [half][residue][slot][lane]
     if (grp > 0) {
 #pragma unroll
-        for (int r = 0; r < kRes; ++r)
+        for (int r = 0; r < kMfRes; ++r)
 #pragma unroll
-            for (int k = 0; k < NS; ++k) xch[((((grp - 1) * 2 + s) * kRes + r) * NS + k) * 64 + lane] = fs[r][k];
+            for (int k = 0; k < 8; ++k) xch[((s * kMfRes + r) * 8 + k) * 64 + lane] = fs[r][k];
     }
     __syncthreads();
     if (grp == 0) {
         const int row = t * 64 + 32 * s + col;
         const int pair_rows = M & ~1;
 #pragma unroll
-        for (int k = 0; k < NS; ++k) {
-            float f[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int gq = q / kRes, rq = q % kRes;
-                f[q] = gq == 0 ? fs[rq][k] : xch[((((gq - 1) * 2 + s) * kRes + rq) * NS + k) * 64 + lane];
-            }
-            const int i = I0 + k;
-            const int v = 8 * (i / 4) + 4 * kh + (i % 4);
-            const float y = (f[0] + f[2]) + (f[1] + f[3]);
+        for (int k = 0; k < 8; ++k) {
+            const float f2 = xch[((s * kMfRes + 0) * 8 + k) * 64 + lane], f3 = xch[((s * kMfRes + 1) * 8 + k) * 64 + lane];
+            const int v = 8 * (k / 4) + 4 * kh + (k % 4);
+            const float y = (fs[0][k] + f2) + (fs[1][k] + f3);
             if (v < B && row < pair_rows) Y[(size_t)v * M + row] = y;
         }
     }
@@ -339,33 +314,34 @@ __device__ __forceinline__ void mf_body(MfLds<CH>& L, float* __restrict__ Y, con
 // would win every issue slot and leave the other to finish alone, so each
 // wavefront lowers its priority as it progresses (s_setprio 3 .. 0 over the
 // blocks): the one behind is served first.
+// Up to eight vectors finish four of the eight result slots per lane (NS = 4):
+// 65536 x 1024, B = 4 17.3 us (a dot-product kernel) -> 12.2 (NS = 8) -> 11.6.
 constexpr int kCuWaves = 8;
 constexpr int kCuMaxNb = 16;
 
+template <int NS>
 struct CuOps {
-    uint64_t a[4];  // MFMA A operands (split activations) per residue
-    f32x4 x0, x1;   // block scales of the lane's slots 0..3 and 4..7
+    uint64_t a[4];    // MFMA A operands (split activations) per residue
+    f32x4 x[NS / 4];  // block scales of the lane's slots 0..3 (and 4..7)
     int lo, hi;     // the block's one-product exponent range
 };
 
 // The epilogue of one block for the four residues (as mf_block's)
-__device__ __forceinline__ void cu_epilogue(float (&fs)[4][8], const i32x16 (&d)[4], const CuOps& o, uint32_t e) {
-    float xs[8];
+template <int NS>
+__device__ __forceinline__ void cu_epilogue(float (&fs)[4][NS], const i32x16 (&d)[4], const CuOps<NS>& o, uint32_t e) {
+    float xs[NS];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        xs[m] = o.x0[m];
-        xs[4 + m] = o.x1[m];
-    }
+    for (int m = 0; m < NS; ++m) xs[m] = o.x[m / 4][m % 4];
     const float es = exp_scale_ftz(e);
     const bool one_product = (e < 8u) | ((uint32_t)((int)e - o.lo) <= (uint32_t)(o.hi - o.lo));
     if (__builtin_amdgcn_ballot_w64(!one_product) == 0) {
-        float c[8];
+        float c[NS];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) c[k] = es * xs[k];
+        for (int k = 0; k < NS; ++k) c[k] = es * xs[k];
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
+            for (int k = 0; k < NS; ++k) {
                 const int S = (int)((uint32_t)d[r][k] << 8) + d[r][k + 8];
                 fs[r][k] = fs[r][k] + (float)S * c[k];
             }
@@ -373,7 +349,7 @@ __device__ __forceinline__ void cu_epilogue(float (&fs)[4][8], const i32x16 (&d)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
+            for (int k = 0; k < NS; ++k) {
                 const int S = (int)((uint32_t)d[r][k] << 8) + d[r][k + 8];
                 const float t1 = (float)S * es;
                 fs[r][k] = fs[r][k] + t1 * xs[k];
@@ -395,7 +371,7 @@ __device__ __forceinline__ void cu_priority(int u) {
         __builtin_amdgcn_s_setprio(0);
 }
 
-template <int kAhead>
+template <int kAhead, int NS>
 __global__ __launch_bounds__(64 * kCuWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 bfp8_gemv_batch_cu_kernel(float* __restrict__ Y, const uint32_t* __restrict__ xsplit, const float* __restrict__ xscale,
                           const uint8_t* __restrict__ mant, const uint8_t* __restrict__ exps, int M, int K, int B) {
@@ -412,7 +388,7 @@ bfp8_gemv_batch_cu_kernel(float* __restrict__ Y, const uint32_t* __restrict__ xs
     // weights (from HBM): a wavefront's loads complete in issue order, so the
     // staging then waits for its own round trip only
     MfStaged<NT, kCuMaxNb> S0;
-    mf_stage_load<NT, -1, kCuMaxNb>(S0, xsplit, xscale, nb, B, 0, nb);
+    mf_stage_load<NT, NS == 4 ? 0 : -1, kCuMaxNb>(S0, xsplit, xscale, nb, B, 0, nb);
     const __amdgpu_buffer_rsrc_t ers = make_rsrc(exps + (size_t)tt * nb4 * 256u, (uint32_t)nb4 * 256u);
     uint32_t ev[kCuMaxNb / 4];
 #pragma unroll
@@ -442,22 +418,22 @@ bfp8_gemv_batch_cu_kernel(float* __restrict__ Y, const uint32_t* __restrict__ xs
     asm volatile("" ::: "memory");
     if (!live) return;
 
-    float fs[4][8];
+    float fs[4][NS];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) fs[r][k] = 0.0f;
+        for (int k = 0; k < NS; ++k) fs[r][k] = 0.0f;
     const i32x16 zero = {};
     // block u's LDS operands are read behind block u - 1's MFMAs
-    auto ops = [&](CuOps& o, int u) {
+    auto ops = [&](CuOps<NS>& o, int u) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) o.a[q] = L.xa[u][q][lane];
-        o.x0 = *reinterpret_cast<const f32x4*>(&L.xs[u][4 * kh]);
-        o.x1 = *reinterpret_cast<const f32x4*>(&L.xs[u][8 + 4 * kh]);
+#pragma unroll
+        for (int h = 0; h < NS / 4; ++h) o.x[h] = *reinterpret_cast<const f32x4*>(&L.xs[u][8 * h + 4 * kh]);
         o.lo = L.lo[u];
         o.hi = L.hi[u];
     };
-    CuOps o[2];
+    CuOps<NS> o[2];
     ops(o[0], 0);
 #pragma unroll
     for (int u = 0; u < kCuMaxNb; ++u) {
@@ -478,227 +454,277 @@ bfp8_gemv_batch_cu_kernel(float* __restrict__ Y, const uint32_t* __restrict__ xs
     const int row = t * 64 + 32 * s + col;
     const int pair_rows = M & ~1;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < NS; ++k) {
         const int v = 8 * (k / 4) + 4 * kh + (k % 4);
         const float y = (fs[0][k] + fs[2][k]) + (fs[1][k] + fs[3][k]);
         if (v < B && row < pair_rows) __builtin_nontemporal_store(y, Y + (size_t)v * M + row);
     }
 }
 
-// The block's terms float(S) * es * xs of the lane's four result slots of
-// vector half kVH (one product where es * xs is normal for the batch, as
-// mf_block's)
-template <int kVH>
-__device__ __forceinline__ void half_terms(float (&tv)[4], const i32x16& d, f32x4 x4, int lo, int hi, uint32_t e) {
-    constexpr int I0 = 4 * kVH;
-    const float es = exp_scale_ftz(e);
-    const bool one_product = (e < 8u) | ((uint32_t)((int)e - lo) <= (uint32_t)(hi - lo));
-    if (__builtin_amdgcn_ballot_w64(!one_product) == 0) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float c = es * x4[k];
-            const int S = (int)((uint32_t)d[I0 + k] << 8) + d[I0 + k + 8];
-            tv[k] = (float)S * c;
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int S = (int)((uint32_t)d[I0 + k] << 8) + d[I0 + k + 8];
-            const float t1 = (float)S * es;
-            tv[k] = t1 * x4[k];
-        }
-    }
-}
-// ---- few tiles, K <= 1024: a workgroup per 32-row half and half of the vectors,
-// the blocks split over four wavefronts per residue ---------------------------
-// Few tiles leave about one wavefront per SIMD with a workgroup of four
-// (one per residue), so a wavefront's chain of sixteen blocks (LDS read, MFMA,
-// epilogue, each waiting for the last) set the time.  Here wavefront (q, j)
-// computes residue q's terms float(S) * es * xs of blocks 4j .. 4j + 3 only,
-// each block's MFMA issued before the previous block's terms; the terms of
-// blocks 4 .. 15 go through LDS to wavefront (q, 0), which adds all sixteen in
-// block order (the reference's chain, unchanged).  All blocks run, also past
-// nb (K < 1024): their weights, activations and scales read as zeros, so each
-// adds an exact +0 to a sum that is never -0.
-constexpr int kSplitParts = 4;
-struct SplitLds {
-    MfLds<kCuMaxNb> a;
-    f32x4 t[kSplitParts - 1][4][4][64];     // [group - 1][residue][block of the group][lane]: the 4 slots
-    float xch[3][4][64];                     // residues 1..3: [residue - 1][slot][lane]
+// ---- few tiles: a workgroup per 32-row half and group of vectors, each residue's
+// blocks in four spans, one per wavefront ----------------------------------------
+// Wavefront (q, j) computes residue q's terms of blocks jP .. jP + P - 1 (P =
+// kP, a multiple of 4: whole exponent dwords) and keeps them in registers.  The
+// in-order chain then visits the spans, j = 0 .. 3, one handing its sum to the
+// next through LDS; with K <= 1024 (kP = 4) the sixteen terms of a sum go
+// through LDS instead and wavefront (q, k) adds those of slot k, which needs
+// two barriers instead of four (3584 x 1024, B = 16: 4.65 us against 4.82).
+//
+// Bound by latency (launch, the staging's round trip, the chain) and, with
+// many vectors, by the epilogue's VALU work on the CUs that the launch
+// reaches, so a workgroup takes few vectors when there are few tiles.  Result
+// slot i < NS of a lane is MFMA row 4 * (lane / 32) + i: a workgroup of NS
+// slots serves 2 NS vectors, and the MFMA rows of no slot read another
+// vector's operand (their results are never used).
+//
+// Measured (us per call, back to back), against a dot-product kernel of four,
+// two or one vectors per launch (B < 8) and a wavefront per residue and chain
+// of all blocks (B >= 8, K > 1024) before: 2048 x 3584, B = 5 23.3 -> 7.0;
+// 2048 x 3584, B = 16 15.7 -> 8.7; 3584 x 1024, B = 7 15.5 -> 3.9; 16384 x 1024,
+// B = 4 8.7 -> 5.0; 16384 x 1024, B = 16 13.4 -> 9.4.
+constexpr int kSpanMaxNb = 64;
+template <int NS, int kP>
+struct SpanLds {
+    static constexpr int kV = 2 * NS, kNb = 4 * kP;
+    // A operands: [block][residue][k half][part][vector], 8 bytes each
+    __attribute__((aligned(16))) uint64_t xa[kNb][4][2][2][kV];
+    __attribute__((aligned(16))) float xs[kNb][kV];  // [block][vector] block scales
+    int2 range[kNb];            // per block: e range of the one-product epilogue
+    float chain[4][NS][64];     // [residue][slot][lane]: a span's sums for the next; at the end fs_q
+    float terms[4][NS][kP == 4 ? kNb : 1][64];  // kP = 4: [residue][slot][block][lane]
 };
 
-template <int kVH>
-__device__ __forceinline__ void split_body(SplitLds& L, float* __restrict__ Y, const uint32_t* __restrict__ xsplit,
-                                           const float* __restrict__ xscale, const uint8_t* __restrict__ mant,
-                                           const uint8_t* __restrict__ exps, int M, int K, int B, int t, int s, int q,
-                                           int j) {
-    constexpr int NT = 64 * 4 * kSplitParts;
-    const int lane = threadIdx.x & 63, col = lane & 31, kh = lane >> 5;
-    const int nb = K >> 6, nb4 = (nb + 3) >> 2;  // nb <= kCuMaxNb (host-checked)
-    // the staging of the half's split activations and scales (the workgroup's
-    // sixteen wavefronts together), its loads issued before the exponents'
-    // and the weights' so that the staging waits for them alone (loads
-    // complete in issue order)
-    MfStaged<NT, kCuMaxNb> S0;
-    mf_stage_load<NT, kVH, kCuMaxNb>(S0, xsplit, xscale, nb, B, 0, nb);
+template <int NS, int kP>
+__global__ __launch_bounds__(64 * 16) void bfp8_gemv_batch_span_kernel(
+    float* __restrict__ Y, const uint32_t* __restrict__ xsplit, const float* __restrict__ xscale,
+    const uint8_t* __restrict__ mant, const uint8_t* __restrict__ exps, int M, int K, int B, int ngroups) {
+    using Lds = SpanLds<NS, kP>;
+    constexpr int kV = Lds::kV, kNb = Lds::kNb, NT = 64 * 16;
+    constexpr bool kExchange = kP == 4;
+    __shared__ Lds L;
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, kh = lane >> 5;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = w & 3, j = w >> 2;
+    // the ngroups workgroups of a unit (tile, 32-row half) on one XCD (blocks
+    // go to the 8 XCDs in turn): the first reads the weights, the rest find
+    // them in that L2
+    const int a = (int)blockIdx.x / (8 * ngroups), ar = (int)blockIdx.x % (8 * ngroups);
+    const int unit = 8 * a + (ar & 7), v0 = (ar >> 3) * kV;
+    if (unit >= 2 * bfp8_ntiles(M)) return;  // the whole workgroup: no barrier is left waiting
+    const int t = unit >> 1, s = unit & 1;
+    const int nb = K >> 6, nb4 = (nb + 3) >> 2;  // nb <= kNb (host-checked)
+
+    // the group's split activations and scales (from L2) go out before the
+    // exponents and weights (loads complete in issue order); piece i = one
+    // part of one residue of one block of one vector, 16 bytes
+    constexpr int kItems = kNb * 8 * kV, kRounds = (kItems + NT - 1) / NT;
+    u32x4 xv[kRounds];
+#pragma unroll
+    for (int n = 0; n < kRounds; ++n) {
+        const int i = tid + n * NT;
+        const int v = v0 + i % kV, rp = (i / kV) % 8, b = i / (8 * kV);
+        xv[n] = u32x4{0u, 0u, 0u, 0u};
+        if (v < B && b < nb)
+            xv[n] = *reinterpret_cast<const u32x4*>(xsplit + ((size_t)v * nb + b) * BFP8_XSPLIT_WORDS_PER_BLOCK + rp * 4);
+    }
+    float xsv = 0.0f;  // scale tid: block tid / kV, vector tid % kV
+    static_assert(kNb * kV <= NT, "one scale per thread");
+    if (tid < kNb * kV && v0 + tid % kV < B && tid / kV < nb) xsv = xscale[(size_t)(v0 + tid % kV) * nb + tid / kV];
     const __amdgpu_buffer_rsrc_t ers = make_rsrc(exps + (size_t)t * nb4 * 256u, (uint32_t)nb4 * 256u);
-    const uint32_t ev = load_e(ers, (32 * s + col) * 4 + j * 256, 0);  // blocks 4j .. 4j + 3
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(mant + (size_t)t * nb * 4096u, (uint32_t)nb * 4096u);
     const int wv = q * 1024 + (32 * s + col) * 16 + kh * 8;
-    uint64_t wq[4];
+    uint32_t ev[kP / 4];
+    uint64_t wq[kP];  // blocks past the tile read zeros without touching memory
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const u32x2 v = __builtin_bit_cast(
-            u32x2, __builtin_amdgcn_raw_buffer_load_b64(wrs, wv + (4 * j + i) * 4096, 0, kNonTemporal));
+    for (int g = 0; g < kP / 4; ++g) ev[g] = load_e(ers, (32 * s + col) * 4 + (j * (kP / 4) + g) * 256, 0);
+#pragma unroll
+    for (int i = 0; i < kP; ++i) {
+        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wrs, wv + (kP * j + i) * 4096, 0, 0));
         wq[i] = ((uint64_t)v.y << 32) | v.x;
     }
-    mf_stage_store<NT, kCuMaxNb, false>(L.a, S0);
+#pragma unroll
+    for (int n = 0; n < kRounds; ++n) {
+        const int i = tid + n * NT;
+        const int v = i % kV, p = (i / kV) % 2, rq = (i / (2 * kV)) % 4, b = i / (8 * kV);
+        if (kItems % NT == 0 || i < kItems) {
+            L.xa[b][rq][0][p][v] = ((uint64_t)xv[n].y << 32) | xv[n].x;
+            L.xa[b][rq][1][p][v] = ((uint64_t)xv[n].w << 32) | xv[n].z;
+        }
+    }
+    if (tid < kNb * kV) {  // whole wavefronts, or whole groups of kV lanes
+        const int E = (int)((__float_as_uint(xsv) >> 23) & 0xffu);
+        const bool normal = E >= 1 && E <= 254;
+        int emin = normal ? E : 255, emax = normal ? E : 0;
+#pragma unroll
+        for (int m = 1; m < kV; m <<= 1) {
+            emin = min(emin, __shfl_xor(emin, m, 64));
+            emax = max(emax, __shfl_xor(emax, m, 64));
+        }
+        L.xs[tid / kV][tid % kV] = xsv;
+        if (tid % kV == 0) L.range[tid / kV] = make_int2(135 - emin, min(236, 388 - emax));
+    }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the staging is in LDS; the weight loads stay in flight
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    uint64_t a[4];
-    f32x4 x4[4];
-    int lo[4], hi[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int b = 4 * j + i;
-        a[i] = L.a.xa[b][q][lane];
-        x4[i] = *reinterpret_cast<const f32x4*>(&L.a.xs[b][8 * kVH + 4 * kh]);
-        lo[i] = L.a.lo[b];
-        hi[i] = L.a.hi[b];
-    }
+
+    // the span's terms
+    const int pa = col >> 4, va = ((col >> 2) & 1) * NS + min(col & 3, NS - 1);  // this lane's A row: part, vector
     const i32x16 zero = {};
-    float tv[4][4];
-    i32x16 d = __builtin_amdgcn_mfma_i32_32x32x16_i8((long)a[0], (long)wq[0], zero, 0, 0, 0);
+    float tv[kP][NS];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        i32x16 dn = zero;
-        if (i + 1 < 4) dn = __builtin_amdgcn_mfma_i32_32x32x16_i8((long)a[i + 1], (long)wq[i + 1], zero, 0, 0, 0);
-        half_terms<kVH>(tv[i], d, x4[i], lo[i], hi[i], (ev >> (8 * i)) & 0xffu);
-        d = dn;
-    }
-    if (j > 0) {
+    for (int i = 0; i < kP; ++i) {
+        const int b = kP * j + i;
+        const i32x16 d = __builtin_amdgcn_mfma_i32_32x32x16_i8((long)L.xa[b][q][kh][pa][va], (long)wq[i], zero, 0, 0, 0);
+        float xs[NS];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) L.t[j - 1][q][i][lane] = f32x4{tv[i][0], tv[i][1], tv[i][2], tv[i][3]};
-    }
-    __syncthreads();
-    float fs[4];
-    if (j == 0) {
-        f32x4 tg[kSplitParts - 1][4];  // every read out first, then the chain
+        for (int k = 0; k < NS; ++k) xs[k] = L.xs[b][kh * NS + k];
+        const int2 range = L.range[b];
+        const uint32_t e = (ev[i >> 2] >> (8 * (i & 3))) & 0xffu;
+        const float es = exp_scale_ftz(e);
+        const bool one_product = (e < 8u) | ((uint32_t)((int)e - range.x) <= (uint32_t)(range.y - range.x));
+        if (__builtin_amdgcn_ballot_w64(!one_product) == 0) {
 #pragma unroll
-        for (int g = 0; g < kSplitParts - 1; ++g)
+            for (int k = 0; k < NS; ++k) {
+                const float c = es * xs[k];
+                tv[i][k] = (float)((int)((uint32_t)d[k] << 8) + d[k + 8]) * c;
+            }
+        } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) tg[g][i] = L.t[g][q][i][lane];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            float f = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) f = f + tv[i][k];
-#pragma unroll
-            for (int g = 0; g < kSplitParts - 1; ++g)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) f = f + tg[g][i][k];
-            fs[k] = f;
-        }
-        if (q > 0) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) L.xch[q - 1][k][lane] = fs[k];
+            for (int k = 0; k < NS; ++k) {
+                const float t1 = (float)((int)((uint32_t)d[k] << 8) + d[k + 8]) * es;
+                tv[i][k] = t1 * xs[k];
+            }
         }
     }
-    __syncthreads();
-    if (j == 0 && q == 0) {
-        const int row = t * 64 + 32 * s + col;
-        const int pair_rows = M & ~1;
+
+    // the in-order chain (blocks past nb are in no sum)
+    if constexpr (kExchange) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float y = (fs[k] + L.xch[1][k][lane]) + (L.xch[0][k][lane] + L.xch[2][k][lane]);
-            const int v = 8 * kVH + 4 * kh + k;
-            if (v < B && row < pair_rows) __builtin_nontemporal_store(y, Y + (size_t)v * M + row);  // as the cu kernel's
+        for (int i = 0; i < kP; ++i)
+#pragma unroll
+            for (int k = 0; k < NS; ++k) L.terms[q][k][kP * j + i][lane] = tv[i][k];
+        __syncthreads();
+        if (j < NS) {  // slot j of residue q
+            float t[kNb], fs = 0.0f;
+#pragma unroll
+            for (int b = 0; b < kNb; ++b) t[b] = L.terms[q][j][b][lane];
+#pragma unroll
+            for (int b = 0; b < kNb; ++b)
+                if (b < nb) fs = fs + t[b];
+            L.chain[q][j][lane] = fs;
         }
+        __syncthreads();
+    } else {
+#pragma unroll
+        for (int turn = 0; turn < 4; ++turn) {
+            if (j == turn) {
+                float fs[NS];
+#pragma unroll
+                for (int k = 0; k < NS; ++k) fs[k] = turn ? L.chain[q][k][lane] : 0.0f;
+#pragma unroll
+                for (int i = 0; i < kP; ++i) {
+                    if (kP * turn + i < nb) {
+#pragma unroll
+                        for (int k = 0; k < NS; ++k) fs[k] = fs[k] + tv[i][k];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < NS; ++k) L.chain[q][k][lane] = fs[k];
+            }
+            __syncthreads();
+        }
+    }
+    if (w < NS) {  // wavefront w: slot w, y = (fs_0 + fs_2) + (fs_1 + fs_3)
+        const float y = (L.chain[0][w][lane] + L.chain[2][w][lane]) + (L.chain[1][w][lane] + L.chain[3][w][lane]);
+        const int row = t * 64 + 32 * s + col, v = v0 + kh * NS + w;
+        if (v < B && row < (M & ~1)) __builtin_nontemporal_store(y, Y + (size_t)v * M + row);
     }
 }
 
-// Blocks 16a + x and 16a + 8 + x (x < 8, the same XCD, so the second reads
-// the weights from its L2) take unit 8a + x's two vector halves; unit =
-// (tile, 32-row half); blocks past the last unit exit.
-__global__ __launch_bounds__(64 * 4 * kSplitParts) void bfp8_gemv_batch_split_kernel(
+template <int NS>
+hipError_t launch_span(float* Y, const uint32_t* xsplit, const float* xscale, const uint8_t* mant, const uint8_t* exps,
+                       int M, int K, int B, hipStream_t s) {
+    const int groups = (B + 2 * NS - 1) / (2 * NS);
+    const dim3 grid(8 * groups * ((2 * bfp8_ntiles(M) + 7) / 8)), block(64 * 16);
+    switch (((K >> 6) + 15) / 16) {
+        case 1: hipLaunchKernelGGL((bfp8_gemv_batch_span_kernel<NS, 4>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B, groups); break;
+        case 2: hipLaunchKernelGGL((bfp8_gemv_batch_span_kernel<NS, 8>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B, groups); break;
+        case 3: hipLaunchKernelGGL((bfp8_gemv_batch_span_kernel<NS, 12>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B, groups); break;
+        case 4: hipLaunchKernelGGL((bfp8_gemv_batch_span_kernel<NS, 16>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B, groups); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+// ---- many tiles, K > 1024: a workgroup per tile ---------------------------------
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void bfp8_gemv_batch_mfma_kernel(
     float* __restrict__ Y, const uint32_t* __restrict__ xsplit, const float* __restrict__ xscale,
     const uint8_t* __restrict__ mant, const uint8_t* __restrict__ exps, int M, int K, int B) {
-    __shared__ SplitLds L;
+    __shared__ MfLds<kMfChunk> L;
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int b = (int)blockIdx.x;
-    const int unit = 8 * (b >> 4) + (b & 7);
-    if (unit >= 2 * bfp8_ntiles(M)) return;  // the whole workgroup: no barrier is left waiting
-    if (((b >> 3) & 1) == 0)
-        split_body<0>(L, Y, xsplit, xscale, mant, exps, M, K, B, unit >> 1, unit & 1, w & 3, w >> 2);
-    else
-        split_body<1>(L, Y, xsplit, xscale, mant, exps, M, K, B, unit >> 1, unit & 1, w & 3, w >> 2);
-}
-
-// kHalves: halves of a tile per workgroup (2: both, workgroup per tile; 1:
-// workgroup per 32-row half, twice the workgroups for GEMVs with few tiles).
-// kSplit: 1, every vector in each workgroup; 2, a workgroup per half of the
-// vectors, each wavefront then finishing 4 of the 8 result slots of its
-// lanes -- half the epilogue per wavefront, on twice the wavefronts, for
-// GEMVs whose wavefronts are too few to hide the epilogue's latencies.  The
-// two workgroups of a unit are blocks 16a + x and 16a + 8 + x (x < 8), which
-// go to the same XCD (blocks are dealt to the 8 XCDs in turn), so the second
-// reads the unit's weights from that XCD's L2; unit 8a + x, blocks past the
-// last unit exit at once.
-template <int kRes, int kHalves, int kDepth, int kSplit, int CH>
-__global__ __launch_bounds__(64 * kHalves * (4 / kRes)) __attribute__((amdgpu_waves_per_eu(kSplit == 2 ? 2 : 4))) void
-bfp8_gemv_batch_mfma_kernel(float* __restrict__ Y, const uint32_t* __restrict__ xsplit,
-                            const float* __restrict__ xscale, const uint8_t* __restrict__ mant,
-                            const uint8_t* __restrict__ exps, int M, int K, int B) {
-    __shared__ MfLds<CH> L;
-    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int b = (int)blockIdx.x;
-    const int bid = kSplit == 2 ? 8 * (b >> 4) + (b & 7) : b;
-    const int nunits = kHalves == 2 ? bfp8_ntiles(M) : 2 * bfp8_ntiles(M);
-    if (kSplit == 2 && bid >= nunits) return;  // the grid's last 16 blocks may hold fewer units
-    // 32-row half, residue group, tile
-    const int s = kHalves == 2 ? (w & 1) : (bid & 1), grp = kHalves == 2 ? (w >> 1) : w;
-    const int t = kHalves == 2 ? bid : (bid >> 1);
-    if (kSplit == 1)
-        mf_body<kRes, kHalves, kDepth, -1, CH>(L, Y, xsplit, xscale, mant, exps, M, K, B, t, s, grp);
-    else if (((b >> 3) & 1) == 0)
-        mf_body<kRes, kHalves, kDepth, 0, CH>(L, Y, xsplit, xscale, mant, exps, M, K, B, t, s, grp);
-    else
-        mf_body<kRes, kHalves, kDepth, 1, CH>(L, Y, xsplit, xscale, mant, exps, M, K, B, t, s, grp);
+    mf_body(L, Y, xsplit, xscale, mant, exps, M, K, B, (int)blockIdx.x, w & 1, w >> 1);
 }
 
 }  // namespace
 
-hipError_t bfp8_launch_gemv_batch_mfma(float* Y, const uint32_t* xsplit, const float* xscale, const uint8_t* mant,
-                                       const uint8_t* exps, int M, int K, int B, hipStream_t s) {
+hipError_t bfp8_launch_gemv_batch(float* Y, const uint32_t* xsplit, const float* xscale, const uint8_t* mant,
+                                  const uint8_t* exps, int M, int K, int B, hipStream_t s) {
     const int nt = bfp8_ntiles(M);
     if (nt == 0) return hipSuccess;
     // a ragged K drops its last K % 64 elements, as every other GEMV path does
     // (nb = K / 64 blocks; the split activation's stride is nb blocks)
-    if (B < 1 || B > kMfVec || K < 64) return hipErrorInvalidValue;
-    // few tiles: a workgroup per 32-row half (and, above 8 vectors, per half
-    // of the vectors) so that more run; with K <= 1024 and above 8 vectors
-    // the blocks are split over four wavefronts per residue (3584 x 1024,
-    // B = 16: 5.5-5.7 us against 6.5-6.8 on one box), else one residue per
-    // wavefront, 16-block staging, all of a chunk's weight loads in flight.  Many tiles: a
-    // workgroup per four tiles, four residues per wavefront (K <= 1024; at
-    // 65536 x 1024, B = 16: 14.9-15.0 us against 18.4 for a workgroup per
-    // tile, on one box); beyond that, a workgroup per tile with 8-block staging.
-    if (nt < 512 && B > 8 && (K >> 6) <= kCuMaxNb)  // four wavefronts per residue, a workgroup per half of the vectors
-        hipLaunchKernelGGL(bfp8_gemv_batch_split_kernel, dim3(16 * ((2 * nt + 7) / 8)), dim3(64 * 4 * kSplitParts), 0, s,
-                           Y, xsplit, xscale, mant, exps, M, K, B);
-    else if (nt < 512 && B > 8)  // and a workgroup per half of the vectors: 2 nt units, 16 blocks per 8
-        hipLaunchKernelGGL((bfp8_gemv_batch_mfma_kernel<1, 1, 16 / kMfGroup, 2, 16>), dim3(16 * ((2 * nt + 7) / 8)),
-                           dim3(256), 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
-    else if (nt < 512)
-        hipLaunchKernelGGL((bfp8_gemv_batch_mfma_kernel<1, 1, 16 / kMfGroup, 1, 16>), dim3(2 * nt), dim3(256), 0, s,
-                           Y, xsplit, xscale, mant, exps, M, K, B);
-    else if ((K >> 6) <= kCuMaxNb)  // many tiles, K <= 1024: a workgroup per four tiles, two blocks ahead
-        hipLaunchKernelGGL((bfp8_gemv_batch_cu_kernel<2>), dim3((nt + kCuWaves / 2 - 1) / (kCuWaves / 2)),
-                           dim3(64 * kCuWaves), 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
-    else
-        hipLaunchKernelGGL((bfp8_gemv_batch_mfma_kernel<2, 2, 2, 1, 8>), dim3(nt), dim3(256), 0, s, Y, xsplit, xscale,
-                           mant, exps, M, K, B);
-    return hipGetLastError();
+    if (B < 1 || B > kMfVec || K < 64 || K > 64 * kSpanMaxNb) return hipErrorInvalidValue;
+    const int nb = K >> 6;
+    if (B == 1) {
+        // one vector is a plain GEMV: 2.8 us against the span kernel's 3.4 at
+        // 3584 x 1024, 3.7 against 6.6 at 2048 x 3584, 11.7 against 12.2 (a
+        // workgroup per four tiles) at 65536 x 1024
+        Bfp8GemvDesc d{};
+        d.mant = mant;
+        d.exps = exps;
+        d.xsplit = xsplit;
+        d.xscale = xscale;
+        d.y = Y;
+        d.M = M;
+        d.K = K;
+        d.pair_rows = M & ~1;
+        return bfp8_launch_gemv(d, s);
+    }
+    // Many tiles fill the chip with the weight stream and take the forms that
+    // read the weights once for all vectors; fewer take the span kernel.  The
+    // lines lie where the two cross (us at a number of tiles, span first):
+    // K = 1024, B = 2 6.8 / 9.0 at 469, 9.9 / 9.2 at 625; B = 8 7.9 / 8.7 at
+    // 352, 9.8 / 9.1 at 469; B = 16 9.6 / 11.3 at 256, 12.6 / 11.2 at 352.
+    // K = 2048, B = 8 25.2 / 25.8 at 782, 30.9 / 27.9 at 1024; B = 16 9.6 /
+    // 16.2 at 128, 20.9 / 19.5 at 375.  K = 3584, B = 4 41.6 / 44.8 at 1024; B = 8
+    // 26.6 / 29.7 at 375, 63.3 / 48.3 at 1024; B = 16 20.1 / 26.7 at 128, 33.5 /
+    // 27.4 at 256.
+    if (nb <= kCuMaxNb) {
+        const dim3 grid((nt + kCuWaves / 2 - 1) / (kCuWaves / 2)), block(64 * kCuWaves);
+        if (B > 8 && nt >= 304) {
+            hipLaunchKernelGGL((bfp8_gemv_batch_cu_kernel<2, 8>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
+            return hipGetLastError();
+        }
+        if (B <= 8 && nt >= (B > 4 ? 448 : 544)) {
+            hipLaunchKernelGGL((bfp8_gemv_batch_cu_kernel<2, 4>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
+            return hipGetLastError();
+        }
+    } else if (B > 4 && nt >= (B > 8 ? (nb > 32 ? 192 : 352) : (nb > 32 ? 416 : 832))) {
+        hipLaunchKernelGGL(bfp8_gemv_batch_mfma_kernel, dim3(nt), dim3(256), 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
+        return hipGetLastError();
+    }
+    // The fewest vectors per workgroup that still leave at most one workgroup
+    // per CU; beyond that every vector in as few workgroups as hold them, but
+    // with K > 2048 four at most (eight need 89 registers: one workgroup per CU
+    // instead of two; 16384 x 3584, B = 16: 36.6 us against 33.5).
+    const int units = 2 * nt, cus = bfp8_cu_count();
+    int ns = 1;
+    while (ns < 4 && units * ((B + 2 * ns - 1) / (2 * ns)) > cus) ns *= 2;
+    if (units * ((B + 2 * ns - 1) / (2 * ns)) > cus) ns = B <= 2 ? 1 : (B <= 4 || nb > 32) ? 2 : 4;
+    switch (ns) {
+        case 1: return launch_span<1>(Y, xsplit, xscale, mant, exps, M, K, B, s);
+        case 2: return launch_span<2>(Y, xsplit, xscale, mant, exps, M, K, B, s);
+        default: return launch_span<4>(Y, xsplit, xscale, mant, exps, M, K, B, s);
+    }
 }

@@ -39,7 +39,6 @@ typedef const __attribute__((address_space(4))) uint32_t* sgpr_u32_ptr;
 typedef const __attribute__((address_space(4))) float* sgpr_f32_ptr;
 
 constexpr int kChunk = 4;       // streamed blocks per load batch (4 KiB per wavefront)
-constexpr int kBatchChunk = 8;  // blocks per LDS-staged step of the batched kernel
 static_assert(kChunk == 4 || kChunk == 8, "a chunk spans one or two exponent words");
 // fs += (float(S) * EXP_SCALE[e]) * xscale   (three roundings, flush-to-zero)
 __device__ __forceinline__ float epilogue(float fs, int S, uint32_t e, float xs) {
@@ -660,123 +659,6 @@ extern "C" __global__ __launch_bounds__(kMergeWaves * 64) void bfp8_topk_merge_w
     topk_merge<kMergeWaves, 1, 8, true>(topk_args(d), PlainKeys{}, L);
 }
 
-// Batched GEMV: B activation vectors against one weight matrix, weights read
-// once.  Activations of a chunk of 8 blocks for all B vectors are staged in
-// LDS (wave-uniform broadcast reads); each lane keeps B residue accumulators.
-template <int B>
-__global__ __launch_bounds__(256) void bfp8_gemv_batch_kernel(float* __restrict__ Y,
-                                                              const uint32_t* __restrict__ xsplit,
-                                                              const float* __restrict__ xscale,
-                                                              const uint8_t* __restrict__ mant,
-                                                              const uint8_t* __restrict__ exps, int M,
-                                                              int K) {
-    __shared__ uint32_t xl[B * kBatchChunk * 32];
-    __shared__ float xsl[B * kBatchChunk];  // the chunk's block scales (LDS, like the split words: no scalar loads,
-                                            // whose out-of-order returns would make every LDS wait a full wait)
-    float* red = reinterpret_cast<float*>(xl);  // the cross-wave sums reuse the staging space (4 * 64 * B floats)
-    static_assert(kBatchChunk * 32 >= 4 * 64, "red fits in xl");
-    const int q = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int r = threadIdx.x & 63;
-    const int t = blockIdx.x;
-    const int nb = K >> 6;
-    // blockIdx.y: which B vectors of the call (a GEMV with fewer tiles than
-    // CUs spreads its vectors over several workgroups per tile)
-    Y += (size_t)blockIdx.y * B * M;
-    xsplit += (size_t)blockIdx.y * B * nb * 32;
-    xscale += (size_t)blockIdx.y * B * nb;
-    const int nb4 = (nb + 3) >> 2;
-    const uint8_t* mtile = mant + (size_t)t * nb * 4096u;
-    const uint8_t* etile = exps + (size_t)t * nb4 * 256u;
-    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(mtile, (uint32_t)nb * 4096u);
-    const __amdgpu_buffer_rsrc_t ers = make_rsrc(etile, (uint32_t)nb4 * 256u);
-    const int wv = q * 1024 + r * 16;
-    const int xwords = nb * 32;
-    float fs[B];
-#pragma unroll
-    for (int v = 0; v < B; ++v) fs[v] = 0.0f;
-
-    for (int b0 = 0; b0 < nb; b0 += kBatchChunk) {
-        const int nbc = min(kBatchChunk, nb - b0);
-        u32x4 w[kBatchChunk];
-        uint32_t ew[kBatchChunk / 4] = {};
-#pragma unroll
-        for (int u = 0; u < kBatchChunk; ++u)
-            if (u < nbc) w[u] = load_w(wrs, wv, (b0 + u) * 4096);
-#pragma unroll
-        for (int m = 0; m < kBatchChunk / 4; ++m)
-            if (4 * m < nbc) ew[m] = load_e(ers, r * 4, ((b0 >> 2) + m) * 256);
-        __syncthreads();  // previous chunk's LDS reads are done
-        for (int i = threadIdx.x; i < B * nbc * 32; i += 256) {
-            int v = i / (nbc * 32), o = i - v * nbc * 32;
-            xl[v * kBatchChunk * 32 + o] = xsplit[(size_t)v * xwords + b0 * 32 + o];
-        }
-        for (int i = threadIdx.x; i < B * nbc; i += 256) {
-            const int v = i / nbc, u = i - v * nbc;
-            xsl[v * kBatchChunk + u] = xscale[(size_t)v * nb + b0 + u];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < kBatchChunk; ++u) {
-            if (u >= nbc) break;
-            const uint32_t e = (ew[u >> 2] >> (8 * (u & 3))) & 0xffu;
-            const float sc = exp_scale_ftz(e);
-            // vectors in groups of four: the group's LDS reads go out together,
-            // then its four dot-product chains interleave
-            constexpr int kG = B < 4 ? B : 4;
-#pragma unroll
-            for (int v0 = 0; v0 < B; v0 += kG) {
-                uint4 h[kG], l[kG];
-                float xs[kG];
-#pragma unroll
-                for (int j = 0; j < kG; ++j) {
-                    const uint32_t* xb = xl + ((v0 + j) * kBatchChunk + u) * 32 + q * 8;
-                    h[j] = *reinterpret_cast<const uint4*>(xb);
-                    l[j] = *reinterpret_cast<const uint4*>(xb + 4);
-                    xs[j] = xsl[(v0 + j) * kBatchChunk + u];
-                }
-                int acc[kG];
-#pragma unroll
-                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].x, (int)h[j].x, 0, false);
-#pragma unroll
-                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].y, (int)h[j].y, acc[j], false);
-#pragma unroll
-                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].z, (int)h[j].z, acc[j], false);
-#pragma unroll
-                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].w, (int)h[j].w, acc[j], false);
-#pragma unroll
-                for (int j = 0; j < kG; ++j) {
-                    acc[j] = (int)((uint32_t)acc[j] << 8);
-                    acc[j] = __builtin_amdgcn_sdot4((int)w[u].x, (int)l[j].x, acc[j], false);
-                }
-#pragma unroll
-                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].y, (int)l[j].y, acc[j], false);
-#pragma unroll
-                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].z, (int)l[j].z, acc[j], false);
-#pragma unroll
-                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].w, (int)l[j].w, acc[j], false);
-#pragma unroll
-                for (int j = 0; j < kG; ++j) {
-                    const float t1 = (float)acc[j] * sc;
-                    const float t2 = t1 * xs[j];
-                    fs[v0 + j] = fs[v0 + j] + t2;
-                }
-            }
-        }
-    }
-    __syncthreads();  // every wavefront is done with the staged activations
-#pragma unroll
-    for (int v = 0; v < B; ++v) red[(v * 4 + q) * 64 + r] = fs[v];
-    __syncthreads();
-    const int pair_rows = M & ~1;
-    for (int i = threadIdx.x; i < B * 64; i += 256) {
-        int v = i >> 6, rr = i & 63;
-        int row = t * 64 + rr;
-        const float* p = red + v * 256;
-        float y = (p[rr] + p[128 + rr]) + (p[64 + rr] + p[192 + rr]);
-        if (row < pair_rows) Y[(size_t)v * M + row] = y;
-    }
-}
-
 // ---- launchers ---------------------------------------------------------------
 // Workgroups a persistent kernel keeps resident: all CUs times the kernel's
 // occupancy (capped at BFP8_STREAM_WG_PER_CU), queried once per kernel.
@@ -884,16 +766,7 @@ hipError_t bfp8_launch_gemv_wide_grouped(const Bfp8GemvDesc* descs_dev, const Bf
     return hipGetLastError();
 }
 
-template <int B>
-static hipError_t launch_batch_t(float* Y, const uint32_t* xsplit, const float* xscale,
-                                 const uint8_t* mant, const uint8_t* exps, int M, int K, int groups,
-                                 hipStream_t s) {
-    hipLaunchKernelGGL(bfp8_gemv_batch_kernel<B>, dim3(bfp8_ntiles(M), groups), dim3(256), 0, s, Y, xsplit,
-                       xscale, mant, exps, M, K);
-    return hipGetLastError();
-}
-
-static int cu_count() {
+int bfp8_cu_count() {
     static const int n = [] {
         int dev = 0, cus = 256;
         hipDeviceProp_t p;
@@ -901,40 +774,4 @@ static int cu_count() {
         return cus;
     }();
     return n;
-}
-
-// One launch of the dot-product kernel for B in {1, 2, 4}.
-static hipError_t launch_batch_pow2(float* Y, const uint32_t* xsplit, const float* xscale, const uint8_t* mant,
-                                    const uint8_t* exps, int M, int K, int B, hipStream_t s) {
-    const int nt = bfp8_ntiles(M);
-    // while the tiles leave CUs idle, split the vectors over more workgroups
-    // (each re-reads its tile's weights, from L2 / MALL for such small GEMVs)
-    int groups = 1;
-    while (groups * 2 <= B && nt * groups * 2 <= cu_count()) groups *= 2;
-    switch (B / groups) {
-        case 1: return launch_batch_t<1>(Y, xsplit, xscale, mant, exps, M, K, groups, s);
-        case 2: return launch_batch_t<2>(Y, xsplit, xscale, mant, exps, M, K, groups, s);
-        default: return launch_batch_t<4>(Y, xsplit, xscale, mant, exps, M, K, groups, s);
-    }
-}
-
-hipError_t bfp8_launch_gemv_batch(float* Y, const uint32_t* xsplit, const float* xscale,
-                                  const uint8_t* mant, const uint8_t* exps, int M, int K, int B,
-                                  hipStream_t s) {
-    if (bfp8_ntiles(M) == 0) return hipSuccess;
-    if (B < 1 || B > 16) return hipErrorInvalidValue;
-    // from 8 vectors on, the matrix cores: their epilogue costs the same for
-    // 8 and for 16 vectors, the dot-product kernel's grows with B
-    if (B >= 8) return bfp8_launch_gemv_batch_mfma(Y, xsplit, xscale, mant, exps, M, K, B, s);
-    const int nb = K >> 6;
-    int done = 0;
-    while (done < B) {
-        int step = 4;
-        while (step > B - done) step >>= 1;
-        const hipError_t e = launch_batch_pow2(Y + (size_t)done * M, xsplit + (size_t)done * nb * 32,
-                                               xscale + (size_t)done * nb, mant, exps, M, K, step, s);
-        if (e != hipSuccess) return e;
-        done += step;
-    }
-    return hipSuccess;
 }

@@ -68,6 +68,9 @@ extern "C" __global__ __launch_bounds__(64) void bfp8_tail_row_kernel(
     const int m = M - 1;
     const int nb = K >> 6;
     const int b = threadIdx.x;
+    y += (size_t)blockIdx.x * M;  // a workgroup per activation
+    xsplit += (size_t)blockIdx.x * nb * 32;
+    xscale += (size_t)blockIdx.x * nb;
     __shared__ float prod[64];
     float p = 0.0f;
     if (b < nb) {
@@ -364,10 +367,10 @@ hipError_t bfp8_launch_quantize1(const Bfp8QuantDesc& d, hipStream_t s) {
 }
 
 hipError_t bfp8_launch_tail_row(float* y, const uint32_t* xsplit, const float* xscale,
-                                const uint8_t* mant, const uint8_t* exps, int M, int K, hipStream_t s) {
-    if (M <= 0 || !(M & 1)) return hipSuccess;
+                                const uint8_t* mant, const uint8_t* exps, int M, int K, hipStream_t s, int nvec) {
+    if (M <= 0 || !(M & 1) || nvec <= 0) return hipSuccess;
     if (bfp8_nblocks(K) > 64) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(bfp8_tail_row_kernel, dim3(1), dim3(64), 0, s, y, xsplit, xscale, mant, exps, M, K);
+    hipLaunchKernelGGL(bfp8_tail_row_kernel, dim3(nvec), dim3(64), 0, s, y, xsplit, xscale, mant, exps, M, K);
     return hipGetLastError();
 }
 

@@ -205,15 +205,12 @@ int bfp8_sweep_grid(int per_cu);
 hipError_t bfp8_launch_sweep(const Bfp8SweepArgs& a, int nwg, hipStream_t s);
 // Y[v][M] for v < B (1..16): B split activations (rows of nb*32 words) and
 // scales (rows of nb floats); pair rows only (the odd last row is the tail
-// kernel's).  8..16 vectors run on the matrix cores (batch_mfma.hip), fewer
-// on the dot-product kernel, in power-of-two steps.
+// kernel's); K <= 4096.  One vector is a plain GEMV, more run on the matrix
+// cores (batch_mfma.hip).
 hipError_t bfp8_launch_gemv_batch(float* Y, const uint32_t* xsplit, const float* xscale,
                                   const uint8_t* mant, const uint8_t* exps, int M, int K, int B,
                                   hipStream_t s);
-
-// ---- batch_mfma.hip -------------------------------------------------------
-hipError_t bfp8_launch_gemv_batch_mfma(float* Y, const uint32_t* xsplit, const float* xscale, const uint8_t* mant,
-                                       const uint8_t* exps, int M, int K, int B, hipStream_t s);
+int bfp8_cu_count();
 
 // ---- bf16_head.hip --------------------------------------------------------
 hipError_t bf16_launch_lm_head(const Bf16HeadDesc& d, hipStream_t s);
@@ -252,8 +249,9 @@ hipError_t bfp8_launch_sample(const Bfp8SampleArgs& a, hipStream_t s);
 // ---- bfp8_ieee.hip -------------------------------------------------------
 hipError_t bfp8_launch_quantize(const Bfp8QuantDesc* descs_dev, int ndesc, int max_nb, hipStream_t s);
 hipError_t bfp8_launch_quantize1(const Bfp8QuantDesc& d, hipStream_t s);
-hipError_t bfp8_launch_tail_row(float* y, const uint32_t* xsplit, const float* xscale,
-                                const uint8_t* mant, const uint8_t* exps, int M, int K, hipStream_t s);
+// The odd last row of nvec activations (rows of y M floats apart, records of xsplit / xscale K / 64 blocks).
+hipError_t bfp8_launch_tail_row(float* y, const uint32_t* xsplit, const float* xscale, const uint8_t* mant,
+                                const uint8_t* exps, int M, int K, hipStream_t s, int nvec = 1);
 hipError_t bfp8_launch_gemv_float(float* y, const float* x, const uint8_t* mant, const uint8_t* exps,
                                   int M, int K, hipStream_t s);
 // The engine's numpy fallback (04/qwen_real_engine.py:1230-1238): unquantized

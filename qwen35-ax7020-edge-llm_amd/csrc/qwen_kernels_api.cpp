@@ -680,9 +680,9 @@ void bfp8_gemv_batch(float* Y, const float* X, const int8_t* mantissas, const ui
             rc = BFP8_EHIP;
         }
     }
-    for (int b = 0; !rc && b < B && (M & 1); ++b) {
-        hipError_t e = bfp8_launch_tail_row(g.y.as<float>() + (size_t)b * M, g.xsplit.as<uint32_t>() + (size_t)b * nb * 32,
-                                            g.xscale.as<float>() + (size_t)b * nb, w.mant, w.exps, M, K, g.stream);
+    if (!rc) {
+        hipError_t e = bfp8_launch_tail_row(g.y.as<float>(), g.xsplit.as<uint32_t>(), g.xscale.as<float>(), w.mant, w.exps,
+                                            M, K, g.stream, B);
         if (e != hipSuccess) {
             set_error("tail row launch: %s", hipGetErrorString(e));
             rc = BFP8_EHIP;
@@ -935,12 +935,8 @@ int bfp8_dev_gemv_batch(float* Y, const uint32_t* xsplit, const float* xscale, c
     if (M == 0) return BFP8_OK;
     DEV_PROLOGUE();
     hipStream_t s = pick_stream(stream);
-    const int nb = bfp8_nblocks(K);
     HIP_OK(bfp8_launch_gemv_batch(Y, xsplit, xscale, (const uint8_t*)mant_gpu, exps_gpu, M, K, B, s));
-    if (M & 1)
-        for (int b = 0; b < B; ++b)
-            HIP_OK(bfp8_launch_tail_row(Y + (size_t)b * M, xsplit + (size_t)b * nb * 32, xscale + (size_t)b * nb,
-                                        (const uint8_t*)mant_gpu, exps_gpu, M, K, s));
+    HIP_OK(bfp8_launch_tail_row(Y, xsplit, xscale, (const uint8_t*)mant_gpu, exps_gpu, M, K, s, B));
     return BFP8_OK;
 }
 

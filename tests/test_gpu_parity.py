@@ -903,6 +903,33 @@ def test_batch_odd_sizes(gpu, torch_mod):
         assert same_f32(Y[b], ol.gemv_neon(X[b], mant, exps)[0]), b
 
 
+@pytest.mark.parametrize("B,M,K", [(2, 65, 64), (5, 2049, 3584), (7, 100, 1088), (4, 33, 4096), (3, 200, 2112),
+                                   (16, 97, 3136), (9, 4100, 2049), (6, 28674, 320), (2, 34815, 128), (16, 19460, 64),
+                                   (5, 26623, 2112), (16, 12290, 2112), (1, 131, 1000)])
+def test_batch_dispatch_edges(gpu, torch_mod, B, M, K):
+    """Each form of the batched GEMV at the edges of its range: spans of 4, 8,
+    12 and 16 blocks per wavefront with the last span partly or wholly empty,
+    1, 2 and 4 result slots with idle vectors, row counts just past a tile and
+    a half tile, odd last rows, the first tile counts of the many-tile
+    kernels, and one vector (the plain GEMV).  Every exponent byte and block
+    scales from subnormal to huge (no value depends on how the work is split:
+    bit-exact against the restatement)."""
+    qk = gpu
+    rng = np.random.default_rng(B * 7919 + M)
+    nb = K // 64
+    mant = rng.integers(-128, 128, size=(M, K), dtype=np.int8)
+    exps = ((np.arange(M)[:, None] * 7 + np.arange(nb)[None, :] * 29) % 256).astype(np.uint8)
+    X = np.empty((B, K), dtype=F32)
+    for b in range(B):
+        X[b] = (rng.standard_normal(K) * 10.0 ** (-38 + 14 * (b % 6))).astype(F32)
+        X[b, (b % nb) * 64:(b % nb) * 64 + 64] = 0.0
+    say("batch dispatch edges", B, M, K)
+    Y = qk.Bfp8Kernels().gemv_batch(X, mant, exps, M, K)
+    for b in range(B):
+        y_ref, *_ = ol.gemv_neon(X[b], mant, exps)
+        assert same_f32(Y[b], y_ref), (B, M, K, b, mismatch(Y[b], y_ref))
+
+
 @pytest.mark.parametrize("with_head", [True, False])
 def test_sweep_plan_24_layers_and_lm_head(gpu, torch_mod, with_head):
     """The full synthetic decode sweep in one plan: 24 x {gate, up, down, in, out}
