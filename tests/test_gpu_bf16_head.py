@@ -196,6 +196,34 @@ def test_sampler_host_abi_matches_oracle(gpu):
         assert (got, st.value) == want, trial
 
 
+@pytest.mark.parametrize("n,order", [(1, "given"), (2, "tied"), (63, "given"), (64, "shuffled"), (64, "tied"), (64, "nan"),
+                                     (65, "given"), (1500, "shuffled")])
+def test_sampler_wavefront_and_workgroup_forms(gpu, n, order):
+    """Candidate counts on both sides of the one-wavefront form, lists of equal
+    scores and with NaN / infinite scores, every top_p and top_k edge: the
+    chosen id and the state as the oracle's."""
+    smp = gpu.load_sampling()
+    rng = np.random.default_rng(n * 10 + len(order))
+    sc = np.sort(rng.standard_normal(n).astype(F32) * F32(3.0))[::-1].copy()
+    if order == "shuffled":
+        rng.shuffle(sc)
+    elif order == "tied":
+        sc[:] = F32(-0.5)
+    elif order == "nan":
+        sc[0], sc[1], sc[-1] = np.nan, np.inf, -np.inf  # (in order: the comparator that sorts gives NaN no place)
+    ids = rng.permutation(70000)[:n].astype(np.int32)
+    say("sampler forms", n, order)
+    for temp, top_k, top_p in ((0.0, 0, 1.0), (0.7, 0, 0.9), (0.7, n, 1.0), (1.5, max(n - 1, 1), 0.999), (1.0, 1, 0.5),
+                               (0.01, 0, 0.3), (100.0, 0, 0.0), (0.7, 0, 2.0), (0.7, 50, 0.9)):
+        for state in (0, 1, int(rng.integers(0, 2**32))):
+            want = ol.sample_from_topk(ids, sc, temp, top_k, top_p, state)
+            st = ctypes.c_uint(state)
+            got = smp.sample_from_topk(ids.ctypes.data_as(ctypes.POINTER(ctypes.c_int)),
+                                       sc.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), n, temp, top_k, top_p,
+                                       ctypes.byref(st))
+            assert (got, st.value) == want, (n, order, temp, top_k, top_p, state)
+
+
 def test_device_topk_then_sample_chain(gpu, head_case):
     """lm_head top-64 and the draw stay on the device (the sampler reads the
     candidate count the merge wrote); the xorshift32 state advances on the
