@@ -4,13 +4,15 @@
 //   * per-tile top-k partials of a logits vector (k <= 64), merged by the
 //     stand-alone merge kernel of bfp8_ftz.hip: odd vocabularies, hidden
 //     sizes the fused launches do not take;
-//   * for k > 64 (04/qwen_sampling.c:283-353 returns min(k, vocab) entries
-//     for any k) the (score desc, id asc) keys sorted in 2048-key blocks in
+//   * for k from 65 to 512 of at most 65,536 logits the same lists of whole
+//     tiles, and one workgroup that takes the k best by threshold;
+//   * beyond (04/qwen_sampling.c:283-353 returns min(k, vocab) entries for any
+//     k) the (score desc, id asc) keys sorted in 2048-key blocks in
 //     LDS and registers, one workgroup each, then each block's first
 //     min(k, 2048) keys ranked against every block's (one bisection in LDS per
 //     candidate and block; keys are unique, so a key's rank is the count of
-//     keys above it).  At 65536 keys: 13.8 us of block sorts, then 5.5 us
-//     (k = 65) to 49 us (all keys) of ranking.  Beyond 2^20 keys one workgroup
+//     keys above it).  At 65536 keys: 13.8 us of block sorts, then 49 us (all
+//     keys) of ranking.  Beyond 2^20 keys one workgroup
 //     sorts them all in global memory (about 2 ms at 65536 keys);
 //   * sample_from_topk (04/qwen_sampling.c:384-529) for any candidate count.
 //
@@ -266,6 +268,177 @@ extern "C" __global__ __launch_bounds__(kSortThreads) void bfp8_select_rank_kern
         }
     }
 }
+// ---- 64 < k <= 512 of at most 65,536 logits ----------------------------------------
+// bfp8_select_partials_kernel sorts every 64-row tile on a wavefront of its own;
+// this one workgroup then takes the k best of the sorted lists by threshold.
+// A thread reads its list's key at depth d; wavefront w takes the c-th best of
+// its lists' (c = ceil(k / 16 (d + 1))), T is the lowest of the sixteen: every
+// wavefront has c lists with d + 1 keys >= T, so the k best are among the keys
+// >= T, which are prefixes of the lists -- about 1.7 k keys, gathered into LDS.
+// Where more than 1024 are left (equal scores, tiles in order), T is raised by
+// bisection on the keys until between k and 1024 are.  Ranks: each wavefront
+// sorts 64 of the gathered keys in registers, and a key's rank is its place in
+// its own list plus, by one bisection each, the keys above it in the others.
+//
+// Bound by latency: two launches, the lists' first reads, a dozen short steps
+// on one CU (which cannot look at every key: 50,001 logits in three passes of
+// one workgroup took 30.8 us).  The depth leaves a wavefront twice the lists
+// that it needs.  k = 200 of 50,001 logits: 3.4 + 7.9 us against 12.3 + 8.0 for
+// the block sort and rank above.
+namespace {
+
+constexpr int kThrWaves = 16, kThrThreads = 64 * kThrWaves;
+constexpr int kThrCap = 1024;  // keys gathered at most: one per thread
+constexpr int kThrMaxK = 512, kThrMaxN = 64 * kThrThreads;
+
+struct ThrLds {
+    uint64_t keys[kThrCap];
+    uint32_t thr[kThrWaves];  // per wavefront: the score of its c-th best key
+    int sum[kThrWaves];       // ... its keys gathered
+};
+
+}  // namespace
+
+extern "C" __global__ __launch_bounds__(kThrThreads) void bfp8_select_lists_kernel(
+    const uint64_t* __restrict__ keys, int n, int kk, int* __restrict__ ids, float* __restrict__ scores,
+    int* __restrict__ count, int* __restrict__ argmax) {
+    __shared__ ThrLds L;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // list lane * 16 + w: the wavefronts share the lists evenly, also few of them
+    const int nl = (n + 63) >> 6, l = lane * kThrWaves + w;
+    const int len = l < nl ? min(64, n - l * 64) : 0;
+    const uint64_t* list = keys + (size_t)l * 64;
+    auto at = [&](int i) { return i < len ? list[i] : 0ull; };
+    const int share = max(nl / kThrWaves, 1);                                      // lists of every wavefront
+    const int d = min((kk + 8 * share - 1) / (8 * share), 64) - 1;                 // depth
+    const int c = (kk + kThrWaves * (d + 1) - 1) / (kThrWaves * (d + 1));          // (<= 64: kk <= 512)
+    uint64_t head[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) head[i] = at(i);
+    const uint32_t deep = (uint32_t)(at(d) >> 32);
+    uint32_t best = deep;  // sorted over the lanes, descending
+#pragma unroll
+    for (int k = 2; k <= 64; k <<= 1)
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            const uint32_t o = xor_lane32(best, j);
+            best = ((lane & j) == 0) == ((lane & k) == 0) ? max(best, o) : min(best, o);
+        }
+    if (lane == c - 1) L.thr[w] = best;
+    __syncthreads();
+    uint32_t ts = L.thr[0];
+#pragma unroll
+    for (int i = 1; i < kThrWaves; ++i) ts = min(ts, L.thr[i]);
+    uint64_t T = max((uint64_t)ts << 32, (uint64_t)1);  // (0: no candidate)
+    // this list's keys >= t
+    auto prefix = [&](uint64_t t) {
+        int m = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m += head[i] >= t ? 1 : 0;
+        if (m == 4) {
+            uint64_t v[4];
+            do {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = at(m + i);
+                int more = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) more += v[i] >= t ? 1 : 0;
+                m += more;
+                if (more < 4) break;
+            } while (m < 64);
+        }
+        return m;
+    };
+    int mine = prefix(T), pos = mine;
+    // a lane's place among the keys: a scan in the wavefront, the wavefronts' sums
+    int base = 0;
+    auto scan = [&] {
+        pos = mine;
+#pragma unroll
+        for (int s = 1; s < 64; s <<= 1) {
+            const int up = __shfl_up(pos, s, 64);
+            if (lane >= s) pos += up;
+        }
+    };
+    auto total = [&] {
+        if (lane == 63) L.sum[w] = pos;
+        __syncthreads();
+        int v = 0;
+        base = pos - mine;
+#pragma unroll
+        for (int i = 0; i < kThrWaves; ++i) {
+            const int s = L.sum[i];
+            base += i < w ? s : 0;
+            v += s;
+        }
+        __syncthreads();
+        return v;
+    };
+    scan();
+    int S = total();
+    if (S > kThrCap) {  // uniform
+        // count(>= lo) > cap, count(>= hi) < kk; keys differ, so some T between keeps kk .. cap
+        uint64_t lo = T, hi = ~0ull;
+        while (S > kThrCap || S < kk) {
+            T = lo + (hi - lo) / 2;
+            mine = prefix(T);
+            scan();
+            S = total();
+            if (S > kThrCap)
+                lo = T;
+            else
+                hi = T;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (i < mine) L.keys[base + i] = head[i];
+    for (int i = 4; i < mine; ++i) L.keys[base + i] = list[i];
+    __syncthreads();
+    // 64 keys per wavefront sorted, then every key ranked against the lists
+    const int lists = (S + 63) >> 6;
+    uint64_t key[1] = {tid < S ? L.keys[tid] : 0ull};
+    if (w < lists) {
+        const bool desc[1] = {true};
+        wave_sort<1>(key, desc, lane);
+        L.keys[tid] = key[0];  // (a wavefront's own 64 places)
+    }
+    __syncthreads();
+    if (w < lists) {
+        int rank = lane;
+        for (int o0 = 0; o0 < lists; o0 += 4) {  // four bisections at a time
+            int m[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int step = 32; step > 0; step >>= 1)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {  // lists descend, keys differ, 0s last
+                    const uint64_t t = L.keys[64 * min(o0 + u, lists - 1) + m[u] + step - 1];
+                    m[u] += t > key[0] ? step : 0;
+                }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {  // m <= 63
+                const int o = o0 + u;
+                m[u] += L.keys[64 * min(o, lists - 1) + m[u]] > key[0] ? 1 : 0;
+                rank += o < lists && o != w ? m[u] : 0;
+            }
+        }
+        if (key[0] && rank < kk) {
+            ids[rank] = key_id(key[0]);
+            scores[rank] = key_score(key[0]);
+            if (rank == 0) *argmax = key_score(key[0]) > -1e30f ? key_id(key[0]) : 0;
+        }
+    }
+    const int cnt = min(kk, S);
+    for (int i = cnt + tid; i < kk; i += kThrThreads) {
+        ids[i] = -1;
+        scores[i] = 0.0f;
+    }
+    if (tid == 0) {
+        *count = cnt;
+        if (S == 0) *argmax = 0;
+    }
+}
+
 // keys[i] = the (score desc, id asc) key of logits[i] (0: not a candidate).
 extern "C" __global__ __launch_bounds__(256) void bfp8_select_keys_kernel(const float* __restrict__ logits, int n,
                                                                           uint64_t* __restrict__ keys) {
@@ -274,8 +447,10 @@ extern "C" __global__ __launch_bounds__(256) void bfp8_select_keys_kernel(const 
 
 // One wavefront per 64-row tile: its `topk` best keys, sorted, as the tile's
 // partial list ([ntiles][topk], 0-padded), which the merge kernel reads.
+// size: keys that fit partials (whole lists, or n for lists of all 64 rows).
 extern "C" __global__ __launch_bounds__(256) void bfp8_select_partials_kernel(const float* __restrict__ logits, int n,
-                                                                              int topk, uint64_t* __restrict__ partials) {
+                                                                              int topk, uint64_t* __restrict__ partials,
+                                                                              size_t size) {
     const int lane = threadIdx.x & 63;
     const int ntiles = (n + 63) >> 6;
     for (int t = blockIdx.x * 4 + (threadIdx.x >> 6); t < ntiles; t += gridDim.x * 4) {
@@ -283,7 +458,8 @@ extern "C" __global__ __launch_bounds__(256) void bfp8_select_partials_kernel(co
         uint64_t key[1] = {row < n ? topk_key(logits[row], row) : 0ull};
         const bool desc[1] = {true};
         wave_sort<1>(key, desc, lane);
-        if (lane < topk) partials[(size_t)t * topk + lane] = key[0];
+        const size_t at = (size_t)t * topk + lane;
+        if (lane < topk && at < size) partials[at] = key[0];
     }
 }
 
@@ -587,13 +763,22 @@ hipError_t bfp8_launch_select_partials(const float* logits, int n, int topk, uin
     if (n <= 0) return hipSuccess;
     if (topk < 1 || topk > BFP8_TOPK_MAX) return hipErrorInvalidValue;
     hipLaunchKernelGGL(bfp8_select_partials_kernel, dim3(select_grid(bfp8_ntiles(n), 4)), dim3(256), 0, s, logits, n,
-                       topk, partials);
+                       topk, partials, (size_t)bfp8_ntiles(n) * topk);
     return hipGetLastError();
 }
 
 hipError_t bfp8_launch_select_sort(const float* logits, int n, int kk, uint64_t* keys, int* ids, float* scores,
                                    int* count, int* argmax, hipStream_t s) {
     if (n <= 0 || kk < 1 || kk > n || n > BFP8_SELECT_MAX) return hipErrorInvalidValue;
+    if (n <= kThrMaxN && kk <= kThrMaxK) {
+        hipLaunchKernelGGL(bfp8_select_partials_kernel, dim3(select_grid(bfp8_ntiles(n), 4)), dim3(256), 0, s, logits, n, 64,
+                           keys, (size_t)n);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(bfp8_select_lists_kernel, dim3(1), dim3(kThrThreads), 0, s, keys, n, kk, ids, scores, count,
+                           argmax);
+        return hipGetLastError();
+    }
     if (n <= BFP8_SELECT_RANK_MAX) {
         const int nblk = (n + kSelBlock - 1) / kSelBlock;
         uint32_t* valid = reinterpret_cast<uint32_t*>(keys + n);

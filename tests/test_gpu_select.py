@@ -307,6 +307,48 @@ def test_bf16_device_lm_head_k_above_64(gpu, layout):
     assert int(cnt[1].item()) == ol.argmax(logits)
 
 
+@pytest.mark.parametrize("n,k", [(65, 65), (513, 512), (1000, 300), (2049, 65), (20000, 500), (65535, 512), (65536, 70)])
+@pytest.mark.parametrize("kind", ["random", "equal", "rising", "falling", "three", "few"])
+def test_top_k_of_sorted_tiles(gpu, n, k, kind):
+    """64 < k <= 512 of up to 65,536 scores, chosen one by one (hidden = 1, h = 1:
+    the scores are the table's bf16 values): scores whose tiles say little
+    about the threshold (all equal, in order, three values) and fewer
+    candidates than k (the rest NaN, -inf)."""
+    import torch
+
+    lib = gpu.load()
+    rng = np.random.default_rng(n + k)
+    sc = rng.standard_normal(n).astype(np.float32)
+    if kind == "equal":
+        sc[:] = 0.25
+    elif kind == "rising":
+        sc = np.sort(sc)
+    elif kind == "falling":
+        sc = np.sort(sc)[::-1].copy()
+    elif kind == "three":
+        sc = rng.choice(np.array([-1.0, 0.5, 2.0], np.float32), n)
+    elif kind == "few":
+        bad = rng.random(n) < 0.999
+        sc[bad] = rng.choice(np.array([np.nan, -np.inf], np.float32), int(bad.sum()))
+    table = torch.from_numpy(sc).to(torch.bfloat16).cuda()
+    sc = table.float().cpu().numpy()
+    one = torch.ones(1, dtype=torch.float32, device="cuda")
+    ids = torch.full((k,), 7, dtype=torch.int32, device="cuda")
+    out = torch.full((k,), 7, dtype=torch.float32, device="cuda")
+    cnt = torch.full((2,), 7, dtype=torch.int32, device="cuda")
+    say("top-k of sorted tiles", n, k, kind)
+    gpu.check(lib.bf16_dev_lm_head(ids.data_ptr(), out.data_ptr(), cnt.data_ptr(), cnt.data_ptr() + 4, None,
+                                   one.data_ptr(), table.data_ptr(), n, 1, k, 1, None))
+    torch.cuda.synchronize()
+    ok = np.nonzero(sc > -np.finfo(np.float32).max)[0]
+    best = ok[np.lexsort((ok, -sc[ok]))][:k]
+    want_ids, want_sc = np.full(k, -1, np.int32), np.zeros(k, np.float32)
+    want_ids[:len(best)], want_sc[:len(best)] = best, sc[best]
+    assert int(cnt[0].item()) == len(best)
+    assert np.array_equal(ids.cpu().numpy(), want_ids) and np.array_equal(out.cpu().numpy(), want_sc)
+    assert int(cnt[1].item()) == (best[0] if len(best) else 0)
+
+
 # ---- the sampler ---------------------------------------------------------------------------------
 @pytest.mark.parametrize("n,shuffled", [(5000, False), (5000, True), (20000, True), (4097, True)])
 def test_sampler_any_candidate_count(gpu, n, shuffled):
