@@ -266,6 +266,11 @@ size_t bfp8_device_bytes(void);
  * without an error channel (bfp8_gemv and the other void entry points),
  * aborts. */
 void bfp8_debug_device_limit(size_t bytes);
+/* Testing aid: the wait, in ticks of the GPU's 100 MHz clock, after which a
+ * launch of a run of layers gives up on its other workgroups and the forward
+ * calls repeat the run by separate launches (0: at the first vector that is
+ * not there yet; negative: the default, a quarter of a second). */
+void qwen_debug_chain_wait(long long ticks);
 
 /* ---- 3. device-level symbols ------------------------------------------------ */
 

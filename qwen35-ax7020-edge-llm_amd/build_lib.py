@@ -10,6 +10,7 @@ Translation units:
   csrc/bf16_head.hip         bf16 tied-embedding lm_head, f32 flush-to-zero
   csrc/runtime_ftz.hip       decode runtime kernels (norms, conv, GDN, swiglu), f32 flush-to-zero
   csrc/fused_gemv.hip        the forward's GEMVs with their activation prologue, f32 flush-to-zero
+  csrc/forward_chain.hip     a run of decode layers in one launch, f32 flush-to-zero
   csrc/sweep.hip             a whole plan in one launch (a tile queue, LDS-quantized activations, in-launch top-k)
   csrc/batch_mfma.hip        the batched GEMV (up to 16 vectors) on the matrix cores, f32 flush-to-zero
   csrc/qwen_kernels_api.cpp  C ABI host code (include/qwen_kernels.h)
@@ -47,6 +48,10 @@ UNITS = {
     "bf16_head.hip": ["-fgpu-flush-denormals-to-zero"],
     "runtime_ftz.hip": ["-fgpu-flush-denormals-to-zero"],
     "fused_gemv.hip": ["-fgpu-flush-denormals-to-zero"],
+    # (nothing hoisted out of the layer loop: with the doubles' constants and
+    # every address kept in registers across it the kernel spills)
+    "forward_chain.hip": ["-fgpu-flush-denormals-to-zero", "-mllvm", "-disable-machine-licm", "-mllvm",
+                          "-hoist-const-loads=false", "-mllvm", "-sink-insts-to-avoid-spills"],
     # (the ticket atomic stays one plain atomic: no wave-level combining,
     # whose result arithmetic would wait for every load in flight)
     "sweep.hip": ["-fgpu-flush-denormals-to-zero", "-mllvm", "-amdgpu-atomic-optimizer-strategy=None"],

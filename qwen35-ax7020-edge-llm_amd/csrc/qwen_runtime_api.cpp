@@ -90,8 +90,12 @@ struct ParamKey {
 };
 
 struct DevState {
-    DevBuf conv[2], rec;  // [3][6144] taps (the current one conv[cur]), [16][128*128] blocked state
-    int cur = 0;
+    // [3][6144] taps and [16][128*128] blocked state, the current ones conv[cur]
+    // and rec[rcur] (the separate launches update rec in place; rec[1] is there
+    // where the device holds it: the layer can run in a chain)
+    DevBuf buf;                              // all of them
+    float *conv[2], *rec[2] = {nullptr, nullptr};
+    int cur = 0, rcur = 0;
     float* host_conv;     // the caller's buffers
     float* host_rec;
     bool resident_used = false;  // advanced on the device while resident
@@ -109,6 +113,26 @@ struct FwdLayer {
     DevState* st = nullptr;
     // GPU planes: linear = qkv, z, o, gate, up, down; MLP = gate, up, down
     DevWeights w[6];
+    int slot = -1;  // in the chain's layer table (-1: runs as separate launches)
+};
+
+// Runs of layers in one launch (forward_chain.hip).
+constexpr uint64_t kChainWait = 25000000;  // 0.25 s of the 100 MHz clock: other streams' work may hold workgroups back
+struct Chain {
+    std::vector<RtChainLayer> host;  // the layer table
+    DevBuf layers;                   // ... its device copy, the first `uploaded` entries
+    size_t uploaded = 0;
+    DevBuf xch;                      // two sets of exchange words; each launch takes the other one and clears its predecessor's
+    int set = 0;                     // the clean set
+    int used[2] = {0, 0};            // words of each that are not clean
+    PinnedBuf io;                    // ChainIo
+    uint64_t wait_ticks = kChainWait;
+};
+// Host memory that the launches read and write.
+struct ChainIo {
+    float h_in[RT_HIDDEN], h_out[RT_HIDDEN];
+    int lm[4];        // [ids 1, scores 1, count, argmax]
+    uint32_t status;  // 1: the launch gave up
 };
 
 struct Workspace {
@@ -127,6 +151,7 @@ struct Forward {
     Workspace ws{};
     bool ws_ready = false;
     int resident = 0;
+    Chain chain;
 };
 
 Forward F;
@@ -221,29 +246,35 @@ int fwd_state(float* conv_s, float* state, DevState** out) {
         return BFP8_OK;
     }
     std::unique_ptr<DevState> st(new DevState());
-    int rc;
-    if ((rc = st->conv[0].reserve((size_t)3 * kConv * 4)) || (rc = st->conv[1].reserve((size_t)3 * kConv * 4)) ||
-        (rc = st->rec.reserve((size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM * 4)))
-        return rc;
+    constexpr size_t nc = (size_t)3 * kConv, nr = (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM;
+    const bool two = rt_chain_fits() && st->buf.reserve((2 * nc + 2 * nr) * 4) == BFP8_OK;
+    if (!two)
+        if (int rc = st->buf.reserve((2 * nc + nr) * 4)) return rc;
+    float* p = st->buf.as<float>();
+    st->rec[0] = p;
+    if (two) st->rec[1] = p + nr;
+    p += two ? 2 * nr : nr;
+    st->conv[0] = p;
+    st->conv[1] = p + nc;
     st->host_conv = conv_s;
     st->host_rec = state;
-    HIP_OK(hipMemcpy(st->conv[0].p, conv_s, (size_t)3 * kConv * 4, hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(st->rec.p, state, (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM * 4, hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(st->conv[0], conv_s, (size_t)3 * kConv * 4, hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(st->rec[0], state, (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM * 4, hipMemcpyHostToDevice));
     *out = st.get();
     F.states[key] = std::move(st);
     return BFP8_OK;
 }
 
 int state_in(DevState* st) {
-    HIP_OK(hipMemcpyAsync(st->conv[st->cur].p, st->host_conv, (size_t)3 * kConv * 4, hipMemcpyHostToDevice, g.stream));
-    HIP_OK(hipMemcpyAsync(st->rec.p, st->host_rec, (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM * 4,
+    HIP_OK(hipMemcpyAsync(st->conv[st->cur], st->host_conv, (size_t)3 * kConv * 4, hipMemcpyHostToDevice, g.stream));
+    HIP_OK(hipMemcpyAsync(st->rec[st->rcur], st->host_rec, (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM * 4,
                           hipMemcpyHostToDevice, g.stream));
     return BFP8_OK;
 }
 
 int state_out(DevState* st) {
-    HIP_OK(hipMemcpyAsync(st->host_conv, st->conv[st->cur].p, (size_t)3 * kConv * 4, hipMemcpyDeviceToHost, g.stream));
-    HIP_OK(hipMemcpyAsync(st->host_rec, st->rec.p, (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM * 4,
+    HIP_OK(hipMemcpyAsync(st->host_conv, st->conv[st->cur], (size_t)3 * kConv * 4, hipMemcpyDeviceToHost, g.stream));
+    HIP_OK(hipMemcpyAsync(st->host_rec, st->rec[st->rcur], (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM * 4,
                           hipMemcpyDeviceToHost, g.stream));
     return BFP8_OK;
 }
@@ -253,6 +284,61 @@ std::vector<char> key_of(const void* p, size_t n, char tag) {
     k[0] = tag;
     memcpy(k.data() + 1, p, n);
     return k;
+}
+
+// Enters a layer into the chain's table, where it fits (else slot stays -1).
+void chain_add(FwdLayer* L) {
+    Chain& c = F.chain;
+    if (!rt_chain_fits() || c.host.size() >= 0xffff) return;
+    RtChainLayer y{};
+    for (int i = 0; i < (L->linear ? 6 : 3); ++i) {
+        y.mant[L->linear ? i : 3 + i] = L->w[i].mant;
+        y.exps[L->linear ? i : 3 + i] = L->w[i].exps;
+    }
+    y.post_ln_w = L->post_ln_w;
+    if (L->linear) {
+        DevState* st = L->st;
+        if (!st->rec[1]) return;  // (no room: separate launches)
+        y.in_ln_w = L->in_ln_w;
+        y.conv_w = L->conv_w;
+        y.wa = L->wa;
+        y.wb = L->wb;
+        y.nea = L->nea;
+        y.dt = L->dt;
+        y.norm_w = L->norm_w;
+        for (int i = 0; i < 2; ++i) {
+            y.conv[i] = st->conv[i];
+            y.rec[i] = st->rec[i];
+        }
+        y.linear = 1;
+    }
+    constexpr size_t kSet = (size_t)RT_CHAIN_SET_WORDS * 8;
+    if (!c.xch.p) {
+        if (c.xch.reserve(2 * kSet) || hipMemsetAsync(c.xch.p, 0xff, 2 * kSet, g.stream) != hipSuccess) {
+            c.xch.release();
+            return;
+        }
+        c.used[0] = c.used[1] = 0;
+    }
+    if (c.io.reserve(sizeof(ChainIo))) return;
+    c.host.push_back(y);
+    L->slot = (int)c.host.size() - 1;
+}
+
+// The table's new entries to the device (no launch of this library is in
+// flight: its forward calls wait for theirs).
+int chain_upload() {
+    Chain& c = F.chain;
+    const size_t n = c.host.size(), bytes = n * sizeof(RtChainLayer);
+    if (c.uploaded == n) return BFP8_OK;
+    if (bytes > c.layers.n) {
+        c.uploaded = 0;
+        if (int rc = c.layers.reserve(std::max<size_t>(2 * bytes, 64 * sizeof(RtChainLayer)))) return rc;
+    }
+    HIP_OK(hipMemcpy(c.layers.as<RtChainLayer>() + c.uploaded, c.host.data() + c.uploaded,
+                     (n - c.uploaded) * sizeof(RtChainLayer), hipMemcpyHostToDevice));
+    c.uploaded = n;
+    return BFP8_OK;
 }
 
 int fwd_linear_layer(const LinearLayerPlan* p, FwdLayer** out) {
@@ -284,6 +370,7 @@ int fwd_linear_layer(const LinearLayerPlan* p, FwdLayer** out) {
         (rc = fwd_vec(p->dt, RT_HEADS, &L->dt)) || (rc = fwd_vec(p->norm_w, RT_HEAD_DIM, &L->norm_w)) ||
         (rc = fwd_vec(p->post_ln_w, kHidden, &L->post_ln_w)) || (rc = fwd_state(p->conv_s, p->state, &L->st)))
         return rc;
+    chain_add(L.get());
     *out = L.get();
     F.layers.emplace(key, std::move(L));
     return BFP8_OK;
@@ -312,6 +399,7 @@ int fwd_mlp_layer(const MlpPlan* p, FwdLayer** out) {
     for (int i = 0; i < 3; ++i)
         if ((rc = fwd_planes(m[i], e[i], Ms[i], Ks[i], &L->w[i]))) return rc;
     if ((rc = fwd_vec(p->post_ln_w, kHidden, &L->post_ln_w))) return rc;
+    chain_add(L.get());
     *out = L.get();
     F.layers.emplace(key, std::move(L));
     return BFP8_OK;
@@ -423,14 +511,14 @@ int linear_steps(const FwdLayer& L, float** h, const float* res) {
         RtLinearAttnArgs la{};
         la.qkv = w.qkv;
         la.normed = w.normed;
-        la.conv_in = st->conv[st->cur].as<float>();
-        la.conv_out = st->conv[st->cur ^ 1].as<float>();
+        la.conv_in = st->conv[st->cur];
+        la.conv_out = st->conv[st->cur ^ 1];
         la.conv_w = L.conv_w;
         la.wa = L.wa;
         la.wb = L.wb;
         la.nea = L.nea;
         la.dt = L.dt;
-        la.state = st->rec.as<float>();
+        la.state = st->rec[st->rcur];
         la.attn = w.attn;
         la.z = w.z;
         la.zsilu = w.zsilu;
@@ -532,16 +620,166 @@ int states_out(const std::vector<FwdLayer*>& layers) {
     return BFP8_OK;
 }
 
+// ---- runs of layers in one launch -------------------------------------------------------
+ChainIo& chain_io() { return *static_cast<ChainIo*>(F.chain.io.p); }
+
+// Every layer in the table, and no per-step profile asked for.
+bool chain_ok(const std::vector<FwdLayer*>& layers) {
+    if (g_prof_on) return false;
+    for (const FwdLayer* L : layers)
+        if (L->slot < 0) return false;
+    return chain_upload() == BFP8_OK;  // (no room for the table: separate launches)
+}
+
+// Layers [l, e) in one launch, from row `row` of the table (table != null) or
+// from io.h_in, the hidden state to io.h_out; with fnorm also its final norm
+// to ws.normed.  chain_done says whether it ran to its end.
+int chain_launch(const std::vector<FwdLayer*>& layers, int l, int e, const uint16_t* table, int ntiles, int row,
+                 const float* fnorm) {
+    Chain& c = F.chain;
+    ChainIo& io = chain_io();
+    RtChainArgs a{};
+    a.layers = c.layers.as<RtChainLayer>();
+    a.n = e - l;
+    for (int i = l; i < e; ++i) {
+        const FwdLayer* L = layers[i];
+        a.idx[i - l] = (uint16_t)L->slot;
+        if (L->linear) {
+            a.cur |= (uint32_t)L->st->cur << (i - l);
+            a.rcur |= (uint32_t)L->st->rcur << (i - l);
+        }
+    }
+    a.table = table;
+    a.ntiles = ntiles;
+    a.row = row;
+    a.h_in = io.h_in;
+    a.h_out = io.h_out;
+    a.final_w = fnorm;
+    a.y_norm = fnorm ? F.ws.normed : nullptr;
+    a.eps = 1e-6f;
+    uint64_t* sets = c.xch.as<uint64_t>();
+    a.xch = sets + (size_t)c.set * RT_CHAIN_SET_WORDS;
+    a.xch_clear = sets + (size_t)(c.set ^ 1) * RT_CHAIN_SET_WORDS;
+    a.clear_words = c.used[c.set ^ 1];
+    a.wait_ticks = c.wait_ticks;
+    a.status = &io.status;
+    io.status = 0;
+    RT_LAUNCH(rt_launch_chain(a, g.stream));
+    c.used[c.set] = a.n * RT_CHAIN_LAYER_WORDS + RT_HIDDEN / 2;
+    c.used[c.set ^ 1] = 0;
+    c.set ^= 1;
+    return BFP8_OK;
+}
+
+// After the stream is synchronized: the run's states become the current ones
+// (*ok), or it gave up, and nothing of it counts (!*ok).
+int chain_done(const std::vector<FwdLayer*>& layers, int l, int e, bool* ok) {
+    Chain& c = F.chain;
+    *ok = __atomic_load_n(&chain_io().status, __ATOMIC_ACQUIRE) == 0;
+    if (*ok) {
+        for (int i = l; i < e; ++i) {
+            if (!layers[i]->linear) continue;
+            layers[i]->st->cur ^= 1;
+            layers[i]->st->rcur ^= 1;
+        }
+        return BFP8_OK;
+    }
+    HIP_OK(hipMemsetAsync(c.xch.p, 0xff, 2 * (size_t)RT_CHAIN_SET_WORDS * 8, g.stream));
+    c.used[0] = c.used[1] = 0;
+    return BFP8_OK;
+}
+
 int layer_call(const FwdLayer& L, float* h, int slot) {
     const double t0 = g_prof_on ? now_ms() : 0.0;
     int rc;
     const std::vector<FwdLayer*> one{const_cast<FwdLayer*>(&L)};
+    if (chain_ok(one)) {
+        if ((rc = states_in(one))) return rc;
+        memcpy(chain_io().h_in, h, (size_t)kHidden * 4);
+        if ((rc = chain_launch(one, 0, 1, nullptr, 0, 0, nullptr))) return rc;
+        HIP_OK(hipStreamSynchronize(g.stream));
+        bool ok;
+        if ((rc = chain_done(one, 0, 1, &ok))) return rc;
+        if (ok) {
+            if ((rc = states_out(one))) return rc;
+            if (L.linear && !F.resident) HIP_OK(hipStreamSynchronize(g.stream));
+            memcpy(h, chain_io().h_out, (size_t)kHidden * 4);
+            return BFP8_OK;
+        }
+    }
     float* hd = F.ws.h;
     if ((rc = h_in(hd, h)) || (rc = states_in(one))) return rc;
     if ((rc = layer_steps(L, &hd, nullptr)) || (rc = add_pending(hd, F.ws.down))) return rc;
     if ((rc = states_out(one))) return rc;
     if ((rc = h_out(h, hd))) return rc;
     if (g_prof_on) g_prof_ms[slot] += now_ms() - t0;
+    return BFP8_OK;
+}
+
+// Layers [l, e) as separate launches from the hidden state in F.ws.h, which
+// ends, the last residual added, at *hd.
+int separate_steps(const std::vector<FwdLayer*>& layers, int l, int e, float** hd) {
+    const float* pending = nullptr;
+    int rc;
+    *hd = F.ws.h;
+    for (int i = l; i < e; ++i, pending = F.ws.down)
+        if ((rc = layer_steps(*layers[i], hd, pending))) return rc;
+    return add_pending(*hd, pending);
+}
+
+// forward_token_c's layers and head, the layers in runs of one launch: up to
+// the next full-attention layer whose callback edits the hidden state on the
+// host, or to the end.  A run that gives up is done again by separate launches.
+int token_chain(std::unique_lock<std::mutex>& lk, const std::vector<FwdLayer*>& layers, const int* layer_is_full,
+                FullAttnCallback cb, void* py_context, const uint16_t* table, int tiled, int row, const float* fnorm, float* h,
+                int* id) {
+    Workspace& w = F.ws;
+    const size_t hb = (size_t)kHidden * 4;
+    const int ntiles = tiled ? bfp8_ntiles(kVocab) : 0;
+    int rc;
+    if ((rc = states_in(layers))) return rc;
+    bool embed = true;  // the hidden state is still the table's row, else it is in h
+    for (int l = 0, e; l < kLayers; l = e) {
+        if (layer_is_full[l] && cb) {
+            if (embed) {
+                RT_LAUNCH(rt_launch_embed(w.h, table, ntiles, row, kHidden, g.stream));
+                if ((rc = h_out(h, w.h))) return rc;
+                embed = false;
+            }
+            lk.unlock();
+            cb(l, h, py_context);
+            lk.lock();
+        }
+        for (e = l + 1; e < kLayers && !(layer_is_full[e] && cb); ++e) {}
+        const bool last = e == kLayers;
+        ChainIo& io = chain_io();
+        auto head = [&] {
+            return bf16_lm_head_dev(io.lm, reinterpret_cast<float*>(io.lm + 1), io.lm + 2, io.lm + 3, nullptr, w.normed, table,
+                                    tiled, kVocab, kHidden, 1, 0, g.stream);
+        };
+        if (!embed) memcpy(io.h_in, h, hb);
+        if ((rc = chain_launch(layers, l, e, embed ? table : nullptr, ntiles, row, last ? fnorm : nullptr))) return rc;
+        if (last && (rc = head())) return rc;
+        HIP_OK(hipStreamSynchronize(g.stream));
+        bool ok;
+        if ((rc = chain_done(layers, l, e, &ok))) return rc;
+        if (ok) {
+            memcpy(h, io.h_out, hb);
+        } else {
+            float* hd;
+            if (embed)
+                RT_LAUNCH(rt_launch_embed(w.h, table, ntiles, row, kHidden, g.stream));
+            else if ((rc = h_in(w.h, h)))
+                return rc;
+            if ((rc = separate_steps(layers, l, e, &hd))) return rc;
+            if (last && ((rc = norm_step(hd, nullptr, fnorm, w.normed)) || (rc = head()))) return rc;
+            if ((rc = h_out(h, hd))) return rc;
+        }
+        embed = false;
+    }
+    *id = chain_io().lm[3];
+    if ((rc = states_out(layers))) return rc;
+    if (!F.resident) HIP_OK(hipStreamSynchronize(g.stream));
     return BFP8_OK;
 }
 
@@ -555,11 +793,13 @@ void drop_forward() {
     }
     F.planes.clear();
     for (auto& kv : F.states) {
-        kv.second->conv[0].release();
-        kv.second->conv[1].release();
-        kv.second->rec.release();
+        kv.second->buf.release();
     }
     F.states.clear();
+    F.chain.host.clear();
+    F.chain.uploaded = 0;
+    F.chain.layers.release();
+    F.chain.xch.release();
 }
 
 }  // namespace
@@ -810,13 +1050,19 @@ int forward_token_c(int token_id, float* h, const LinearLayerPlan* linear_plans,
     } else {
         RT_CHECK("forward_token_c", fwd_vec(embed_table, (size_t)kVocab * kHidden, &table));
     }
+    int row = token_id % kVocab;
+    if (row < 0) row += kVocab;
+    if (chain_ok(layers)) {
+        int id = 0;
+        RT_CHECK("forward_token_c", token_chain(lk, layers, layer_is_full, full_attn_cb, py_context, table, tiled, row, fnorm,
+                                                h, &id));
+        return id;
+    }
     Workspace& w = F.ws;
     float* hd = w.start_h2 ? w.h2 : w.h;  // the hidden state on the device
     RT_CHECK("forward_token_c", states_in(layers));
     {
         Step s(QP_EMBED);
-        int row = token_id % kVocab;
-        if (row < 0) row += kVocab;
         if (rt_launch_embed(hd, table, tiled ? bfp8_ntiles(kVocab) : 0, row, kHidden, g.stream) != hipSuccess) {
             set_error("embedding launch failed");
             fatal("forward_token_c");
@@ -862,6 +1108,11 @@ int forward_token_c(int token_id, float* h, const LinearLayerPlan* linear_plans,
     return out[3];
 }
 
+void qwen_debug_chain_wait(long long ticks) {
+    std::lock_guard<std::mutex> lk(g.mu);
+    F.chain.wait_ticks = ticks < 0 ? kChainWait : (uint64_t)ticks;
+}
+
 int qwen_forward_state_resident(int on) {
     std::lock_guard<std::mutex> lk(g.mu);
     const int prev = F.resident;
@@ -876,8 +1127,8 @@ void qwen_forward_reset_state(void) {
     for (auto& kv : F.states) {
         DevState* st = kv.second.get();
         // hipMemsetAsync is fine here: this call is never captured in a graph
-        if (hipMemsetAsync(st->conv[st->cur].p, 0, st->conv[st->cur].n, g.stream) != hipSuccess ||
-            hipMemsetAsync(st->rec.p, 0, st->rec.n, g.stream) != hipSuccess) {
+        if (hipMemsetAsync(st->conv[st->cur], 0, (size_t)3 * kConv * 4, g.stream) != hipSuccess ||
+            hipMemsetAsync(st->rec[st->rcur], 0, (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM * 4, g.stream) != hipSuccess) {
             set_error("state reset failed");
             fatal("qwen_forward_reset_state");
         }

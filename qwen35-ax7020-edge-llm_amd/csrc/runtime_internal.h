@@ -148,6 +148,41 @@ struct RtRowsArgs {
 };
 hipError_t rt_launch_rows(const RtRowsArgs& a, hipStream_t s);
 
+// A run of the forward's layers in one launch (forward_chain.hip).  Shapes are
+// the model's (hidden 1024, 16 heads of 128, MLP 3584).
+#define RT_CHAIN_WGS 256
+#define RT_CHAIN_MAX_LAYERS 24
+#define RT_CHAIN_LAYER_WORDS (512 + 512 + 3072 + 1024 + 1024 + 1024 + 1792 + 1792)
+#define RT_CHAIN_SET_WORDS (RT_CHAIN_MAX_LAYERS * RT_CHAIN_LAYER_WORDS + 512)  // 512: the hidden state handed in
+struct RtChainLayer {     // device memory
+    const uint8_t* mant[6];  // GPU planes: qkv, z, o, gate, up, down (an MLP layer: the last three)
+    const uint8_t* exps[6];
+    const float *in_ln_w, *conv_w, *wa, *wb, *nea, *dt, *norm_w, *post_ln_w;
+    float* conv[2];          // [3][6144] taps
+    float* rec[2];           // [16][128*128] blocked state
+    int linear, pad_;
+};
+struct RtChainArgs {
+    const RtChainLayer* layers;
+    uint16_t idx[RT_CHAIN_MAX_LAYERS];  // the run's layers
+    int n;
+    uint32_t cur, rcur;   // bit l: the current buffer of layer l's taps / state; the other one is written
+    const uint16_t* table;  // the run starts from row `row` of this embedding table (ntiles as in rt_launch_embed) ...
+    int ntiles, row;
+    const float* h_in;      // ... or from these 1024 floats
+    float* h_out;           // the hidden state after the run
+    const float* final_w;   // with y_norm: rmsnorm(h) with this weight
+    float* y_norm;          // optional
+    float eps;
+    uint64_t* xch;          // exchange words (RT_CHAIN_SET_WORDS), all ones
+    uint64_t* xch_clear;    // the other set: its first clear_words words are set to all ones
+    int clear_words;
+    uint64_t wait_ticks;    // of the 100 MHz clock, until a wait gives up
+    uint32_t* status;       // host memory: 1 when the launch gave up (nothing of it is to be used)
+};
+bool rt_chain_fits();
+hipError_t rt_launch_chain(const RtChainArgs& a, hipStream_t s);
+
 hipError_t rt_launch_rmsnorm(const RtNormArgs& a, hipStream_t s);
 hipError_t rt_launch_swiglu(const RtSwigluArgs& a, hipStream_t s);
 hipError_t rt_launch_conv1d(const RtConvArgs& a, hipStream_t s);

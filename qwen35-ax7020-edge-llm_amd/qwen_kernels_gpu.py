@@ -153,6 +153,8 @@ def bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.bfp8_device_bytes.restype = ctypes.c_size_t
     lib.bfp8_debug_device_limit.argtypes = [ctypes.c_size_t]
     lib.bfp8_debug_device_limit.restype = None
+    lib.qwen_debug_chain_wait.argtypes = [ctypes.c_longlong]
+    lib.qwen_debug_chain_wait.restype = None
     # device level
     for name in ("bfp8_dev_mant_bytes", "bfp8_dev_exps_bytes"):
         getattr(lib, name).argtypes = [i, i]

@@ -438,6 +438,54 @@ def test_forward_state_resident_mode(gpu, fresh_cache):
         lib.qwen_forward_state_resident(prev)
 
 
+@pytest.mark.parametrize("resident", [0, 1])
+def test_runs_of_layers_match_separate_launches(gpu, fresh_cache, resident):
+    """A token's and a layer's runs in one launch, the separate launches (as
+    while profiling), and runs that give up at once and are done again: the
+    same hidden states, ids and recurrent states, bit for bit, over calls that
+    alternate between the three, with the callback and without."""
+    lib = gpu.load()
+
+    def body(layer, hp, ctx):
+        h = np.ctypeslib.as_array(ctypes.cast(hp, ctypes.POINTER(ctypes.c_float)), shape=(1024,))
+        h += np.float32(0.01 * (layer + 1))
+
+    cb = gpu.FULL_ATTN_CALLBACK(body)
+    none = gpu.FULL_ATTN_CALLBACK()
+
+    def run(mode):
+        lib.bfp8_cache_clear()
+        m = Model(2031)
+        out = []
+        prev = lib.qwen_forward_state_resident(resident)
+        try:
+            for step, (token, c) in enumerate(((7, none), (65535, cb), (3, cb), (9, none), (12345, none))):
+                say("runs of layers", mode, resident, token)
+                separate = mode == "separate" or (mode == "mixed" and step % 2)
+                lib.qwen_prof_enable(1 if separate else 0)
+                lib.qwen_debug_chain_wait(0 if mode == "gives up" else -1)
+                h = np.zeros(1024, dtype=F32)
+                out.append(lib.forward_token_c(token, ptr(h), ctypes.addressof(m.gpu_lin), ctypes.addressof(m.gpu_mlp),
+                                               ptr(m.is_full), ptr(m.final_w), ptr(m.embed), c, None))
+                out.append(h)
+                h = h * np.float32(0.5)
+                lib.forward_linear_layer(ctypes.addressof(m.gpu_lin[step]), ptr(h))
+                lib.forward_mlp(ctypes.addressof(m.gpu_mlp[3]), ptr(h))
+                out.append(h)
+            lib.qwen_forward_sync_state()
+            return out + [a.copy() for st in m.gpu_states for a in st]
+        finally:
+            lib.qwen_prof_enable(0)
+            lib.qwen_debug_chain_wait(-1)
+            lib.qwen_forward_state_resident(prev)
+
+    want = run("separate")
+    for mode in ("one launch", "gives up", "mixed"):
+        got = run(mode)
+        for i, (a, b) in enumerate(zip(got, want)):
+            assert a == b if isinstance(a, int) else same(a, b), (mode, i)
+
+
 def test_profiler_slots(gpu, model):
     lib = gpu.load()
     assert lib.qwen_prof_count() == 15
