@@ -307,7 +307,8 @@ def test_bf16_device_lm_head_k_above_64(gpu, layout):
     assert int(cnt[1].item()) == ol.argmax(logits)
 
 
-@pytest.mark.parametrize("n,k", [(65, 65), (513, 512), (1000, 300), (2049, 65), (20000, 500), (65535, 512), (65536, 70)])
+@pytest.mark.parametrize("n,k", [(65, 65), (513, 512), (1000, 300), (1025, 500), (2049, 65), (4096, 400),
+                                 (8193, 512), (20000, 500), (33000, 512), (65535, 512), (65536, 70)])
 @pytest.mark.parametrize("kind", ["random", "equal", "rising", "falling", "three", "few"])
 def test_top_k_of_sorted_tiles(gpu, n, k, kind):
     """64 < k <= 512 of up to 65,536 scores, chosen one by one (hidden = 1, h = 1:
