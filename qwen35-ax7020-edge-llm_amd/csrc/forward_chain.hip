@@ -17,9 +17,20 @@
 //     other of two sets, which this one leaves cleared;
 //   * every workgroup keeps the hidden state in registers and computes each
 //     norm and activation itself, as the separate launches do;
-//   * weights and parameters are loaded into registers a step or more ahead,
-//     right after the inputs of the current step have arrived (a wavefront's
-//     loads complete in order: issued earlier they would hold up the inputs).
+//   * a ninth wavefront loads the weights a step or more ahead, into LDS.  In the
+//     others' registers they held up the exchange (a wavefront's loads complete
+//     in order), and so do any loads of the CU in flight: they go out where the
+//     workgroup computes (see loader);
+//   * the workgroup that has 16 rows of gate has those of up too and hands on
+//     their swiglu: half the words, and no workgroup computes all 3584.
+//
+// Bound by latency: a linear-attention layer is 21.2 us, of them 6.6 in five
+// exchanges, of which one between all workgroups takes 1.2 to 2.3 us (store,
+// memory-side cache, the last of 256 readers' polls) and one between a head's
+// 0.8; 2.9 in 824 dependent float adds, 8 cycles each, that the results' order
+// fixes; its 21.5 MB of weights would stream in 4.  Before the loader wavefront,
+// the pair of rows and 32-bit layer indices (16-bit ones are read by vector
+// loads): 24.0 us; a token's launch 517 us, now 438.
 //
 // Every operation and its order are those of the separate kernels (the GEMV
 // terms and block-order sums of fused_gemv.hip, the attention step of
@@ -43,23 +54,39 @@
 
 namespace {
 
-constexpr int kThreads = 512, kWaves = kThreads / 64;
+constexpr int kThreads = 512, kWaves = kThreads / 64;  // and one more wavefront, the loader
 constexpr int kMlpRows = 3584;
 constexpr int kHD = RT_HEADS * RT_HEAD_DIM;
 constexpr int kMaxNb = kMlpRows / 64;
 constexpr uint64_t kNotYet = ~0ull;
 // words of one layer's vectors
 constexpr int kWDown = 0, kWO = kWDown + RT_HIDDEN / 2, kWQkv = kWO + RT_HIDDEN / 2, kWZ = kWQkv + RT_CONV_CH / 2,
-              kWAttn = kWZ + kHD / 2, kWZs = kWAttn + kHD / 2, kWGate = kWZs + kHD / 2, kWUp = kWGate + kMlpRows / 2,
-              kWEnd = kWUp + kMlpRows / 2;
+              kWAttn = kWZ + kHD / 2, kWZs = kWAttn + kHD / 2, kWMlp = kWZs + kHD / 2, kWEnd = kWMlp + kMlpRows / 2;
 static_assert(kWEnd == RT_CHAIN_LAYER_WORDS, "exchange words of a layer");
 // the attention step's columns of a workgroup: 16 workgroups per head
 constexpr int kParts = RT_CHAIN_WGS / RT_HEADS, kCols = RT_HEAD_DIM / kParts;
 static_assert(kCols == 8 && kCols * RT_HEAD_DIM == 2 * kThreads, "two state elements per thread");
+constexpr int kWaitLoads = 0x0F70;             // s_waitcnt vmcnt(0)
 constexpr int kBigRows = 32;                  // rows per workgroup of the K = 1024 GEMVs
 constexpr int kBigPitch = 16 + 4, kSmallPitch = kMaxNb + 4;  // floats per chain of terms (16-byte rows)
 
+// Weights of 2 x 16 rows of K = 1024 (16 blocks) and the norm weights of their
+// activation.  Block b of half m: one load, lane = residue * 16 + row.
+struct BigLds {
+    u32x4 w[16][2][64];
+    uint32_t e[2][4][16];  // exponents of blocks 4i .. 4i + 3 of a row
+    float4 nw[RT_HIDDEN / 4];
+};
+// Weights of 4 rows of up to kMaxNb blocks.  Blocks 4j .. 4j + 3: one load, lane =
+// block * 16 + residue * 4 + row.
+struct SmallLds {
+    u32x4 w[kMaxNb / 4][64];
+    uint32_t e[16][4];
+};
+
 struct ChainLds {
+    BigLds big[2];  // a step's, the next one's
+    SmallLds small[2];
     __attribute__((aligned(16))) uint32_t xs[kMaxNb * 32];  // split activation records
     float xsc[kMaxNb];
     __attribute__((aligned(16))) float terms[4 * kBigRows * kBigPitch];
@@ -99,15 +126,18 @@ __device__ __forceinline__ void publish(uint64_t* p, float lo, float hi) {
 }
 
 // v[i] = *p[i], re-read until each has been written (lanes without `mine` read
-// nothing); false when the launch's time is up.
+// nothing, lanes that have all of theirs no more: every workgroup reads every
+// word past its L2, so re-reads get in the way of the stores they wait for);
+// false when the launch's time is up.
 template <int N>
 __device__ __forceinline__ bool await(uint64_t (&v)[N], const uint64_t* const (&p)[N], bool mine, uint64_t deadline) {
     for (int i = 0; i < N; ++i) v[i] = 0;
+    bool ok = !mine;
     for (uint32_t spin = 1;; ++spin) {
-        bool ok = true;
-        if (mine) {
+        if (!ok) {
 #pragma unroll
             for (int i = 0; i < N; ++i) v[i] = __hip_atomic_load(p[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ok = true;
 #pragma unroll
             for (int i = 0; i < N; ++i) ok &= v[i] != kNotYet;
         }
@@ -116,43 +146,46 @@ __device__ __forceinline__ bool await(uint64_t (&v)[N], const uint64_t* const (&
     }
 }
 
-// Weights of 32 rows (half s of tile t) of a K = 1024 GEMV: wavefront w blocks
-// 2w and 2w + 1; lane = row (lane & 31), residue 2p + lane / 32 of load p.
-struct BigW {
-    u32x4 w[2][2];
-    uint32_t e;  // the row's exponents of blocks 4(w / 2) ..
-};
-__device__ __forceinline__ void load_big(BigW& r, const uint8_t* mant, const uint8_t* exps, int half, int w, int lane) {
-    const int t = half >> 1, row = (half & 1) * 32 + (lane & 31);
-    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(mant + (size_t)t * 16 * 4096u, 16 * 4096u);
-    const __amdgpu_buffer_rsrc_t ers = make_rsrc(exps + (size_t)t * 4 * 256u, 4 * 256u);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-            r.w[i][p] = load_w(wrs, (2 * w + i) * 4096 + (2 * p + (lane >> 5)) * 1024 + row * 16, 0);
-    r.e = load_e(ers, (w >> 1) * 256 + row * 4, 0);
+// The loader's side of BigLds and SmallLds: loads straight into LDS (lane i's
+// piece goes to base + i * its size).
+__device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t rs, void* lds, int voff, int soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, kNonTemporal);
 }
-
-// Weights of 4 rows (sub-tile sub) of a GEMV of kNb blocks: lane = row (lane &
-// 3), residue (lane >> 2) & 3, block 4(w + 8i) + lane / 16 of load i.
-template <int kNb>
-struct SmallW {
-    static constexpr int kLd = (kNb / 4 + kWaves - 1) / kWaves;
-    u32x4 w[kLd];
-    uint32_t e[kLd];
-};
-template <int kNb>
-__device__ __forceinline__ void load_small(SmallW<kNb>& r, const uint8_t* mant, const uint8_t* exps, int sub, int w,
-                                           int lane) {
-    const int t = sub >> 4, row = (sub & 15) * 4 + (lane & 3), q = (lane >> 2) & 3;
-    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(mant + (size_t)t * kNb * 4096u, kNb * 4096u);
-    const __amdgpu_buffer_rsrc_t ers = make_rsrc(exps + (size_t)t * (kNb / 4) * 256u, (kNb / 4) * 256u);
+__device__ __forceinline__ void lds_load4(__amdgpu_buffer_rsrc_t rs, void* lds, int voff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)lds, 4, voff, 0, 0, 0);
+}
+// Blocks b0 .. b1 - 1 of rows 16 r0 .. and 16 r1 .. of two (or one) matrices of
+// 1024 columns, the norm weights and exponents with block 0.
+__device__ __forceinline__ void load_big(BigLds& L, const uint8_t* m0, const uint8_t* e0, int r0, const uint8_t* m1,
+                                         const uint8_t* e1, int r1, const float* nw, bool rows, int b0, int b1, int lane) {
+    const int at[2] = {(r0 & 3) * 16 + (lane & 15), (r1 & 3) * 16 + (lane & 15)};
+    if (b0 == 0) {
+        const __amdgpu_buffer_rsrc_t nr = make_rsrc(nw, RT_HIDDEN * 4);
 #pragma unroll
-    for (int i = 0; i < SmallW<kNb>::kLd; ++i) {  // (past the tile: zeros, no memory touched)
-        r.w[i] = load_w(wrs, ((w + kWaves * i) * 4 + (lane >> 4)) * 4096 + q * 1024 + row * 16, 0);
-        r.e[i] = load_e(ers, (w + kWaves * i) * 256 + row * 4, 0);
+        for (int i = 0; i < 4; ++i) lds_load16(nr, &L.nw[64 * i], lane * 16, i * 1024);
     }
+    if (!rows) return;
+    if (b0 == 0) {
+        const __amdgpu_buffer_rsrc_t er[2] = {make_rsrc(e0 + (size_t)(r0 >> 2) * 4 * 256u, 4 * 256u),
+                                              make_rsrc(e1 + (size_t)(r1 >> 2) * 4 * 256u, 4 * 256u)};
+#pragma unroll
+        for (int m = 0; m < 2; ++m) lds_load4(er[m], &L.e[m][0][0], (lane >> 4) * 256 + at[m] * 4);
+    }
+    const __amdgpu_buffer_rsrc_t wr[2] = {make_rsrc(m0 + (size_t)(r0 >> 2) * 16 * 4096u, 16 * 4096u),
+                                          make_rsrc(m1 + (size_t)(r1 >> 2) * 16 * 4096u, 16 * 4096u)};
+#pragma unroll 1
+    for (int b = b0; b < b1; ++b)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) lds_load16(wr[m], &L.w[b][m][0], (lane >> 4) * 1024 + at[m] * 16, b * 4096);
+}
+// Rows 4 sub .. of a matrix of nb blocks.
+__device__ __forceinline__ void load_small(SmallLds& L, const uint8_t* mant, const uint8_t* exps, int nb, int sub, int lane) {
+    const int t = sub >> 4, row = (sub & 15) * 4 + (lane & 3), q = (lane >> 2) & 3;
+    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(mant + (size_t)t * nb * 4096u, nb * 4096u);
+    const __amdgpu_buffer_rsrc_t ers = make_rsrc(exps + (size_t)t * (nb / 4) * 256u, (nb / 4) * 256u);
+    lds_load4(ers, &L.e[0][0], (lane >> 2) * 256 + row * 4);  // (past the tile: zeros, no memory touched)
+#pragma unroll 1
+    for (int j = 0; j < nb / 4; ++j) lds_load16(wrs, &L.w[j][0], (lane >> 4) * 4096 + q * 1024 + row * 16, j * 4 * 4096);
 }
 
 // The block's term (float(S) * 2^(e-134)) * xscale of one residue chunk.
@@ -194,27 +227,48 @@ __device__ __forceinline__ float chain_n(const float* p) {
     return s;
 }
 
-// Four swiglu elements (swiglu_elem's vector part): the float instructions
-// where everything is normal, else the exact helpers, in one place.
-__device__ __forceinline__ void swiglu4(float (&y)[4], const float (&gt)[4], const float (&up)[4]) {
-    uint32_t ok = 1;
+// swiglu_elem's vector part: the float instructions where everything is
+// normal, else the exact helpers.
+__device__ __forceinline__ float swiglu1(float gt, float up) {
+    const float d = 1.0f + exp_neon(-gt), r = __fdiv_rn(gt, d);
+    if (normal_u(gt) & normal_u(d) & normal_u(r)) return r * up;
+    return swiglu_elem(gt, up, true);
+}
+
+// One block of 64 elements quantized by 8 lanes, eight consecutive elements
+// per lane (bfp8_quant4_store_lds with a lane's elements 4 ii and 4 ii + 4 as one
+// 16-bit store).  ii: the lane's place among the eight.
+__device__ __forceinline__ void quant8_store_lds(const float (&x)[8], int ii, float* xscale_b, uint32_t* xsplit_b) {
+    float v = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float aj = fabsf(x[j]);
+        v = fmaxf(v, (aj > 0.0f) ? aj : 0.0f);  // a NaN never wins `v > amax`
+    }
+    int m = __float_as_int(v);
+    m = max(m, __builtin_amdgcn_mov_dpp(m, 0xB1, 0xF, 0xF, false));
+    m = max(m, __builtin_amdgcn_mov_dpp(m, 0x4E, 0xF, 0xF, false));
+    m = max(m, __builtin_amdgcn_mov_dpp(m, 0x141, 0xF, 0xF, false));
+    const float amax = __int_as_float(m);
+    const bool live = amax > 1e-20f;
+    const float q = __fdiv_rn(16384.0f, live ? amax : 1.0f);
+    typedef __attribute__((address_space(3))) uint16_t lds_u16;
+    typedef __attribute__((address_space(3))) float lds_f32;
+    lds_u16* rb = (lds_u16*)xsplit_b;
+    if (ii == 0) *(lds_f32*)xscale_b = live ? amax * 0x1p-14f : 0.0f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float d = 1.0f + exp_neon(-gt[j]), r = __fdiv_rn(gt[j], d);
-        ok &= normal_u(gt[j]) & normal_u(d) & normal_u(r);
-        y[j] = r * up[j];
-    }
-    if (!ok) {
-#pragma unroll 1
-        for (int j = 0; j < 4; ++j) {
-            const float gj = j == 0 ? gt[0] : j == 1 ? gt[1] : j == 2 ? gt[2] : gt[3];
-            const float uj = j == 0 ? up[0] : j == 1 ? up[1] : j == 2 ? up[2] : up[3];
-            const float v = swiglu_elem(gj, uj, true);
-            y[0] = j == 0 ? v : y[0];
-            y[1] = j == 1 ? v : y[1];
-            y[2] = j == 2 ? v : y[2];
-            y[3] = j == 3 ? v : y[3];
+        uint32_t hi = 0, lo = 0;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const float p = __fmul_rn(x[j + 4 * t], q);
+            const int xq = (int)__builtin_rintf((live && p == p) ? p : 0.0f);
+            const int xl = (int)(int8_t)(xq & 0xff);
+            lo |= (uint32_t)(xl & 0xff) << (8 * t);
+            hi |= (uint32_t)(((xq - xl) >> 8) & 0xff) << (8 * t);
         }
+        rb[j * 16 + ii] = (uint16_t)hi;
+        rb[j * 16 + 8 + ii] = (uint16_t)lo;
     }
 }
 
@@ -243,16 +297,15 @@ __device__ __forceinline__ void gated4(float (&y)[4], const float (&x)[4], float
     }
 }
 
-__device__ __forceinline__ void big_terms(ChainLds& L, const BigW& W, int w, int lane) {
+__device__ __forceinline__ void big_terms(ChainLds& L, const BigLds& W, int w, int lane) {
+    const int row = lane & 15, q = lane >> 4;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int b = 2 * w + i;
-        const uint32_t e = (W.e >> (8 * (b & 3))) & 0xffu;
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const int q = 2 * p + (lane >> 5);
-            L.terms[(q * kBigRows + (lane & 31)) * kBigPitch + b] = chunk_term(L, W.w[i][p], b, q, e);
-        }
+        for (int m = 0; m < 2; ++m)
+            L.terms[(q * kBigRows + 16 * m + row) * kBigPitch + b] =
+                chunk_term(L, W.w[b][m][lane], b, q, (W.e[m][b >> 2][row] >> (8 * (b & 3))) & 0xffu);
     }
 }
 // Wavefronts 0 and 1: rows 16w .. 16w + 15, lane = residue * 16 + row; the
@@ -266,13 +319,30 @@ __device__ __forceinline__ void big_sums(const ChainLds& L, uint64_t* out, int w
     if (lane < 8) publish(out + 8 * w + lane, lo, hi);
 }
 
+// Wavefront 0, the halves being 16 rows of gate and up: swiglu of the 16 rows.
+__device__ __forceinline__ void mlp_sums(const ChainLds& L, uint64_t* out, int lane) {
+    const int q = lane >> 4, r = lane & 15;
+    float y[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        const float fs = chain_n<16>(&L.terms[(q * kBigRows + 16 * m + r) * kBigPitch]);
+        const float f0 = __shfl(fs, r, 64), f1 = __shfl(fs, 16 + r, 64), f2 = __shfl(fs, 32 + r, 64), f3 = __shfl(fs, 48 + r, 64);
+        y[m] = (f0 + f2) + (f1 + f3);
+    }
+    const float v = swiglu1(y[0], y[1]);
+    const float lo = __shfl(v, 2 * (lane & 7), 64), hi = __shfl(v, 2 * (lane & 7) + 1, 64);
+    if (lane < 8) publish(out + lane, lo, hi);
+}
+
 template <int kNb>
-__device__ __forceinline__ void small_terms(ChainLds& L, const SmallW<kNb>& W, int w, int lane) {
+__device__ __forceinline__ void small_terms(ChainLds& L, const SmallLds& W, int w, int lane) {
     const int r = lane & 3, q = (lane >> 2) & 3, blk = lane >> 4;
 #pragma unroll
-    for (int i = 0; i < SmallW<kNb>::kLd; ++i) {
-        const int b = (w + kWaves * i) * 4 + blk;
-        if (b < kNb) L.terms[(q * 4 + r) * kSmallPitch + b] = chunk_term(L, W.w[i], b, q, (W.e[i] >> (8 * blk)) & 0xffu);
+    for (int i = 0; i < (kNb / 4 + kWaves - 1) / kWaves; ++i) {
+        const int j = w + kWaves * i;
+        if (j < kNb / 4)
+            L.terms[(q * 4 + r) * kSmallPitch + 4 * j + blk] =
+                chunk_term(L, W.w[j][lane], 4 * j + blk, q, (W.e[j][r] >> (8 * blk)) & 0xffu);
     }
 }
 // Wavefront 0: 16 chains, lane = residue * 4 + row; the four rows' two words.
@@ -286,10 +356,10 @@ __device__ __forceinline__ void small_sums(const ChainLds& L, uint64_t* out, int
     if (lane < 2) publish(out + lane, lo, hi);
 }
 
-// rmsnorm of x (threads below 256, elements 4 tid + j) times (1 + nw): into
+// rmsnorm of x (threads below 256, elements 4 tid + j) times (1 + nws): into
 // L.normed, and quantized into the LDS activation.  false: give up.
-__device__ __forceinline__ bool norm_step(ChainLds& L, const float (&x)[4], const float4& nw, float eps, int tid, int lane,
-                                          int w) {
+__device__ __forceinline__ bool norm_step(ChainLds& L, const float (&x)[4], const float4* nws, float eps, int tid,
+                                          int lane, int w) {
     if (tid < 256) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) L.sq[j][tid] = x[j] * x[j];
@@ -305,6 +375,7 @@ __device__ __forceinline__ bool norm_step(ChainLds& L, const float (&x)[4], cons
     lds_barrier();
     const float r = L.scale;
     if (tid < 256) {
+        const float4 nw = nws[tid];
         const float y[4] = {x[0] * (r * (1.0f + nw.x)), x[1] * (r * (1.0f + nw.y)), x[2] * (r * (1.0f + nw.z)),
                             x[3] * (r * (1.0f + nw.w))};
         *reinterpret_cast<float4*>(&L.normed[4 * tid]) = make_float4(y[0], y[1], y[2], y[3]);
@@ -314,9 +385,77 @@ __device__ __forceinline__ bool norm_step(ChainLds& L, const float (&x)[4], cons
     return true;
 }
 
+// The loader: the wavefront that does every load of weights, into LDS, a step
+// ahead.  A step is a norm, its GEMVs, and the GEMV behind them that the hidden
+// state waits for: norm .. o of a linear-attention layer, or norm .. down.  The
+// next step's loads go out in pieces right behind the barriers that tell that
+// an exchange is over: a CU's loads return in order, so a read of the exchange
+// words waits for every load before it (all of a buffer's loads as soon as it
+// is free: 530 us for a token's launch instead of 438).  The loader passes every barrier of
+// the steps with the others; its loads are waited for by a step's first one.  It
+// waits for nothing else, and runs on alone where the others gave up.
+__device__ __forceinline__ void loader(ChainLds& L, const RtChainArgs& a, ChainLayer* layers, int sub, int lane, int g) {
+    // step t (of layer l): blocks b0 .. b1 - 1, and with the last ones the second GEMV's weights
+    constexpr int kSplit = 10;
+    auto load = [&](int l, bool attn, int t, int b0, int b1) {
+        if (l >= a.n) return;
+        ChainLayer& y = layers[a.idx[l]];
+        BigLds& B = L.big[t & 1];
+        if (attn) {
+            const uint8_t *m = g < 192 ? y.mant[0] : y.mant[1], *e = g < 192 ? y.exps[0] : y.exps[1];
+            const int r = 2 * (g < 192 ? g : g - 192);
+            load_big(B, m, e, r, m, e, r + 1, y.in_ln_w, true, b0, b1, lane);
+            if (b1 == 16) load_small(L.small[t & 1], y.mant[2], y.exps[2], kHD / 64, sub, lane);
+        } else {
+            // (the last workgroups use only the norm weights)
+            load_big(B, y.mant[3], y.exps[3], g, y.mant[4], y.exps[4], g, y.post_ln_w, g < kMlpRows / 16, b0, b1, lane);
+            if (b1 == 16) load_small(L.small[t & 1], y.mant[5], y.exps[5], kMaxNb, sub, lane);
+        }
+    };
+    auto linear = [&](int l) { return l < a.n && layers[a.idx[l]].linear; };
+    auto barriers = [&](int n) {
+        for (int i = 0; i < n; ++i) lds_barrier();
+    };
+    // a layer's description into the scalar cache, for everyone, during a wait
+    // (read cold, it holds up a layer's first loads by more than 1 us)
+    auto touch = [&](int l) {
+        const auto* p = reinterpret_cast<const volatile __attribute__((address_space(4))) uint32_t*>(
+            &layers[a.idx[min(l, a.n - 1)]]);
+        uint32_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = p[min(16 * i, (int)sizeof(RtChainLayer) / 4 - 1)];
+        asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]));
+    };
+    static_assert(sizeof(RtChainLayer) <= 256, "four lines");
+    load(0, linear(0), 0, 0, 16);
+    touch(1);
+    int t = 0;
+    for (int l = 0; l < a.n; ++l) {
+        if (linear(l)) {
+            __builtin_amdgcn_s_waitcnt(kWaitLoads);
+            barriers(1);
+            load(l, false, t + 1, 0, kSplit);
+            barriers(4);  // norm (2), terms, q / k / v
+            load(l, false, t + 1, kSplit, 16);
+            barriers(5);  // the attention step (4), its output's squares
+            load(l + 1, linear(l + 1), t + 2, 0, kSplit);  // (this step's first buffer)
+            barriers(3);  // scale, activation, terms
+            ++t;
+        }
+        __builtin_amdgcn_s_waitcnt(kWaitLoads);
+        barriers(1);
+        load(l + 1, linear(l + 1), t + 1, linear(l) ? kSplit : 0, 16);
+        barriers(3);  // norm (2), terms
+        touch(l + 2);
+        barriers(2);  // activation, terms
+        ++t;
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitLoads);  // nothing lands after the workgroup's end
+}
+
 }  // namespace
 
-extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void rt_chain_kernel(
+extern "C" __global__ __launch_bounds__(kThreads + 64) void rt_chain_kernel(
     RtChainArgs a) {
     __shared__ ChainLds L;
     const int tid = threadIdx.x, lane = tid & 63, g = blockIdx.x;
@@ -333,26 +472,15 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
         __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     };
 
-    BigW bw;
-    SmallW<32> sc;
-    SmallW<56> se;
-    float4 nw;  // norm weights of elements 4 tid + j (tid < 256)
+    lds_barrier();  // L.fail
+    if (w == kWaves) {
+        loader(L, a, layers, sub, lane, g);
+        return;
+    }
     const int t4 = 4 * (tid & 255);
-    // a layer's first step: qkv / z, or gate / up
-    auto load_first = [&](ChainLayer& y) {
-        if (y.linear) {
-            load_big(bw, g < 192 ? y.mant[0] : y.mant[1], g < 192 ? y.exps[0] : y.exps[1], g < 192 ? g : g - 192, w, lane);
-            nw = *reinterpret_cast<const float4*>(y.in_ln_w + t4);
-        } else {
-            if (g < 224)
-                load_big(bw, g < 112 ? y.mant[3] : y.mant[4], g < 112 ? y.exps[3] : y.exps[4], g < 112 ? g : g - 112, w, lane);
-            nw = *reinterpret_cast<const float4*>(y.post_ln_w + t4);
-        }
-    };
 
     // the hidden state, elements 4 tid + j of threads below 256
     float h[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    lds_barrier();  // L.fail
     if (a.table) {
         if (tid < 256) {
 #pragma unroll
@@ -369,7 +497,6 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
                 h[j] = __uint_as_float((uint32_t)a.table[at] << 16);
             }
         }
-        load_first(layers[a.idx[0]]);
     } else {
         // one workgroup reads the host's copy and hands it on
         uint64_t* in = a.xch + (size_t)a.n * kWEnd;
@@ -380,7 +507,6 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
         }
         uint64_t v[2];
         if (!await(v, {in + 2 * (tid & 255), in + 2 * (tid & 255) + 1}, tid < 256, deadline)) give_up();
-        load_first(layers[a.idx[0]]);
         h[0] = word_lo(v[0]);
         h[1] = word_hi(v[0]);
         h[2] = word_lo(v[1]);
@@ -397,6 +523,7 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
         h[3] = h[3] + word_hi(v[1]);
     };
 
+    int t = 0;  // step
     for (int l = 0; l < a.n; ++l) {
         ChainLayer& y = layers[a.idx[l]];
         uint64_t* const X = a.xch + (size_t)l * kWEnd;
@@ -406,7 +533,10 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
             // ---- rmsnorm, then qkv and z (04/qwen_kernels_opt.c:925-941) ----
             // loads for the gates, the attention step and o
             const float4 gwt = *reinterpret_cast<const float4*>((tid < 256 ? y.wa : y.wb) + (size_t)head * RT_HIDDEN + t4);
-            const float nea = y.nea[head], dt = y.dt[head];
+            // (through the vector path: a scalar load in flight holds up every LDS wait)
+            int zero;
+            asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+            const float nea = y.nea[head + zero], dt = y.dt[head + zero];
             const int sect = min(tid >> 6, 2), ch = sect * kHD + head * RT_HEAD_DIM + 2 * lane;  // two channels (tid < 192)
             const float* ci = y.conv[cur];
             const float2 c0 = *reinterpret_cast<const float2*>(ci + ch);
@@ -419,9 +549,8 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
             const float2 S = *reinterpret_cast<const float2*>(y.rec[rcur] + so);
             const int si = 4 * ((tid >> 3) & 31) + 2 * (tid & 1);        // their row i (and i + 1)
             const int sj = 4 * (tid >> 8) + ((tid >> 1) & 3);            // and column of the eight
-            load_small<32>(sc, y.mant[2], y.exps[2], sub, w, lane);
             const float4 gnw = *reinterpret_cast<const float4*>(y.norm_w + ((4 * tid) & (RT_HEAD_DIM - 1)));
-            if (!norm_step(L, h, nw, a.eps, tid, lane, w)) return;
+            if (!norm_step(L, h, L.big[t & 1].nw, a.eps, tid, lane, w)) return;
             {
                 const float4 n4 = *reinterpret_cast<const float4*>(&L.normed[t4]);
                 float(*pg)[kChunk / 4 + 4] = L.pg[tid >> 8];
@@ -430,7 +559,7 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
                 pg[2][tid & 255] = gwt.z * n4.z;
                 pg[3][tid & 255] = gwt.w * n4.w;
             }
-            big_terms(L, bw, w, lane);
+            big_terms(L, L.big[t & 1], w, lane);
             lds_barrier();
             if (w < 2) {
                 big_sums(L, X + (g < 192 ? kWQkv + g * 16 : kWZ + (g - 192) * 16), w, lane);
@@ -449,11 +578,6 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
                 if (!await(v, {X + (conv ? kWQkv + (sect * kHD + head * RT_HEAD_DIM) / 2 + lane : zcol ? kWZ + zi : kWQkv)},
                            conv || zcol, deadline))
                     give_up();
-                // the next step's weights, behind the inputs
-                if (g < 224)
-                    load_big(bw, g < 112 ? y.mant[3] : y.mant[4], g < 112 ? y.exps[3] : y.exps[4], g < 112 ? g : g - 112, w,
-                             lane);
-                nw = *reinterpret_cast<const float4*>(y.post_ln_w + t4);
                 const float x0 = word_lo(v[0]), x1 = word_hi(v[0]);
                 if (conv) {
                     float d0 = cw0.x * c0.x, d1 = cw1.x * c0.y;
@@ -567,46 +691,32 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
                 bfp8_quant4_store_lds(v, tid & 15, &L.xsc[tid >> 4], &L.xs[(tid >> 4) * 32], true);
             }
             lds_barrier();
-            small_terms<32>(L, sc, w, lane);
+            small_terms<kHD / 64>(L, L.small[t & 1], w, lane);
             lds_barrier();
-            if (w == 0) small_sums<32>(L, X + kWO + 2 * sub, lane);
+            if (w == 0) small_sums<kHD / 64>(L, X + kWO + 2 * sub, lane);
             add_words(X + kWO);
+            ++t;
         }
-        // ---- rmsnorm, gate and up (:987-997) ----
-        load_small<56>(se, y.mant[5], y.exps[5], sub, w, lane);
-        if (!norm_step(L, h, nw, a.eps, tid, lane, w)) return;
-        if (g < 224) big_terms(L, bw, w, lane);
+        // ---- rmsnorm, gate and up, swiglu (:987-1001) ----
+        if (!norm_step(L, h, L.big[t & 1].nw, a.eps, tid, lane, w)) return;
+        if (g < kMlpRows / 16) big_terms(L, L.big[t & 1], w, lane);
         lds_barrier();
-        if (g < 224 && w < 2) big_sums(L, X + (g < 112 ? kWGate + g * 16 : kWUp + (g - 112) * 16), w, lane);
-        // ---- swiglu, down (:998-1004) ----
-        {
-            uint64_t v[4], u[4];
-            const uint64_t* pg = X + kWGate + 2 * tid;
-            const uint64_t* pu = X + kWUp + 2 * tid;
-            bool ok = await(v, {pg, pg + 1, pu, pu + 1}, true, deadline);
-            // (the last 1536 elements: threads below 384)
-            const int m = tid < 384 ? 1024 : 0;
-            ok = await(u, {pg + m, pg + m + 1, pu + m, pu + m + 1}, tid < 384, deadline) && ok;
-            if (!ok) give_up();
-            if (l + 1 < a.n) load_first(layers[a.idx[l + 1]]);
-            // (one body for both halves: the code stays short)
-#pragma unroll 1
-            for (int half = 0; half < 2; ++half) {
-                if (half && w >= 6) break;
-                const uint64_t g0 = half ? u[0] : v[0], g1 = half ? u[1] : v[1], u0 = half ? u[2] : v[2], u1 = half ? u[3] : v[3];
-                const float gt[4] = {word_lo(g0), word_hi(g0), word_lo(g1), word_hi(g1)};
-                const float up[4] = {word_lo(u0), word_hi(u0), word_lo(u1), word_hi(u1)};
-                float s[4];
-                swiglu4(s, gt, up);
-                const int b = 32 * half + (tid >> 4);
-                bfp8_quant4_store_lds(s, tid & 15, &L.xsc[b], &L.xs[b * 32], true);
-            }
+        if (g < kMlpRows / 16 && w == 0) mlp_sums(L, X + kWMlp + g * 8, lane);
+        // ---- down (:1002-1004) ----
+        if (w < kMlpRows / 512) {
+            uint64_t v[4];
+            const uint64_t* p = X + kWMlp + 4 * tid;
+            if (!await(v, {p, p + 1, p + 2, p + 3}, true, deadline)) give_up();
+            const float x[8] = {word_lo(v[0]), word_hi(v[0]), word_lo(v[1]), word_hi(v[1]),
+                                word_lo(v[2]), word_hi(v[2]), word_lo(v[3]), word_hi(v[3])};
+            quant8_store_lds(x, tid & 7, &L.xsc[tid >> 3], &L.xs[(tid >> 3) * 32]);
         }
         lds_barrier();
         if (L.fail) return;
-        small_terms<56>(L, se, w, lane);
+        small_terms<kMaxNb>(L, L.small[t & 1], w, lane);
         lds_barrier();
-        if (w == 0) small_sums<56>(L, X + kWDown + 2 * sub, lane);
+        if (w == 0) small_sums<kMaxNb>(L, X + kWDown + 2 * sub, lane);
+        ++t;
     }
 
     // the other set's words, for the launch after this one
@@ -616,8 +726,7 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
     add_words(a.xch + (size_t)(a.n - 1) * kWEnd + kWDown);
     if (tid < 256) *reinterpret_cast<float4*>(a.h_out + 4 * tid) = make_float4(h[0], h[1], h[2], h[3]);
     if (a.y_norm) {
-        nw = *reinterpret_cast<const float4*>(a.final_w + t4);
-        if (!norm_step(L, h, nw, a.eps, tid, lane, w)) return;
+        if (!norm_step(L, h, reinterpret_cast<const float4*>(a.final_w), a.eps, tid, lane, w)) return;
         if (tid < 256) *reinterpret_cast<float4*>(a.y_norm + 4 * tid) = *reinterpret_cast<const float4*>(&L.normed[4 * tid]);
     }
 }
@@ -626,7 +735,7 @@ extern "C" __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_pe
 bool rt_chain_fits() {
     static const bool fits = [] {
         int occ = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(rt_chain_kernel), kThreads, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(rt_chain_kernel), kThreads + 64, 0) !=
             hipSuccess) {
             (void)hipGetLastError();
             return false;
@@ -640,6 +749,6 @@ hipError_t rt_launch_chain(const RtChainArgs& a, hipStream_t s) {
     if (a.n < 1 || a.n > RT_CHAIN_MAX_LAYERS || (!a.table && !a.h_in) || !a.h_out || !a.status || !a.xch ||
         a.xch == a.xch_clear || (a.y_norm && !a.final_w))
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(rt_chain_kernel, dim3(RT_CHAIN_WGS), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL(rt_chain_kernel, dim3(RT_CHAIN_WGS), dim3(kThreads + 64), 0, s, a);
     return hipGetLastError();
 }

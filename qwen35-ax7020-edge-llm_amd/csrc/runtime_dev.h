@@ -150,13 +150,14 @@ __device__ __forceinline__ float conv_elem(float xc, float* s0, float* s1, float
 // 1 / sqrtf(ss / n + eps), scalar
 // Each step is one IEEE operation.  The float instructions answer when every
 // operand and intermediate is normal (one combined test, no branch per step;
-// the square root of a normal positive float is normal), else the exact
+// the square root of a normal positive float is normal, and sqrtf's refined
+// instruction rounds every one of them as the double square root does), else the exact
 // helpers do; a power-of-two n divides exactly as a product with 1/n.
 __device__ __forceinline__ float rms_scale(float ss, int n, float eps) {
     const float fn = (float)n;
     const float m = ((n & (n - 1)) == 0) ? ss * (1.0f / fn) : __fdiv_rn(ss, fn);
     const float t = m + eps;
-    const float q = (float)__builtin_sqrt((double)t);
+    const float q = __builtin_sqrtf(t);
     const float r = __fdiv_rn(1.0f, q);
     if (normal_u(ss) & normal_u(fn) & normal_u(m) & normal_u(eps) & normal_u(t) & normal_u(r)) return r;
     return ieee_div(1.0f, ieee_sqrt(ieee_add(ieee_div(ss, fn), eps)));
@@ -165,7 +166,7 @@ __device__ __forceinline__ float rms_scale(float ss, int n, float eps) {
 // num / sqrtf(x + eps), scalar, with one combined normality test as in rms_scale
 __device__ __forceinline__ float div_sqrt_add(float num, float x, float eps) {
     const float t = x + eps;
-    const float q = (float)__builtin_sqrt((double)t);
+    const float q = __builtin_sqrtf(t);
     const float r = __fdiv_rn(num, q);
     if (normal_u(num) & normal_u(x) & normal_u(eps) & normal_u(t) & normal_u(r)) return r;
     return ieee_div(num, ieee_sqrt(ieee_add(x, eps)));

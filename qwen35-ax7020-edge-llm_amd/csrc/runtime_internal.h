@@ -152,7 +152,7 @@ hipError_t rt_launch_rows(const RtRowsArgs& a, hipStream_t s);
 // the model's (hidden 1024, 16 heads of 128, MLP 3584).
 #define RT_CHAIN_WGS 256
 #define RT_CHAIN_MAX_LAYERS 24
-#define RT_CHAIN_LAYER_WORDS (512 + 512 + 3072 + 1024 + 1024 + 1024 + 1792 + 1792)
+#define RT_CHAIN_LAYER_WORDS (512 + 512 + 3072 + 1024 + 1024 + 1024 + 1792)
 #define RT_CHAIN_SET_WORDS (RT_CHAIN_MAX_LAYERS * RT_CHAIN_LAYER_WORDS + 512)  // 512: the hidden state handed in
 struct RtChainLayer {     // device memory
     const uint8_t* mant[6];  // GPU planes: qkv, z, o, gate, up, down (an MLP layer: the last three)
@@ -164,7 +164,7 @@ struct RtChainLayer {     // device memory
 };
 struct RtChainArgs {
     const RtChainLayer* layers;
-    uint16_t idx[RT_CHAIN_MAX_LAYERS];  // the run's layers
+    uint32_t idx[RT_CHAIN_MAX_LAYERS];  // the run's layers (32 bits: read by scalar loads)
     int n;
     uint32_t cur, rcur;   // bit l: the current buffer of layer l's taps / state; the other one is written
     const uint16_t* table;  // the run starts from row `row` of this embedding table (ntiles as in rt_launch_embed) ...
