@@ -24,13 +24,15 @@
 //   * the workgroup that has 16 rows of gate has those of up too and hands on
 //     their swiglu: half the words, and no workgroup computes all 3584.
 //
-// Bound by latency: a linear-attention layer is 21.2 us, of them 6.6 in five
-// exchanges, of which one between all workgroups takes 1.2 to 2.3 us (store,
+// Bound by latency: a linear-attention layer is 20.5 us, of them 8 in five
+// exchanges, of which one between all workgroups takes 1.3 to 2.2 us (store,
 // memory-side cache, the last of 256 readers' polls) and one between a head's
 // 0.8; 2.9 in 824 dependent float adds, 8 cycles each, that the results' order
-// fixes; its 21.5 MB of weights would stream in 4.  Before the loader wavefront,
-// the pair of rows and 32-bit layer indices (16-bit ones are read by vector
-// loads): 24.0 us; a token's launch 517 us, now 438.
+// fixes; its 21.5 MB of weights would stream in 4.  Weights in the wavefronts'
+// registers, gate and up from different workgroups, 16-bit layer indices (read
+// by vector loads): 24.0 us, a token's launch 517; with the loader, 438; with
+// the attention step on four wavefronts without barriers and stores of 32
+// bytes, 422.
 //
 // Every operation and its order are those of the separate kernels (the GEMV
 // terms and block-order sums of fused_gemv.hip, the attention step of
@@ -60,12 +62,13 @@ constexpr int kHD = RT_HEADS * RT_HEAD_DIM;
 constexpr int kMaxNb = kMlpRows / 64;
 constexpr uint64_t kNotYet = ~0ull;
 // words of one layer's vectors
-constexpr int kWDown = 0, kWO = kWDown + RT_HIDDEN / 2, kWQkv = kWO + RT_HIDDEN / 2, kWZ = kWQkv + RT_CONV_CH / 2,
+constexpr int kRowWords = RT_CHAIN_ROW_WORDS;
+constexpr int kWDown = 0, kWO = kWDown + RT_CHAIN_WGS * kRowWords, kWQkv = kWO + RT_CHAIN_WGS * kRowWords, kWZ = kWQkv + RT_CONV_CH / 2,
               kWAttn = kWZ + kHD / 2, kWZs = kWAttn + kHD / 2, kWMlp = kWZs + kHD / 2, kWEnd = kWMlp + kMlpRows / 2;
 static_assert(kWEnd == RT_CHAIN_LAYER_WORDS, "exchange words of a layer");
 // the attention step's columns of a workgroup: 16 workgroups per head
 constexpr int kParts = RT_CHAIN_WGS / RT_HEADS, kCols = RT_HEAD_DIM / kParts;
-static_assert(kCols == 8 && kCols * RT_HEAD_DIM == 2 * kThreads, "two state elements per thread");
+static_assert(kCols == 8 && kCols / 2 * 256 == kCols * RT_HEAD_DIM, "four state elements per thread of four wavefronts");
 constexpr int kWaitLoads = 0x0F70;             // s_waitcnt vmcnt(0)
 constexpr int kBigRows = 32;                  // rows per workgroup of the K = 1024 GEMVs
 constexpr int kBigPitch = 16 + 4, kSmallPitch = kMaxNb + 4;  // floats per chain of terms (16-byte rows)
@@ -94,13 +97,13 @@ struct ChainLds {
     __attribute__((aligned(16))) float pg[2][4][kChunk / 4 + 4];   // the gates' products
     __attribute__((aligned(16))) float normed[RT_HIDDEN];
     __attribute__((aligned(16))) float kq[2][RT_HEAD_DIM];         // k, q
-    float vv[RT_HEAD_DIM];
-    __attribute__((aligned(16))) float lq[2][4][36];               // k and q squares; q * k
+    __attribute__((aligned(16))) float vv[RT_HEAD_DIM];
+    __attribute__((aligned(16))) float lq[2][4][36];               // k and q squares
+    __attribute__((aligned(16))) float qk[kCols / 2][4][36];       // a wavefront's q * k
     __attribute__((aligned(16))) float sp[2][kCols][RT_HEAD_DIM + 4];  // S * k, S * q per column
     __attribute__((aligned(16))) float gp[RT_HEADS][4][36];        // the gated norm's squares
-    float gr[RT_HEADS];
-    float dcol[kCols];
-    float sc[5];  // alpha, beta, k scale, q scale, q.k
+    float sc[2];  // alpha, beta
+    __attribute__((aligned(8))) float ocol[kCols];
     float scale;
     int fail;
 };
@@ -114,6 +117,13 @@ __device__ __forceinline__ void lds_barrier() {  // LDS only: loads stay in flig
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+}
+
+// Orders a wavefront's own LDS writes before its reads of other lanes' ones.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ __forceinline__ float word_lo(uint64_t v) { return __uint_as_float((uint32_t)v); }
@@ -154,27 +164,23 @@ __device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t rs, void* lds,
 __device__ __forceinline__ void lds_load4(__amdgpu_buffer_rsrc_t rs, void* lds, int voff) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)lds, 4, voff, 0, 0, 0);
 }
-// Blocks b0 .. b1 - 1 of rows 16 r0 .. and 16 r1 .. of two (or one) matrices of
-// 1024 columns, the norm weights and exponents with block 0.
+// Rows 16 r0 .. and 16 r1 .. of two (or one) matrices of 1024 columns, with the
+// norm weights (only these without `rows`).
 __device__ __forceinline__ void load_big(BigLds& L, const uint8_t* m0, const uint8_t* e0, int r0, const uint8_t* m1,
-                                         const uint8_t* e1, int r1, const float* nw, bool rows, int b0, int b1, int lane) {
+                                         const uint8_t* e1, int r1, const float* nw, bool rows, int lane) {
     const int at[2] = {(r0 & 3) * 16 + (lane & 15), (r1 & 3) * 16 + (lane & 15)};
-    if (b0 == 0) {
-        const __amdgpu_buffer_rsrc_t nr = make_rsrc(nw, RT_HIDDEN * 4);
+    const __amdgpu_buffer_rsrc_t nr = make_rsrc(nw, RT_HIDDEN * 4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) lds_load16(nr, &L.nw[64 * i], lane * 16, i * 1024);
-    }
+    for (int i = 0; i < 4; ++i) lds_load16(nr, &L.nw[64 * i], lane * 16, i * 1024);
     if (!rows) return;
-    if (b0 == 0) {
-        const __amdgpu_buffer_rsrc_t er[2] = {make_rsrc(e0 + (size_t)(r0 >> 2) * 4 * 256u, 4 * 256u),
-                                              make_rsrc(e1 + (size_t)(r1 >> 2) * 4 * 256u, 4 * 256u)};
-#pragma unroll
-        for (int m = 0; m < 2; ++m) lds_load4(er[m], &L.e[m][0][0], (lane >> 4) * 256 + at[m] * 4);
-    }
+    const __amdgpu_buffer_rsrc_t er[2] = {make_rsrc(e0 + (size_t)(r0 >> 2) * 4 * 256u, 4 * 256u),
+                                          make_rsrc(e1 + (size_t)(r1 >> 2) * 4 * 256u, 4 * 256u)};
     const __amdgpu_buffer_rsrc_t wr[2] = {make_rsrc(m0 + (size_t)(r0 >> 2) * 16 * 4096u, 16 * 4096u),
                                           make_rsrc(m1 + (size_t)(r1 >> 2) * 16 * 4096u, 16 * 4096u)};
+#pragma unroll
+    for (int m = 0; m < 2; ++m) lds_load4(er[m], &L.e[m][0][0], (lane >> 4) * 256 + at[m] * 4);
 #pragma unroll 1
-    for (int b = b0; b < b1; ++b)
+    for (int b = 0; b < 16; ++b)
 #pragma unroll
         for (int m = 0; m < 2; ++m) lds_load16(wr[m], &L.w[b][m][0], (lane >> 4) * 1024 + at[m] * 16, b * 4096);
 }
@@ -205,16 +211,15 @@ __device__ __forceinline__ float chunk_term(const ChainLds& L, const u32x4& wq, 
     return t1 * L.xsc[b];
 }
 
-// p[0] + ... + p[n - 1] from +0 in this order (LDS, 16-byte aligned); the
+// s + p[0] + ... + p[n - 1] in this order (LDS, 16-byte aligned); the
 // reads run kAhead ahead of the adds (spread as in chain_add256).
 template <int kN>
-__device__ __forceinline__ float chain_n(const float* p) {
+__device__ __forceinline__ float chain_n(const float* p, float s = 0.0f) {
     constexpr int kV = kN / 4, kAhead = kV < 8 ? kV : 8;
     const float4* p4 = reinterpret_cast<const float4*>(p);
     float4 v[kV];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) v[i] = p4[i];
-    float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < kV; ++i) {
         if (i + kAhead < kV) v[i + kAhead] = p4[i + kAhead];
@@ -345,7 +350,9 @@ __device__ __forceinline__ void small_terms(ChainLds& L, const SmallLds& W, int 
                 chunk_term(L, W.w[j][lane], 4 * j + blk, q, (W.e[j][r] >> (8 * blk)) & 0xffu);
     }
 }
-// Wavefront 0: 16 chains, lane = residue * 4 + row; the four rows' two words.
+// Wavefront 0: 16 chains, lane = residue * 4 + row; the four rows' two words,
+// twice (a store of less than 32 bytes arrives later: 429 us for a token's
+// launch with the 16 bytes alone, 422 with 32).
 template <int kNb>
 __device__ __forceinline__ void small_sums(const ChainLds& L, uint64_t* out, int lane) {
     const float fs = chain_n<kNb>(&L.terms[(lane & 15) * kSmallPitch]);
@@ -353,7 +360,7 @@ __device__ __forceinline__ void small_sums(const ChainLds& L, uint64_t* out, int
     const float f0 = __shfl(fs, r, 64), f1 = __shfl(fs, 4 + r, 64), f2 = __shfl(fs, 8 + r, 64), f3 = __shfl(fs, 12 + r, 64);
     const float y = (f0 + f2) + (f1 + f3);
     const float lo = __shfl(y, 2 * (lane & 1), 64), hi = __shfl(y, 2 * (lane & 1) + 1, 64);
-    if (lane < 2) publish(out + lane, lo, hi);
+    if (lane < kRowWords) publish(out + lane, lo, hi);
 }
 
 // rmsnorm of x (threads below 256, elements 4 tid + j) times (1 + nws): into
@@ -385,32 +392,34 @@ __device__ __forceinline__ bool norm_step(ChainLds& L, const float (&x)[4], cons
     return true;
 }
 
-// The loader: the wavefront that does every load of weights, into LDS, a step
-// ahead.  A step is a norm, its GEMVs, and the GEMV behind them that the hidden
-// state waits for: norm .. o of a linear-attention layer, or norm .. down.  The
-// next step's loads go out in pieces right behind the barriers that tell that
-// an exchange is over: a CU's loads return in order, so a read of the exchange
-// words waits for every load before it (all of a buffer's loads as soon as it
-// is free: 530 us for a token's launch instead of 438).  The loader passes every barrier of
-// the steps with the others; its loads are waited for by a step's first one.  It
-// waits for nothing else, and runs on alone where the others gave up.
+// The loader: the wavefront that does every load of weights, into LDS.  A step
+// is a norm, its GEMVs (the first buffer), and the GEMV behind them that the
+// hidden state waits for (the second): norm .. o of a linear-attention layer, or
+// norm .. down.  The next steps' loads go out right behind the barriers that tell
+// that an exchange is over, and that leave the longest way to the next: a CU's
+// loads return in order, so a read of the exchange words waits for every load
+// before it (a buffer's loads as soon as it is free: 530 us for a token's launch
+// where this took 438).  The loader passes every barrier of the steps with the
+// others; its loads are waited for by a step's first one.  It waits for nothing
+// else, and runs on alone where the others gave up.
 __device__ __forceinline__ void loader(ChainLds& L, const RtChainArgs& a, ChainLayer* layers, int sub, int lane, int g) {
-    // step t (of layer l): blocks b0 .. b1 - 1, and with the last ones the second GEMV's weights
-    constexpr int kSplit = 10;
-    auto load = [&](int l, bool attn, int t, int b0, int b1) {
+    auto load_first = [&](int l, bool attn, int t) {  // step t, of layer l
         if (l >= a.n) return;
         ChainLayer& y = layers[a.idx[l]];
         BigLds& B = L.big[t & 1];
         if (attn) {
             const uint8_t *m = g < 192 ? y.mant[0] : y.mant[1], *e = g < 192 ? y.exps[0] : y.exps[1];
             const int r = 2 * (g < 192 ? g : g - 192);
-            load_big(B, m, e, r, m, e, r + 1, y.in_ln_w, true, b0, b1, lane);
-            if (b1 == 16) load_small(L.small[t & 1], y.mant[2], y.exps[2], kHD / 64, sub, lane);
-        } else {
-            // (the last workgroups use only the norm weights)
-            load_big(B, y.mant[3], y.exps[3], g, y.mant[4], y.exps[4], g, y.post_ln_w, g < kMlpRows / 16, b0, b1, lane);
-            if (b1 == 16) load_small(L.small[t & 1], y.mant[5], y.exps[5], kMaxNb, sub, lane);
+            load_big(B, m, e, r, m, e, r + 1, y.in_ln_w, true, lane);
+        } else {  // (the last workgroups use only the norm weights)
+            load_big(B, y.mant[3], y.exps[3], g, y.mant[4], y.exps[4], g, y.post_ln_w, g < kMlpRows / 16, lane);
         }
+    };
+    auto load_second = [&](int l, bool attn, int t) {
+        if (l >= a.n) return;
+        ChainLayer& y = layers[a.idx[l]];
+        const int i = attn ? 2 : 5;
+        load_small(L.small[t & 1], y.mant[i], y.exps[i], attn ? kHD / 64 : kMaxNb, sub, lane);
     };
     auto linear = [&](int l) { return l < a.n && layers[a.idx[l]].linear; };
     auto barriers = [&](int n) {
@@ -427,24 +436,27 @@ __device__ __forceinline__ void loader(ChainLds& L, const RtChainArgs& a, ChainL
         asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]));
     };
     static_assert(sizeof(RtChainLayer) <= 256, "four lines");
-    load(0, linear(0), 0, 0, 16);
+    load_first(0, linear(0), 0);
+    load_second(0, linear(0), 0);
     touch(1);
     int t = 0;
     for (int l = 0; l < a.n; ++l) {
         if (linear(l)) {
             __builtin_amdgcn_s_waitcnt(kWaitLoads);
             barriers(1);
-            load(l, false, t + 1, 0, kSplit);
-            barriers(4);  // norm (2), terms, q / k / v
-            load(l, false, t + 1, kSplit, 16);
-            barriers(5);  // the attention step (4), its output's squares
-            load(l + 1, linear(l + 1), t + 2, 0, kSplit);  // (this step's first buffer)
-            barriers(3);  // scale, activation, terms
+            load_first(l, false, t + 1);
+            barriers(2);  // norm
+            load_second(l, false, t + 1);
+            barriers(2);  // terms, q / k / v
+            barriers(2);  // the attention step, all heads' outputs
+            load_first(l + 1, linear(l + 1), t + 2);  // (into this step's buffer, read a barrier ago)
+            barriers(2);  // activation, terms
             ++t;
         }
         __builtin_amdgcn_s_waitcnt(kWaitLoads);
         barriers(1);
-        load(l + 1, linear(l + 1), t + 1, linear(l) ? kSplit : 0, 16);
+        if (!linear(l)) load_first(l + 1, linear(l + 1), t + 1);
+        load_second(l + 1, linear(l + 1), t + 1);
         barriers(3);  // norm (2), terms
         touch(l + 2);
         barriers(2);  // activation, terms
@@ -516,7 +528,7 @@ extern "C" __global__ __launch_bounds__(kThreads + 64) void rt_chain_kernel(
     // h += the vector at `words` (add_residual)
     auto add_words = [&](const uint64_t* words) {
         uint64_t v[2];
-        if (!await(v, {words + 2 * (tid & 255), words + 2 * (tid & 255) + 1}, tid < 256, deadline)) give_up();
+        if (!await(v, {words + kRowWords * (tid & 255), words + kRowWords * (tid & 255) + 1}, tid < 256, deadline)) give_up();
         h[0] = h[0] + word_lo(v[0]);
         h[1] = h[1] + word_hi(v[0]);
         h[2] = h[2] + word_lo(v[1]);
@@ -544,11 +556,13 @@ extern "C" __global__ __launch_bounds__(kThreads + 64) void rt_chain_kernel(
             const float2 c2 = *reinterpret_cast<const float2*>(ci + 2 * RT_CONV_CH + ch);
             const float4 cw0 = *reinterpret_cast<const float4*>(y.conv_w + (size_t)ch * 4);
             const float4 cw1 = *reinterpret_cast<const float4*>(y.conv_w + (size_t)ch * 4 + 4);
-            // two elements of this workgroup's eight state columns (blocked layout, contiguous)
-            const size_t so = (size_t)head * RT_HEAD_DIM * RT_HEAD_DIM + (size_t)part * kCols * RT_HEAD_DIM + 2 * tid;
-            const float2 S = *reinterpret_cast<const float2*>(y.rec[rcur] + so);
-            const int si = 4 * ((tid >> 3) & 31) + 2 * (tid & 1);        // their row i (and i + 1)
-            const int sj = 4 * (tid >> 8) + ((tid >> 1) & 3);            // and column of the eight
+            // four rows of one of this workgroup's eight state columns (blocked layout): wavefronts
+            // 0 .. 3 have columns 2w and 2w + 1
+            const int scol = 2 * (w & 3) + (lane & 1);
+            const size_t so = (size_t)head * RT_HEAD_DIM * RT_HEAD_DIM + (size_t)part * kCols * RT_HEAD_DIM +
+                              ((scol >> 2) * (RT_HEAD_DIM / 4) + (lane >> 1)) * 16 + (scol & 3) * 4;
+            float4 S;
+            if (w < kCols / 2) S = *reinterpret_cast<const float4*>(y.rec[rcur] + so);
             const float4 gnw = *reinterpret_cast<const float4*>(y.norm_w + ((4 * tid) & (RT_HEAD_DIM - 1)));
             if (!norm_step(L, h, L.big[t & 1].nw, a.eps, tid, lane, w)) return;
             {
@@ -610,55 +624,47 @@ extern "C" __global__ __launch_bounds__(kThreads + 64) void rt_chain_kernel(
             }
             lds_barrier();
             if (L.fail) return;
-            if (w == 0) {
-                float s = 0.0f;
-                if (lane < 8) s = chain_n<RT_HEAD_DIM / 4>(&L.lq[lane >> 2][lane & 3][0]);
-                const float r = lanes4_combine(s);
-                const float q_sq = readlane_f(r, 4);
-                if (lane == 0) {
-                    // 1 / sqrtf(D): both steps of normal constants, so the instructions are exact
-                    const float q_scale = __fdiv_rn(1.0f, (float)__builtin_sqrt((double)RT_HEAD_DIM));
-                    L.sc[2] = div_sqrt_add(1.0f, r, 1e-6f);
-                    L.sc[3] = div_sqrt_add(q_scale, q_sq, 1e-6f);
+            // (each of the four wavefronts by itself, no barrier: both scales, then the two
+            // columns' sums and q . k as one chain of adds over its lanes)
+            if (w < kCols / 2) {
+                const int c8 = lane & 7;  // k (0 .. 3) and q (4 .. 7) squares of a residue
+                const float sq = lanes4_combine(chain_n<RT_HEAD_DIM / 4>(&L.lq[c8 >> 2][c8 & 3][0]));
+                // 1 / sqrtf(D): both steps of normal constants, so the instructions are exact
+                const float q_scale = __fdiv_rn(1.0f, (float)__builtin_sqrt((double)RT_HEAD_DIM));
+                const float sc = div_sqrt_add(c8 < 4 ? 1.0f : q_scale, sq, 1e-6f);
+                const float ks = readlane_f(sc, 0), qs = readlane_f(sc, 4);
+                const int i4 = lane >> 1;
+                float4 k4 = *reinterpret_cast<const float4*>(&L.kq[0][4 * i4]);
+                float4 q4 = *reinterpret_cast<const float4*>(&L.kq[1][4 * i4]);
+                k4 = make_float4(k4.x * ks, k4.y * ks, k4.z * ks, k4.w * ks);
+                q4 = make_float4(q4.x * qs, q4.y * qs, q4.z * qs, q4.w * qs);
+                *reinterpret_cast<float4*>(&L.sp[0][scol][4 * i4]) = make_float4(S.x * k4.x, S.y * k4.y, S.z * k4.z, S.w * k4.w);
+                *reinterpret_cast<float4*>(&L.sp[1][scol][4 * i4]) = make_float4(S.x * q4.x, S.y * q4.y, S.z * q4.z, S.w * q4.w);
+                if ((lane & 1) == 0) {
+                    L.qk[w][0][i4] = q4.x * k4.x;
+                    L.qk[w][1][i4] = q4.y * k4.y;
+                    L.qk[w][2][i4] = q4.z * k4.z;
+                    L.qk[w][3][i4] = q4.w * k4.w;
                 }
+                wave_lds_sync();
+                // lanes 0 .. 3: k . S and q . S of the two columns; 4 .. 7: q . k's residues,
+                // whose 32 terms are the first quarter (the rest of theirs is not used)
+                const float* row = &L.sp[(c8 >> 1) & 1][2 * w + (c8 & 1)][0];
+                const float s32 = chain_n<RT_HEAD_DIM / 4>(c8 < 4 ? row : &L.qk[w][c8 & 3][0]);
+                const float acc = chain_n<3 * RT_HEAD_DIM / 4>(row + RT_HEAD_DIM / 4, s32);
+                const float qk = readlane_f(lanes4_combine(s32), 4);
+                const float alpha = L.sc[0], beta = L.sc[1];
+                const float2 v2 = *reinterpret_cast<const float2*>(&L.vv[part * kCols + 2 * w]);
+                const float d0 = (v2.x - readlane_f(acc, 0) * alpha) * beta, d1 = (v2.y - readlane_f(acc, 1) * alpha) * beta;
+                const float o0 = readlane_f(acc, 2) * alpha + qk * d0, o1 = readlane_f(acc, 3) * alpha + qk * d1;
+                if (lane == 0) *reinterpret_cast<float2*>(&L.ocol[2 * w]) = make_float2(o0, o1);
+                const float d = (lane & 1) ? d1 : d0;
+                S = make_float4(S.x * alpha + d * k4.x, S.y * alpha + d * k4.y, S.z * alpha + d * k4.z, S.w * alpha + d * k4.w);
             }
-            lds_barrier();
-            if (tid < RT_HEAD_DIM) {
-                const float k = L.kq[0][tid] * L.sc[2], q = L.kq[1][tid] * L.sc[3];
-                L.kq[0][tid] = k;
-                L.kq[1][tid] = q;
-                L.lq[0][tid & 3][tid >> 2] = q * k;
-            }
-            lds_barrier();
-            const float2 k2 = *reinterpret_cast<const float2*>(&L.kq[0][si]);
-            {
-                const float2 q2 = *reinterpret_cast<const float2*>(&L.kq[1][si]);
-                *reinterpret_cast<float2*>(&L.sp[0][sj][si]) = make_float2(S.x * k2.x, S.y * k2.y);
-                *reinterpret_cast<float2*>(&L.sp[1][sj][si]) = make_float2(S.x * q2.x, S.y * q2.y);
-            }
-            if (w == 1) {
-                float s = 0.0f;
-                if (lane < 4) s = chain_n<RT_HEAD_DIM / 4>(&L.lq[0][lane][0]);
-                const float r = lanes4_combine(s);
-                if (lane == 0) L.sc[4] = r;
-            }
-            lds_barrier();
-            const float alpha = L.sc[0], beta = L.sc[1];
-            if (w == 0) {  // lane = role * 8 + column: sum_i k[i] S[i][j], sum_i q[i] S[i][j]
-                const float acc = chain_n<RT_HEAD_DIM>(&L.sp[(lane >> 3) & 1][lane & 7][0]);
-                const int c = lane & 7;
-                const float kvs = __shfl(acc, c, 64), qss = __shfl(acc, 8 + c, 64);
-                const float d = (L.vv[part * kCols + c] - kvs * alpha) * beta;
-                const float o = qss * alpha + L.sc[4] * d;
-                if (lane < kCols) L.dcol[lane] = d;
-                const float lo = __shfl(o, 2 * (lane & 3), 64), hi = __shfl(o, 2 * (lane & 3) + 1, 64);
-                if (lane < kCols / 2) publish(X + kWAttn + (head * RT_HEAD_DIM + part * kCols) / 2 + lane, lo, hi);
-            }
-            lds_barrier();
-            {
-                const float d = L.dcol[sj];
-                *reinterpret_cast<float2*>(y.rec[rcur ^ 1] + so) = make_float2(S.x * alpha + d * k2.x, S.y * alpha + d * k2.y);
-            }
+            lds_barrier();  // (also: no polls before there can be something, they get in the way)
+            // (one store of 32 bytes: four of 8, one by each wavefront, arrive 0.9 us later)
+            if (w == 0 && lane < kCols / 2)
+                publish(X + kWAttn + (head * RT_HEAD_DIM + part * kCols) / 2 + lane, L.ocol[2 * lane], L.ocol[2 * lane + 1]);
             // ---- gated RMSNorm, then o (:968-985) ----
             float at[4], zs[4];
             {
@@ -675,17 +681,18 @@ extern "C" __global__ __launch_bounds__(kThreads + 64) void rt_chain_kernel(
                 zs[2] = word_lo(v[3]);
                 zs[3] = word_hi(v[3]);
             }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) L.gp[tid >> 5][j][tid & 31] = at[j] * at[j];
-            lds_barrier();
+            // (behind the exchange: its reads would wait for the store)
+            if (w < kCols / 2) *reinterpret_cast<float4*>(y.rec[rcur ^ 1] + so) = S;
+            lds_barrier();  // (for the loader: the exchange is over)
             if (L.fail) return;
-            if (w == 0) {
-                const float r = lanes4_combine(chain_n<RT_HEAD_DIM / 4>(&L.gp[lane >> 2][lane & 3][0]));
-                if ((lane & 3) == 0) L.gr[lane >> 2] = rms_scale(r, RT_HEAD_DIM, a.eps);
-            }
-            lds_barrier();
             {
-                const float gr = L.gr[tid >> 5];
+                // wavefront w has heads 2w and 2w + 1; lane & 7 = head * 4 + residue of their squares
+#pragma unroll
+                for (int j = 0; j < 4; ++j) L.gp[tid >> 5][j][tid & 31] = at[j] * at[j];
+                wave_lds_sync();
+                const float ss = lanes4_combine(chain_n<RT_HEAD_DIM / 4>(&L.gp[2 * w + ((lane >> 2) & 1)][lane & 3][0]));
+                const float sc = rms_scale(ss, RT_HEAD_DIM, a.eps);
+                const float gr = lane < 32 ? readlane_f(sc, 0) : readlane_f(sc, 4);
                 float v[4];
                 gated4(v, at, gr, gnw, zs);
                 bfp8_quant4_store_lds(v, tid & 15, &L.xsc[tid >> 4], &L.xs[(tid >> 4) * 32], true);
@@ -693,7 +700,7 @@ extern "C" __global__ __launch_bounds__(kThreads + 64) void rt_chain_kernel(
             lds_barrier();
             small_terms<kHD / 64>(L, L.small[t & 1], w, lane);
             lds_barrier();
-            if (w == 0) small_sums<kHD / 64>(L, X + kWO + 2 * sub, lane);
+            if (w == 0) small_sums<kHD / 64>(L, X + kWO + kRowWords * sub, lane);
             add_words(X + kWO);
             ++t;
         }
@@ -715,7 +722,7 @@ extern "C" __global__ __launch_bounds__(kThreads + 64) void rt_chain_kernel(
         if (L.fail) return;
         small_terms<kMaxNb>(L, L.small[t & 1], w, lane);
         lds_barrier();
-        if (w == 0) small_sums<kMaxNb>(L, X + kWDown + 2 * sub, lane);
+        if (w == 0) small_sums<kMaxNb>(L, X + kWDown + kRowWords * sub, lane);
         ++t;
     }
 

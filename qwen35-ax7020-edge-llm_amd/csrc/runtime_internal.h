@@ -152,7 +152,8 @@ hipError_t rt_launch_rows(const RtRowsArgs& a, hipStream_t s);
 // the model's (hidden 1024, 16 heads of 128, MLP 3584).
 #define RT_CHAIN_WGS 256
 #define RT_CHAIN_MAX_LAYERS 24
-#define RT_CHAIN_LAYER_WORDS (512 + 512 + 3072 + 1024 + 1024 + 1024 + 1792)
+#define RT_CHAIN_ROW_WORDS 4  // a workgroup's four rows, twice: 32 bytes in one store
+#define RT_CHAIN_LAYER_WORDS (2 * RT_CHAIN_WGS * RT_CHAIN_ROW_WORDS + 3072 + 1024 + 1024 + 1024 + 1792)
 #define RT_CHAIN_SET_WORDS (RT_CHAIN_MAX_LAYERS * RT_CHAIN_LAYER_WORDS + 512)  // 512: the hidden state handed in
 struct RtChainLayer {     // device memory
     const uint8_t* mant[6];  // GPU planes: qkv, z, o, gate, up, down (an MLP layer: the last three)
