@@ -117,6 +117,7 @@ struct FwdLayer {
 };
 
 // Runs of layers in one launch (forward_chain.hip).
+constexpr int kChainRest = 256;
 constexpr uint64_t kChainWait = 25000000;  // 0.25 s of the 100 MHz clock: other streams' work may hold workgroups back
 struct Chain {
     std::vector<RtChainLayer> host;  // the layer table
@@ -127,6 +128,7 @@ struct Chain {
     int used[2] = {0, 0};            // words of each that are not clean
     PinnedBuf io;                    // ChainIo
     uint64_t wait_ticks = kChainWait;
+    int rest = 0;  // runs still to go as separate launches, after one gave up
 };
 // Host memory that the launches read and write.
 struct ChainIo {
@@ -625,6 +627,10 @@ ChainIo& chain_io() { return *static_cast<ChainIo*>(F.chain.io.p); }
 
 // Every layer in the table, and no per-step profile asked for.
 bool chain_ok(const std::vector<FwdLayer*>& layers) {
+    if (F.chain.rest > 0) {
+        --F.chain.rest;
+        return false;
+    }
     if (g_prof_on) return false;
     for (const FwdLayer* L : layers)
         if (L->slot < 0) return false;
@@ -686,6 +692,9 @@ int chain_done(const std::vector<FwdLayer*>& layers, int l, int e, bool* ok) {
     }
     HIP_OK(hipMemsetAsync(c.xch.p, 0xff, 2 * (size_t)RT_CHAIN_SET_WORDS * 8, g.stream));
     c.used[0] = c.used[1] = 0;
+    // a workgroup takes a CU's whole LDS: another process's run holds this one back, and
+    // would again
+    c.rest = kChainRest;
     return BFP8_OK;
 }
 
@@ -1111,6 +1120,7 @@ int forward_token_c(int token_id, float* h, const LinearLayerPlan* linear_plans,
 void qwen_debug_chain_wait(long long ticks) {
     std::lock_guard<std::mutex> lk(g.mu);
     F.chain.wait_ticks = ticks < 0 ? kChainWait : (uint64_t)ticks;
+    F.chain.rest = 0;
 }
 
 int qwen_forward_state_resident(int on) {
