@@ -637,9 +637,9 @@ bool chain_ok(const std::vector<FwdLayer*>& layers) {
     return chain_upload() == BFP8_OK;  // (no room for the table: separate launches)
 }
 
-// Layers [l, e) in one launch, from row `row` of the table (table != null) or
-// from io.h_in, the hidden state to io.h_out; with fnorm also its final norm
-// to ws.normed.  chain_done says whether it ran to its end.
+// Layers [l, e), no two with one state, in one launch, from row `row` of the
+// table (table != null) or from io.h_in, the hidden state to io.h_out; with fnorm
+// also its final norm to ws.normed.  chain_done says whether it ran to its end.
 int chain_launch(const std::vector<FwdLayer*>& layers, int l, int e, const uint16_t* table, int ntiles, int row,
                  const float* fnorm) {
     Chain& c = F.chain;
@@ -736,9 +736,19 @@ int separate_steps(const std::vector<FwdLayer*>& layers, int l, int e, float** h
     return add_pending(*hd, pending);
 }
 
+// Whether a layer of [l, e) advances the state that layer e does.  A run takes a
+// state's current buffer as its input and writes the other one, so it advances
+// each state once; plans may name the same buffers for several layers.
+bool state_in_run(const std::vector<FwdLayer*>& layers, int l, int e) {
+    for (int i = l; i < e; ++i)
+        if (layers[e]->st && layers[i]->st == layers[e]->st) return true;
+    return false;
+}
+
 // forward_token_c's layers and head, the layers in runs of one launch: up to
 // the next full-attention layer whose callback edits the hidden state on the
-// host, or to the end.  A run that gives up is done again by separate launches.
+// host, the next layer whose state the run advances already, or the end.  A run
+// that gives up is done again by separate launches.
 int token_chain(std::unique_lock<std::mutex>& lk, const std::vector<FwdLayer*>& layers, const int* layer_is_full,
                 FullAttnCallback cb, void* py_context, const uint16_t* table, int tiled, int row, const float* fnorm, float* h,
                 int* id) {
@@ -759,7 +769,7 @@ int token_chain(std::unique_lock<std::mutex>& lk, const std::vector<FwdLayer*>& 
             cb(l, h, py_context);
             lk.lock();
         }
-        for (e = l + 1; e < kLayers && !(layer_is_full[e] && cb); ++e) {}
+        for (e = l + 1; e < kLayers && !(layer_is_full[e] && cb) && !state_in_run(layers, l, e); ++e) {}
         const bool last = e == kLayers;
         ChainIo& io = chain_io();
         auto head = [&] {

@@ -439,6 +439,46 @@ def test_forward_state_resident_mode(gpu, fresh_cache):
 
 
 @pytest.mark.parametrize("resident", [0, 1])
+def test_layers_that_share_their_states(gpu, fresh_cache, resident):
+    """Linear layers of one token that name the same state buffers: neighbours,
+    layers of different stretches between callbacks, and one plan used twice.
+    Each reads what the one before it wrote, as in the oracle, which updates the
+    caller's buffers in place."""
+    lib = gpu.load()
+    lib.bfp8_cache_clear()
+    m = Model(2033)
+    for lin in (m.gpu_lin, m.ref_lin):
+        for i, j in ((1, 0), (5, 3), (17, 0)):
+            lin[i].conv_s, lin[i].state = lin[j].conv_s, lin[j].state
+        lin[4] = lin[2]
+
+    def body(layer, hp, ctx):
+        h = np.ctypeslib.as_array(ctypes.cast(hp, ctypes.POINTER(ctypes.c_float)), shape=(1024,))
+        h += np.float32(0.01 * (layer + 1))
+
+    cb, none = gpu.FULL_ATTN_CALLBACK(body), gpu.FULL_ATTN_CALLBACK()
+    rt = ol._rt()
+    rt.orc_forward_token.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                     ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, gpu.FULL_ATTN_CALLBACK,
+                                     ctypes.c_void_p, ctypes.c_int]
+    prev = lib.qwen_forward_state_resident(resident)
+    try:
+        with ol.cr_libm():
+            for token, c in ((77, none), (40001, cb), (78, none)):
+                say("layers that share their states", resident, token)
+                h, h_ref = np.zeros(1024, dtype=F32), np.zeros(1024, dtype=F32)
+                got = lib.forward_token_c(token, ptr(h), ctypes.addressof(m.gpu_lin), ctypes.addressof(m.gpu_mlp),
+                                          ptr(m.is_full), ptr(m.final_w), ptr(m.embed), c, None)
+                want = rt.orc_forward_token(token, ptr(h_ref), ctypes.addressof(m.ref_lin), ctypes.addressof(m.ref_mlp),
+                                            ptr(m.is_full), ptr(m.final_w), ptr(m.embed), c, None, 65536)
+                lib.qwen_forward_sync_state()
+                assert same(h, h_ref) and got == want, token
+                assert m.states_match(), token
+    finally:
+        lib.qwen_forward_state_resident(prev)
+
+
+@pytest.mark.parametrize("resident", [0, 1])
 def test_runs_of_layers_match_separate_launches(gpu, fresh_cache, resident):
     """A token's and a layer's runs in one launch, the separate launches (as
     while profiling), and runs that give up at once and are done again: the
