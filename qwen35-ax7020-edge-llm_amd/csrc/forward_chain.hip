@@ -753,7 +753,7 @@ bool rt_chain_fits() {
 }
 
 hipError_t rt_launch_chain(const RtChainArgs& a, hipStream_t s) {
-    if (a.n < 1 || a.n > RT_CHAIN_MAX_LAYERS || (!a.table && !a.h_in) || !a.h_out || !a.status || !a.xch ||
+    if (!a.layers || a.n < 1 || a.n > RT_CHAIN_MAX_LAYERS || (!a.table && !a.h_in) || !a.h_out || !a.status || !a.xch ||
         a.xch == a.xch_clear || (a.y_norm && !a.final_w))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(rt_chain_kernel, dim3(RT_CHAIN_WGS), dim3(kThreads + 64), 0, s, a);

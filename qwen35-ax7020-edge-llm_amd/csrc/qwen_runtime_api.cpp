@@ -328,14 +328,18 @@ void chain_add(FwdLayer* L) {
 }
 
 // The table's new entries to the device (no launch of this library is in
-// flight: its forward calls wait for theirs).
+// flight: its forward calls wait for theirs).  Where there is no room for a
+// larger table the old one stays, with the entries that it has.
 int chain_upload() {
     Chain& c = F.chain;
     const size_t n = c.host.size(), bytes = n * sizeof(RtChainLayer);
     if (c.uploaded == n) return BFP8_OK;
     if (bytes > c.layers.n) {
+        DevBuf larger;
+        if (int rc = larger.reserve(std::max<size_t>(2 * bytes, 64 * sizeof(RtChainLayer)))) return rc;
+        c.layers.release();
+        c.layers = larger;
         c.uploaded = 0;
-        if (int rc = c.layers.reserve(std::max<size_t>(2 * bytes, 64 * sizeof(RtChainLayer)))) return rc;
     }
     HIP_OK(hipMemcpy(c.layers.as<RtChainLayer>() + c.uploaded, c.host.data() + c.uploaded,
                      (n - c.uploaded) * sizeof(RtChainLayer), hipMemcpyHostToDevice));
@@ -625,16 +629,24 @@ int states_out(const std::vector<FwdLayer*>& layers) {
 // ---- runs of layers in one launch -------------------------------------------------------
 ChainIo& chain_io() { return *static_cast<ChainIo*>(F.chain.io.p); }
 
+// Every layer of [l, e) in the device's table (a layer seen while the device was
+// full is not).
+bool chain_has(const std::vector<FwdLayer*>& layers, int l, int e) {
+    int top = -1;
+    for (int i = l; i < e; ++i) {
+        if (layers[i]->slot < 0) return false;
+        top = std::max(top, layers[i]->slot);
+    }
+    return (size_t)top < F.chain.uploaded || chain_upload() == BFP8_OK;
+}
+
 // Every layer in the table, and no per-step profile asked for.
 bool chain_ok(const std::vector<FwdLayer*>& layers) {
     if (F.chain.rest > 0) {
         --F.chain.rest;
         return false;
     }
-    if (g_prof_on) return false;
-    for (const FwdLayer* L : layers)
-        if (L->slot < 0) return false;
-    return chain_upload() == BFP8_OK;  // (no room for the table: separate launches)
+    return !g_prof_on && chain_has(layers, 0, (int)layers.size());
 }
 
 // Layers [l, e), no two with one state, in one launch, from row `row` of the
@@ -776,12 +788,14 @@ int token_chain(std::unique_lock<std::mutex>& lk, const std::vector<FwdLayer*>& 
             return bf16_lm_head_dev(io.lm, reinterpret_cast<float*>(io.lm + 1), io.lm + 2, io.lm + 3, nullptr, w.normed, table,
                                     tiled, kVocab, kHidden, 1, 0, g.stream);
         };
-        if (!embed) memcpy(io.h_in, h, hb);
-        if ((rc = chain_launch(layers, l, e, embed ? table : nullptr, ntiles, row, last ? fnorm : nullptr))) return rc;
-        if (last && (rc = head())) return rc;
-        HIP_OK(hipStreamSynchronize(g.stream));
-        bool ok;
-        if ((rc = chain_done(layers, l, e, &ok))) return rc;
+        bool ok = chain_has(layers, l, e);  // (a callback's calls may have changed the table)
+        if (ok) {
+            if (!embed) memcpy(io.h_in, h, hb);
+            if ((rc = chain_launch(layers, l, e, embed ? table : nullptr, ntiles, row, last ? fnorm : nullptr))) return rc;
+            if (last && (rc = head())) return rc;
+            HIP_OK(hipStreamSynchronize(g.stream));
+            if ((rc = chain_done(layers, l, e, &ok))) return rc;
+        }
         if (ok) {
             memcpy(h, io.h_out, hb);
         } else {

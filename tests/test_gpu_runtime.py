@@ -478,6 +478,68 @@ def test_layers_that_share_their_states(gpu, fresh_cache, resident):
         lib.qwen_forward_state_resident(prev)
 
 
+def test_full_device_in_a_callback(gpu, fresh_cache):
+    """The callback calls the library with plans that it has not seen, and the
+    device has no room for what they add (rehearsed with
+    bfp8_debug_device_limit): those calls and the rest of the token are the
+    oracle's all the same."""
+    lib = gpu.load()
+    lib.bfp8_cache_clear()
+    m = Model(2034)
+    rng = np.random.default_rng(2034)
+    first = int(np.nonzero(m.is_full)[0][0])
+    x0 = normal(rng, 1024)
+    plans = []  # 41 more MLP layers, beside 24 of the token
+    for _ in range(41):
+        w = m._f(normal(rng, 1024, 0.1))
+        pair = (gpu.MlpPlan(), ol.MlpPlan())
+        for plan in pair:
+            plan.post_ln_w = ptr(w)
+            m._gemvs(plan, ("gate", "up", "down"))
+        plans.append(pair)
+    met = []
+
+    def body(layer, hp, ctx):
+        if layer == first and met:
+            x = x0.copy()
+            for i, (p, _) in enumerate(plans):
+                if i == len(plans) - 1:  # room for the last one's norm weights and no more
+                    lib.bfp8_debug_device_limit(lib.bfp8_device_bytes() + 4096)
+                lib.forward_mlp(ctypes.addressof(p), ptr(x))
+            met[0] = x
+        h = np.ctypeslib.as_array(ctypes.cast(hp, ctypes.POINTER(ctypes.c_float)), shape=(1024,))
+        h += np.float32(0.01 * (layer + 1))
+
+    def body_ref(layer, hp, ctx):
+        h = np.ctypeslib.as_array(ctypes.cast(hp, ctypes.POINTER(ctypes.c_float)), shape=(1024,))
+        h += np.float32(0.01 * (layer + 1))
+
+    cb, cb_ref = gpu.FULL_ATTN_CALLBACK(body), gpu.FULL_ATTN_CALLBACK(body_ref)
+    rt = ol._rt()
+    rt.orc_forward_token.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                     ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, gpu.FULL_ATTN_CALLBACK,
+                                     ctypes.c_void_p, ctypes.c_int]
+    try:
+        with ol.cr_libm():
+            for token in (5, 6, 7):
+                say("full device in a callback", token)
+                if token == 6:
+                    met.append(None)
+                h, h_ref = np.zeros(1024, dtype=F32), np.zeros(1024, dtype=F32)
+                got = lib.forward_token_c(token, ptr(h), ctypes.addressof(m.gpu_lin), ctypes.addressof(m.gpu_mlp),
+                                          ptr(m.is_full), ptr(m.final_w), ptr(m.embed), cb, None)
+                lib.bfp8_debug_device_limit(0)
+                want = rt.orc_forward_token(token, ptr(h_ref), ctypes.addressof(m.ref_lin), ctypes.addressof(m.ref_mlp),
+                                            ptr(m.is_full), ptr(m.final_w), ptr(m.embed), cb_ref, None, 65536)
+                assert same(h, h_ref) and got == want and m.states_match(), token
+            x = x0
+            for _, p in plans:
+                x = ol.forward_mlp(p, x)
+            assert same(met[0], x)
+    finally:
+        lib.bfp8_debug_device_limit(0)
+
+
 @pytest.mark.parametrize("resident", [0, 1])
 def test_runs_of_layers_match_separate_launches(gpu, fresh_cache, resident):
     """A token's and a layer's runs in one launch, the separate launches (as
