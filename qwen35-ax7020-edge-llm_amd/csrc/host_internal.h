@@ -57,16 +57,26 @@ struct ProfScope {
 inline size_t g_dev_bytes = 0;
 inline size_t g_dev_limit = 0;
 
+// Gives back what the library holds on the device only to be faster, if that
+// makes room for `bytes` more (false: nothing given back).  g.mu held.
+bool release_spare(size_t bytes);
+
 struct DevBuf {
     void* p = nullptr;
     size_t n = 0;
     // BFP8_ENOMEM when the device cannot hold `bytes` more (the buffer is then
     // empty and HIP's last-error state clear, so that the next launch check
-    // does not report this failure).
-    int reserve(size_t bytes) {
+    // does not report this failure).  spare: memory that a caller can do without,
+    // for which nothing else is given back.
+    int reserve(size_t bytes, bool spare = false) {
         if (bytes <= n) return BFP8_OK;
         release();
         const size_t want = std::max<size_t>(bytes, 256);
+        int rc = allocate(want);
+        if (rc == BFP8_ENOMEM && !spare && release_spare(want)) rc = allocate(want);
+        return rc;
+    }
+    int allocate(size_t want) {
         if (g_dev_limit && g_dev_bytes + want > g_dev_limit) {
             set_error("device memory: %zu more bytes exceed the limit of %zu", want, g_dev_limit);
             return BFP8_ENOMEM;

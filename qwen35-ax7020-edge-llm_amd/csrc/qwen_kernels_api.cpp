@@ -1254,10 +1254,8 @@ void* bfp8_plan_create(const bfp8_plan_item* items, int n) {
         set_error("bfp8_plan_create: no items");
         return nullptr;
     }
-    {
-        std::lock_guard<std::mutex> lk(g.mu);
-        if (ensure_init_locked() != BFP8_OK) return nullptr;
-    }
+    std::lock_guard<std::mutex> lk(g.mu);  // (throughout: an allocation may take the forward's spare memory)
+    if (ensure_init_locked() != BFP8_OK) return nullptr;
     Plan* p = new Plan();
     p->items.assign(items, items + n);
     int ntopk = 0;
@@ -1571,10 +1569,8 @@ int bfp8_plan_run(void* plan, void* stream) {
 void bfp8_plan_destroy(void* plan) {
     Plan* p = static_cast<Plan*>(plan);
     if (!p) return;
-    {
-        std::lock_guard<std::mutex> lk(g.mu);
-        if (g.ready) (void)hipDeviceSynchronize();
-    }
+    std::lock_guard<std::mutex> lk(g.mu);
+    if (g.ready) (void)hipDeviceSynchronize();
     release_plan(p);
     delete p;
 }

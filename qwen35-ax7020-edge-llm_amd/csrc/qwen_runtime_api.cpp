@@ -92,8 +92,9 @@ struct ParamKey {
 struct DevState {
     // [3][6144] taps and [16][128*128] blocked state, the current ones conv[cur]
     // and rec[rcur] (the separate launches update rec in place; rec[1] is there
-    // where the device holds it: the layer can run in a chain)
-    DevBuf buf;                              // all of them
+    // where the device has room for it: the layer can run in a chain)
+    DevBuf buf;                              // conv[0], conv[1], rec[0]
+    DevBuf spare;                            // rec[1]
     float *conv[2], *rec[2] = {nullptr, nullptr};
     int cur = 0, rcur = 0;
     float* host_conv;     // the caller's buffers
@@ -129,6 +130,8 @@ struct Chain {
     PinnedBuf io;                    // ChainIo
     uint64_t wait_ticks = kChainWait;
     int rest = 0;  // runs still to go as separate launches, after one gave up
+    bool in_flight = false;
+    bool off = false;  // its memory was given back: separate launches until the caches are cleared
 };
 // Host memory that the launches read and write.
 struct ChainIo {
@@ -249,15 +252,12 @@ int fwd_state(float* conv_s, float* state, DevState** out) {
     }
     std::unique_ptr<DevState> st(new DevState());
     constexpr size_t nc = (size_t)3 * kConv, nr = (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM;
-    const bool two = rt_chain_fits() && st->buf.reserve((2 * nc + 2 * nr) * 4) == BFP8_OK;
-    if (!two)
-        if (int rc = st->buf.reserve((2 * nc + nr) * 4)) return rc;
+    if (int rc = st->buf.reserve((2 * nc + nr) * 4)) return rc;
     float* p = st->buf.as<float>();
     st->rec[0] = p;
-    if (two) st->rec[1] = p + nr;
-    p += two ? 2 * nr : nr;
-    st->conv[0] = p;
-    st->conv[1] = p + nc;
+    st->conv[0] = p + nr;
+    st->conv[1] = p + nr + nc;
+    if (rt_chain_fits() && !F.chain.off && st->spare.reserve(nr * 4, true) == BFP8_OK) st->rec[1] = st->spare.as<float>();
     st->host_conv = conv_s;
     st->host_rec = state;
     HIP_OK(hipMemcpy(st->conv[0], conv_s, (size_t)3 * kConv * 4, hipMemcpyHostToDevice));
@@ -291,7 +291,7 @@ std::vector<char> key_of(const void* p, size_t n, char tag) {
 // Enters a layer into the chain's table, where it fits (else slot stays -1).
 void chain_add(FwdLayer* L) {
     Chain& c = F.chain;
-    if (!rt_chain_fits() || c.host.size() >= 0xffff) return;
+    if (!rt_chain_fits() || c.off || c.host.size() >= 0xffff) return;
     RtChainLayer y{};
     for (int i = 0; i < (L->linear ? 6 : 3); ++i) {
         y.mant[L->linear ? i : 3 + i] = L->w[i].mant;
@@ -316,7 +316,7 @@ void chain_add(FwdLayer* L) {
     }
     constexpr size_t kSet = (size_t)RT_CHAIN_SET_WORDS * 8;
     if (!c.xch.p) {
-        if (c.xch.reserve(2 * kSet) || hipMemsetAsync(c.xch.p, 0xff, 2 * kSet, g.stream) != hipSuccess) {
+        if (c.xch.reserve(2 * kSet, true) || hipMemsetAsync(c.xch.p, 0xff, 2 * kSet, g.stream) != hipSuccess) {
             c.xch.release();
             return;
         }
@@ -336,7 +336,7 @@ int chain_upload() {
     if (c.uploaded == n) return BFP8_OK;
     if (bytes > c.layers.n) {
         DevBuf larger;
-        if (int rc = larger.reserve(std::max<size_t>(2 * bytes, 64 * sizeof(RtChainLayer)))) return rc;
+        if (int rc = larger.reserve(std::max<size_t>(2 * bytes, 64 * sizeof(RtChainLayer)), true)) return rc;
         c.layers.release();
         c.layers = larger;
         c.uploaded = 0;
@@ -683,6 +683,7 @@ int chain_launch(const std::vector<FwdLayer*>& layers, int l, int e, const uint1
     a.status = &io.status;
     io.status = 0;
     RT_LAUNCH(rt_launch_chain(a, g.stream));
+    c.in_flight = true;
     c.used[c.set] = a.n * RT_CHAIN_LAYER_WORDS + RT_HIDDEN / 2;
     c.used[c.set ^ 1] = 0;
     c.set ^= 1;
@@ -693,6 +694,7 @@ int chain_launch(const std::vector<FwdLayer*>& layers, int l, int e, const uint1
 // (*ok), or it gave up, and nothing of it counts (!*ok).
 int chain_done(const std::vector<FwdLayer*>& layers, int l, int e, bool* ok) {
     Chain& c = F.chain;
+    c.in_flight = false;
     *ok = __atomic_load_n(&chain_io().status, __ATOMIC_ACQUIRE) == 0;
     if (*ok) {
         for (int i = l; i < e; ++i) {
@@ -816,6 +818,13 @@ int token_chain(std::unique_lock<std::mutex>& lk, const std::vector<FwdLayer*>& 
     return BFP8_OK;
 }
 
+void drop_chain() {
+    F.chain.host.clear();
+    F.chain.uploaded = 0;
+    F.chain.layers.release();
+    F.chain.xch.release();
+}
+
 void drop_forward() {
     F.layers.clear();
     for (auto& kv : F.params) kv.second.release();
@@ -827,15 +836,45 @@ void drop_forward() {
     F.planes.clear();
     for (auto& kv : F.states) {
         kv.second->buf.release();
+        kv.second->spare.release();
     }
     F.states.clear();
-    F.chain.host.clear();
-    F.chain.uploaded = 0;
-    F.chain.layers.release();
-    F.chain.xch.release();
+    drop_chain();
+    F.chain.off = false;
 }
 
 }  // namespace
+
+// The chain's memory and the states' second buffers: about 1 MB a layer, without
+// which the layers run as separate launches.
+bool release_spare(size_t bytes) {
+    Chain& c = F.chain;
+    size_t held = c.xch.n + c.layers.n;
+    for (auto& kv : F.states) held += kv.second->spare.n;
+    if (!held || c.in_flight) return false;
+    size_t room = 0, total = 0;
+    if (g_dev_limit)
+        room = g_dev_limit > g_dev_bytes ? g_dev_limit - g_dev_bytes : 0;
+    else if (hipMemGetInfo(&room, &total) != hipSuccess)
+        return false;
+    if (room + held < bytes) return false;
+    for (auto& kv : F.states) {  // a state in its second buffer moves to the first
+        DevState* st = kv.second.get();
+        if (st->rcur && hipMemcpyAsync(st->rec[0], st->rec[1], st->spare.n, hipMemcpyDeviceToDevice, g.stream) != hipSuccess)
+            return false;
+    }
+    if (hipStreamSynchronize(g.stream) != hipSuccess) return false;
+    for (auto& kv : F.states) {
+        DevState* st = kv.second.get();
+        st->rcur = 0;
+        st->rec[1] = nullptr;
+        st->spare.release();
+    }
+    for (auto& kv : F.layers) kv.second->slot = -1;
+    drop_chain();
+    c.off = true;
+    return true;
+}
 
 // Called by bfp8_cache_clear (lock held).
 void forward_cache_clear() { drop_forward(); }
@@ -1083,6 +1122,8 @@ int forward_token_c(int token_id, float* h, const LinearLayerPlan* linear_plans,
     } else {
         RT_CHECK("forward_token_c", fwd_vec(embed_table, (size_t)kVocab * kHidden, &table));
     }
+    // the lm_head's lists, before a run of layers is in flight (nothing is given back then)
+    RT_CHECK("forward_token_c", scratch_for(g.stream).partials.reserve((size_t)bfp8_ntiles(kVocab) * 8));
     int row = token_id % kVocab;
     if (row < 0) row += kVocab;
     if (chain_ok(layers)) {

@@ -541,6 +541,73 @@ def test_full_device_in_a_callback(gpu, fresh_cache):
 
 
 @pytest.mark.parametrize("resident", [0, 1])
+def test_full_device_gives_up_the_second_states(gpu, fresh_cache, resident):
+    """What the forward holds only to run its layers in one launch gives way: on
+    a device that is full (rehearsed with bfp8_debug_device_limit) but for it, a
+    call with a new plan, and a token from cold on a device that holds the rest
+    of the model and not that, give the oracle's results; room that stays too
+    small is still an error, and takes nothing away."""
+    lib = gpu.load()
+    lib.bfp8_cache_clear()
+    m = Model(2035)
+    rng = np.random.default_rng(2035)
+    post = m._f(normal(rng, 1024, 0.1))
+    gp, rp = gpu.MlpPlan(), ol.MlpPlan()
+    for plan in (gp, rp):
+        plan.post_ln_w = ptr(post)
+        m._gemvs(plan, ("gate", "up", "down"))
+    none = gpu.FULL_ATTN_CALLBACK()
+    rt = ol._rt()
+    rt.orc_forward_token.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                     ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, gpu.FULL_ATTN_CALLBACK,
+                                     ctypes.c_void_p, ctypes.c_int]
+
+    def token(t):
+        say("full device, token", resident, t, lib.bfp8_device_bytes())
+        h, h_ref = np.zeros(1024, dtype=F32), np.zeros(1024, dtype=F32)
+        got = lib.forward_token_c(t, ptr(h), ctypes.addressof(m.gpu_lin), ctypes.addressof(m.gpu_mlp), ptr(m.is_full),
+                                  ptr(m.final_w), ptr(m.embed), none, None)
+        want = rt.orc_forward_token(t, ptr(h_ref), ctypes.addressof(m.ref_lin), ctypes.addressof(m.ref_mlp),
+                                    ptr(m.is_full), ptr(m.final_w), ptr(m.embed), none, None, 65536)
+        lib.qwen_forward_sync_state()
+        assert same(h, h_ref) and got == want and m.states_match(), t
+
+    seconds = 18 * 16 * 128 * 128 * 4  # bytes of the second states
+    prev = lib.qwen_forward_state_resident(resident)
+    try:
+        with ol.cr_libm():
+            token(11)
+            # a table that no memory given back makes room for (the first call lets go of the per-call buffer)
+            V, H = 1 << 20, 1024
+            table = np.zeros(V * H, dtype=np.uint16)
+            x = normal(rng, H)
+            ids, sc = np.zeros(4, dtype=np.int32), np.zeros(4, dtype=F32)
+            for _ in range(2):
+                held = lib.bfp8_device_bytes()
+                lib.bfp8_debug_device_limit(held)
+                assert lib.qwen_lm_head_topk_bf16(ptr(x), ptr(table), V, H, 4, ptr(ids), ptr(sc)) == 0
+            assert lib.bfp8_device_bytes() == held
+            h = x.copy()
+            lib.forward_mlp(ctypes.addressof(gp), ptr(h))
+            assert same(h, ol.forward_mlp(rp, x))
+            assert lib.bfp8_device_bytes() <= held - seconds
+            lib.bfp8_debug_device_limit(0)
+            token(12)
+            lib.bfp8_cache_clear()
+            lib.bfp8_debug_device_limit(held - seconds // 2)
+            token(13)
+            token(14)
+            assert lib.bfp8_device_bytes() <= held - seconds
+            lib.bfp8_debug_device_limit(0)
+            lib.bfp8_cache_clear()
+            token(15)  # as at first
+            assert lib.bfp8_device_bytes() > held - seconds // 2
+    finally:
+        lib.bfp8_debug_device_limit(0)
+        lib.qwen_forward_state_resident(prev)
+
+
+@pytest.mark.parametrize("resident", [0, 1])
 def test_runs_of_layers_match_separate_launches(gpu, fresh_cache, resident):
     """A token's and a layer's runs in one launch, the separate launches (as
     while profiling), and runs that give up at once and are done again: the
