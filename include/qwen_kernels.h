@@ -266,11 +266,18 @@ size_t bfp8_device_bytes(void);
  * without an error channel (bfp8_gemv and the other void entry points),
  * aborts. */
 void bfp8_debug_device_limit(size_t bytes);
-/* Testing aid: the wait, in ticks of the GPU's 100 MHz clock, after which a
- * launch of a run of layers gives up on its other workgroups and the forward
- * calls repeat the run by separate launches (0: at the first vector that is
- * not there yet; negative: the default, a quarter of a second). */
+/* Testing aids for the forward's runs of layers in one launch, whose workgroups
+ * wait for one another.  qwen_debug_chain_wait: the wait, in ticks of the GPU's
+ * 100 MHz clock, after which such a run gives up and the forward call does it
+ * again by separate launches, as it then does the rest of the token and the
+ * next 4 calls (twice as many each time, up to 65,536).  0: gives up at the
+ * first vector that is not there yet; negative: the default, 2 ms.  Ends such a
+ * rest.  qwen_debug_chain_rest: the calls that a rest still has; sets them
+ * if calls >= 0.  qwen_debug_chain_runs: the runs so far that ended and that
+ * gave up. */
 void qwen_debug_chain_wait(long long ticks);
+int qwen_debug_chain_rest(int calls);
+void qwen_debug_chain_runs(long long* done, long long* gave_up);
 
 /* ---- 3. device-level symbols ------------------------------------------------ */
 

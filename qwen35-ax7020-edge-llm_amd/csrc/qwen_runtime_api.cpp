@@ -118,8 +118,19 @@ struct FwdLayer {
 };
 
 // Runs of layers in one launch (forward_chain.hip).
-constexpr int kChainRest = 256;
-constexpr uint64_t kChainWait = 25000000;  // 0.25 s of the 100 MHz clock: other streams' work may hold workgroups back
+// A run takes under 0.5 ms once its workgroups are all there.  Other work on the
+// GPU may hold some of them back: longer than kChainWait (2 ms of the 100 MHz
+// clock) and the run gives up and is done again by separate launches, as are
+// the rest of the token and the next calls.  Two processes that both run the
+// forward hold back each other's workgroups now and then (one run in about 500),
+// and a process whose separate launches go in between the other's runs is the
+// slower one, so the rest is short; it doubles when the next run gives up too (and
+// shortens by a call with each run that ends), so that work which never lets go of
+// a CU costs 2 ms once in 65,536 calls.  Two such processes, four tokens: 3.75 ms
+// each (1.94 alone; 3.2 if both only ever took separate launches), at most 10;
+// with a wait of 0.25 s and a rest of 256, 6.1 and 506.
+constexpr uint64_t kChainWait = 200000;
+constexpr int kChainRest = 4, kChainRestMax = 65536;
 struct Chain {
     std::vector<RtChainLayer> host;  // the layer table
     DevBuf layers;                   // ... its device copy, the first `uploaded` entries
@@ -129,7 +140,9 @@ struct Chain {
     int used[2] = {0, 0};            // words of each that are not clean
     PinnedBuf io;                    // ChainIo
     uint64_t wait_ticks = kChainWait;
-    int rest = 0;  // runs still to go as separate launches, after one gave up
+    int rest = 0;                // calls still to go as separate launches, after a run gave up
+    int next_rest = kChainRest;  // ... when the next one does
+    long long done = 0, gave_up = 0;  // runs
     bool in_flight = false;
     bool off = false;  // its memory was given back: separate launches until the caches are cleared
 };
@@ -697,6 +710,8 @@ int chain_done(const std::vector<FwdLayer*>& layers, int l, int e, bool* ok) {
     c.in_flight = false;
     *ok = __atomic_load_n(&chain_io().status, __ATOMIC_ACQUIRE) == 0;
     if (*ok) {
+        ++c.done;
+        c.next_rest = std::max(c.next_rest - 1, kChainRest);
         for (int i = l; i < e; ++i) {
             if (!layers[i]->linear) continue;
             layers[i]->st->cur ^= 1;
@@ -704,11 +719,11 @@ int chain_done(const std::vector<FwdLayer*>& layers, int l, int e, bool* ok) {
         }
         return BFP8_OK;
     }
+    ++c.gave_up;
     HIP_OK(hipMemsetAsync(c.xch.p, 0xff, 2 * (size_t)RT_CHAIN_SET_WORDS * 8, g.stream));
     c.used[0] = c.used[1] = 0;
-    // a workgroup takes a CU's whole LDS: another process's run holds this one back, and
-    // would again
-    c.rest = kChainRest;
+    c.rest = c.next_rest;
+    c.next_rest = std::min(2 * c.next_rest, kChainRestMax);
     return BFP8_OK;
 }
 
@@ -790,7 +805,8 @@ int token_chain(std::unique_lock<std::mutex>& lk, const std::vector<FwdLayer*>& 
             return bf16_lm_head_dev(io.lm, reinterpret_cast<float*>(io.lm + 1), io.lm + 2, io.lm + 3, nullptr, w.normed, table,
                                     tiled, kVocab, kHidden, 1, 0, g.stream);
         };
-        bool ok = chain_has(layers, l, e);  // (a callback's calls may have changed the table)
+        // (an earlier run of the token may have given up, a callback's calls may have changed the table)
+        bool ok = F.chain.rest == 0 && chain_has(layers, l, e);
         if (ok) {
             if (!embed) memcpy(io.h_in, h, hb);
             if ((rc = chain_launch(layers, l, e, embed ? table : nullptr, ntiles, row, last ? fnorm : nullptr))) return rc;
@@ -1186,6 +1202,20 @@ void qwen_debug_chain_wait(long long ticks) {
     std::lock_guard<std::mutex> lk(g.mu);
     F.chain.wait_ticks = ticks < 0 ? kChainWait : (uint64_t)ticks;
     F.chain.rest = 0;
+    F.chain.next_rest = kChainRest;
+}
+
+int qwen_debug_chain_rest(int calls) {
+    std::lock_guard<std::mutex> lk(g.mu);
+    const int prev = F.chain.rest;
+    if (calls >= 0) F.chain.rest = calls;
+    return prev;
+}
+
+void qwen_debug_chain_runs(long long* done, long long* gave_up) {
+    std::lock_guard<std::mutex> lk(g.mu);
+    if (done) *done = F.chain.done;
+    if (gave_up) *gave_up = F.chain.gave_up;
 }
 
 int qwen_forward_state_resident(int on) {

@@ -155,6 +155,10 @@ def bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.bfp8_debug_device_limit.restype = None
     lib.qwen_debug_chain_wait.argtypes = [ctypes.c_longlong]
     lib.qwen_debug_chain_wait.restype = None
+    lib.qwen_debug_chain_rest.argtypes = [i]
+    lib.qwen_debug_chain_rest.restype = i
+    lib.qwen_debug_chain_runs.argtypes = [ctypes.POINTER(ctypes.c_longlong)] * 2
+    lib.qwen_debug_chain_runs.restype = None
     # device level
     for name in ("bfp8_dev_mant_bytes", "bfp8_dev_exps_bytes"):
         getattr(lib, name).argtypes = [i, i]

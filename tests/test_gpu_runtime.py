@@ -655,6 +655,84 @@ def test_runs_of_layers_match_separate_launches(gpu, fresh_cache, resident):
             assert a == b if isinstance(a, int) else same(a, b), (mode, i)
 
 
+def chain_runs(lib):
+    done, gave_up = ctypes.c_longlong(), ctypes.c_longlong()
+    lib.qwen_debug_chain_runs(ctypes.byref(done), ctypes.byref(gave_up))
+    return np.array([done.value, gave_up.value])
+
+
+def test_rest_after_a_run_gave_up(gpu, fresh_cache):
+    """A token of seven runs whose first gives up: the others are not tried, nor
+    are the next four calls' runs; then layers run in one launch again.  The rest
+    doubles when the first run behind it gives up as well, up to its limit, and
+    shortens with the runs that end.  Results and states are the oracle's
+    throughout."""
+    lib = gpu.load()
+    lib.bfp8_cache_clear()
+    m = Model(2036)
+    rng = np.random.default_rng(2036)
+
+    def body(layer, hp, ctx):
+        h = np.ctypeslib.as_array(ctypes.cast(hp, ctypes.POINTER(ctypes.c_float)), shape=(1024,))
+        h += np.float32(0.01 * (layer + 1))
+
+    cb = gpu.FULL_ATTN_CALLBACK(body)
+    rt = ol._rt()
+    rt.orc_forward_token.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                     ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, gpu.FULL_ATTN_CALLBACK,
+                                     ctypes.c_void_p, ctypes.c_int]
+
+    def token(t):
+        h, h_ref = np.zeros(1024, dtype=F32), np.zeros(1024, dtype=F32)
+        got = lib.forward_token_c(t, ptr(h), ctypes.addressof(m.gpu_lin), ctypes.addressof(m.gpu_mlp), ptr(m.is_full),
+                                  ptr(m.final_w), ptr(m.embed), cb, None)
+        want = rt.orc_forward_token(t, ptr(h_ref), ctypes.addressof(m.ref_lin), ctypes.addressof(m.ref_mlp),
+                                    ptr(m.is_full), ptr(m.final_w), ptr(m.embed), cb, None, 65536)
+        assert same(h, h_ref) and got == want and m.states_match(), t
+
+    x = normal(rng, 1024)
+    y = ol.forward_mlp(m.ref_mlp[3], x)
+
+    def mlps(n):
+        for i in range(n):
+            h = x.copy()
+            lib.forward_mlp(ctypes.addressof(m.gpu_mlp[3]), ptr(h))
+            assert same(h, y), i
+
+    try:
+        with ol.cr_libm():
+            say("rest: a token that gives up")
+            lib.qwen_debug_chain_wait(0)
+            at = chain_runs(lib)
+            token(21)
+            assert list(chain_runs(lib) - at) == [0, 1] and lib.qwen_debug_chain_rest(-1) == 4
+            lib.qwen_debug_chain_wait(-1)
+            lib.qwen_debug_chain_rest(4)
+            say("rest: four calls")
+            token(22)
+            mlps(3)
+            assert list(chain_runs(lib) - at) == [0, 1] and lib.qwen_debug_chain_rest(-1) == 0
+            say("rest: runs again")
+            h = x.copy()
+            lib.forward_linear_layer(ctypes.addressof(m.gpu_lin[4]), ptr(h))
+            assert same(h, ol.forward_linear_layer(m.ref_lin[4], x)) and m.states_match()
+            token(23)
+            mlps(1)
+            assert list(chain_runs(lib) - at) == [1 + 7 + 1, 1]
+            say("rest: gives up again and again")
+            lib.qwen_debug_chain_wait(0)
+            at = chain_runs(lib)
+            for i in range(16):
+                mlps(1)
+                assert list(chain_runs(lib) - at) == [0, i + 1]
+                assert lib.qwen_debug_chain_rest(min(i, 2)) == min(4 << i, 65536)
+                mlps(min(i, 2))  # (the rest cut short)
+            token(24)
+            assert list(chain_runs(lib) - at) == [0, 17] and lib.qwen_debug_chain_rest(-1) == 65536
+    finally:
+        lib.qwen_debug_chain_wait(-1)
+
+
 def test_profiler_slots(gpu, model):
     lib = gpu.load()
     assert lib.qwen_prof_count() == 15
