@@ -10,8 +10,10 @@
 //
 //   * a produced vector goes out as 64-bit words of two floats, one agent-scope
 //     atomic store each, and a consumer re-reads the words that it needs until
-//     none is the "not yet" pattern (all ones: a NaN that no operation gives;
-//     a float pair that happens to carry it is stored as the canonical NaN).
+//     none is the "not yet" pattern (all ones: a NaN that no operation gives, but
+//     passes on; a float pair that carries it is stored as the canonical NaN,
+//     which makes no difference but in the hidden state handed in, and the host
+//     takes separate launches for one with such a pair).
 //     Data and flag are one word, so no fence and no second round trip.  Every
 //     (layer, vector) has words of its own, and a launch that follows uses the
 //     other of two sets, which this one leaves cleared;

@@ -662,6 +662,18 @@ bool chain_ok(const std::vector<FwdLayer*>& layers) {
     return !g_prof_on && chain_has(layers, 0, (int)layers.size());
 }
 
+// Whether a run can hand h on as it is: no pair of its words is all ones, the
+// pattern of a pair that is not there yet (NaNs whose bits would be lost).
+bool chain_takes(const float* h) {
+    uint64_t found = 0;
+    for (int i = 0; i < kHidden; i += 2) {
+        uint64_t v;
+        memcpy(&v, h + i, 8);
+        found |= v == ~0ull;
+    }
+    return !found;
+}
+
 // Layers [l, e), no two with one state, in one launch, from row `row` of the
 // table (table != null) or from io.h_in, the hidden state to io.h_out; with fnorm
 // also its final norm to ws.normed.  chain_done says whether it ran to its end.
@@ -731,7 +743,7 @@ int layer_call(const FwdLayer& L, float* h, int slot) {
     const double t0 = g_prof_on ? now_ms() : 0.0;
     int rc;
     const std::vector<FwdLayer*> one{const_cast<FwdLayer*>(&L)};
-    if (chain_ok(one)) {
+    if (chain_ok(one) && chain_takes(h)) {
         if ((rc = states_in(one))) return rc;
         memcpy(chain_io().h_in, h, (size_t)kHidden * 4);
         if ((rc = chain_launch(one, 0, 1, nullptr, 0, 0, nullptr))) return rc;
@@ -806,7 +818,7 @@ int token_chain(std::unique_lock<std::mutex>& lk, const std::vector<FwdLayer*>& 
                                     tiled, kVocab, kHidden, 1, 0, g.stream);
         };
         // (an earlier run of the token may have given up, a callback's calls may have changed the table)
-        bool ok = F.chain.rest == 0 && chain_has(layers, l, e);
+        bool ok = F.chain.rest == 0 && chain_has(layers, l, e) && (embed || chain_takes(h));
         if (ok) {
             if (!embed) memcpy(io.h_in, h, hb);
             if ((rc = chain_launch(layers, l, e, embed ? table : nullptr, ntiles, row, last ? fnorm : nullptr))) return rc;

@@ -733,6 +733,45 @@ def test_rest_after_a_run_gave_up(gpu, fresh_cache):
         lib.qwen_debug_chain_wait(-1)
 
 
+def test_nan_payloads_of_the_hidden_state(gpu, fresh_cache):
+    """Pairs of NaNs with every bit set, which stand for "not there yet" where
+    runs of layers hand vectors on: the hidden state comes back with the bits
+    that the separate launches (as while profiling) leave."""
+    lib = gpu.load()
+    ones = np.full(4, 0xFFFFFFFF, np.uint32).view(F32)
+
+    def body(layer, hp, ctx):
+        h = np.ctypeslib.as_array(ctypes.cast(hp, ctypes.POINTER(ctypes.c_float)), shape=(1024,))
+        if layer == 11:
+            h[510:514] = ones
+
+    cb = gpu.FULL_ATTN_CALLBACK(body)
+
+    def run(separate):
+        lib.bfp8_cache_clear()
+        m = Model(2037)
+        rng = np.random.default_rng(2037)
+        out = []
+        try:
+            lib.qwen_prof_enable(1 if separate else 0)
+            for at in (0, 511, 1020):
+                h = normal(rng, 1024)
+                h[at:at + 4] = ones
+                say("NaN payloads", separate, at)
+                lib.forward_mlp(ctypes.addressof(m.gpu_mlp[3]), ptr(h))
+                lib.forward_linear_layer(ctypes.addressof(m.gpu_lin[0]), ptr(h))
+                out.append(h)
+            h = np.zeros(1024, dtype=F32)
+            lib.forward_token_c(5, ptr(h), ctypes.addressof(m.gpu_lin), ctypes.addressof(m.gpu_mlp), ptr(m.is_full),
+                                ptr(m.final_w), ptr(m.embed), cb, None)
+            return [a.view(np.uint32) for a in out + [h] + [a for st in m.gpu_states for a in st]]
+        finally:
+            lib.qwen_prof_enable(0)
+
+    for i, (a, b) in enumerate(zip(run(False), run(True))):
+        assert np.array_equal(a, b), i
+
+
 def test_profiler_slots(gpu, model):
     lib = gpu.load()
     assert lib.qwen_prof_count() == 15
