@@ -438,6 +438,12 @@ def test_forward_state_resident_mode(gpu, fresh_cache):
         lib.qwen_forward_state_resident(prev)
 
 
+def chain_runs(lib):
+    done, gave_up = ctypes.c_longlong(), ctypes.c_longlong()
+    lib.qwen_debug_chain_runs(ctypes.byref(done), ctypes.byref(gave_up))
+    return np.array([done.value, gave_up.value])
+
+
 @pytest.mark.parametrize("resident", [0, 1])
 def test_layers_that_share_their_states(gpu, fresh_cache, resident):
     """Linear layers of one token that name the same state buffers: neighbours,
@@ -466,6 +472,7 @@ def test_layers_that_share_their_states(gpu, fresh_cache, resident):
         with ol.cr_libm():
             for token, c in ((77, none), (40001, cb), (78, none)):
                 say("layers that share their states", resident, token)
+                at = chain_runs(lib)
                 h, h_ref = np.zeros(1024, dtype=F32), np.zeros(1024, dtype=F32)
                 got = lib.forward_token_c(token, ptr(h), ctypes.addressof(m.gpu_lin), ctypes.addressof(m.gpu_mlp),
                                           ptr(m.is_full), ptr(m.final_w), ptr(m.embed), c, None)
@@ -474,6 +481,8 @@ def test_layers_that_share_their_states(gpu, fresh_cache, resident):
                 lib.qwen_forward_sync_state()
                 assert same(h, h_ref) and got == want, token
                 assert m.states_match(), token
+                # layers 0 | 1 .. 4 | 5 .. 23; with the callback 0 | 1, 2 | 3 .. 5 | 6 | 7 .. 10 | .. | 23
+                assert list(chain_runs(lib) - at) == [9 if c is cb else 3, 0], token
     finally:
         lib.qwen_forward_state_resident(prev)
 
@@ -612,7 +621,8 @@ def test_runs_of_layers_match_separate_launches(gpu, fresh_cache, resident):
     """A token's and a layer's runs in one launch, the separate launches (as
     while profiling), and runs that give up at once and are done again: the
     same hidden states, ids and recurrent states, bit for bit, over calls that
-    alternate between the three, with the callback and without."""
+    alternate between the three, with the callback and without.  The library's
+    counts of runs say that each call went the way that it is here to test."""
     lib = gpu.load()
 
     def body(layer, hp, ctx):
@@ -633,14 +643,22 @@ def test_runs_of_layers_match_separate_launches(gpu, fresh_cache, resident):
                 separate = mode == "separate" or (mode == "mixed" and step % 2)
                 lib.qwen_prof_enable(1 if separate else 0)
                 lib.qwen_debug_chain_wait(0 if mode == "gives up" else -1)
+                at = chain_runs(lib)
                 h = np.zeros(1024, dtype=F32)
                 out.append(lib.forward_token_c(token, ptr(h), ctypes.addressof(m.gpu_lin), ctypes.addressof(m.gpu_mlp),
                                                ptr(m.is_full), ptr(m.final_w), ptr(m.embed), c, None))
                 out.append(h)
                 h = h * np.float32(0.5)
+                if mode == "gives up":  # (each call: one that gave up rests the next ones)
+                    lib.qwen_debug_chain_wait(0)
                 lib.forward_linear_layer(ctypes.addressof(m.gpu_lin[step]), ptr(h))
+                if mode == "gives up":
+                    lib.qwen_debug_chain_wait(0)
                 lib.forward_mlp(ctypes.addressof(m.gpu_mlp[3]), ptr(h))
                 out.append(h)
+                token_runs = 7 if c is cb else 1  # (the callback ends a run; layer 0 is no full-attention layer)
+                runs = [0, 3] if mode == "gives up" else [0, 0] if separate else [token_runs + 2, 0]
+                assert list(chain_runs(lib) - at) == runs, (mode, step)
             lib.qwen_forward_sync_state()
             return out + [a.copy() for st in m.gpu_states for a in st]
         finally:
@@ -653,12 +671,6 @@ def test_runs_of_layers_match_separate_launches(gpu, fresh_cache, resident):
         got = run(mode)
         for i, (a, b) in enumerate(zip(got, want)):
             assert a == b if isinstance(a, int) else same(a, b), (mode, i)
-
-
-def chain_runs(lib):
-    done, gave_up = ctypes.c_longlong(), ctypes.c_longlong()
-    lib.qwen_debug_chain_runs(ctypes.byref(done), ctypes.byref(gave_up))
-    return np.array([done.value, gave_up.value])
 
 
 def test_rest_after_a_run_gave_up(gpu, fresh_cache):
