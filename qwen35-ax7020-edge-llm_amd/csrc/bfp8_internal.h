@@ -238,12 +238,15 @@ hipError_t bfp8_noalloc_setup(void** out);
 // Per-tile top-`topk` partials ([ntiles(n)][topk] keys) of logits[0, n), for
 // bfp8_launch_topk_merge (topk <= BFP8_TOPK_MAX).
 hipError_t bfp8_launch_select_partials(const float* logits, int n, int topk, uint64_t* partials, hipStream_t s);
-// The kk best of logits[0, n) (kk > BFP8_TOPK_MAX): 4096-key blocks sorted
-// in LDS, then ranked (n <= BFP8_SELECT_RANK_MAX), else all n keys sorted by
-// one workgroup; keys: bfp8_select_scratch_bytes(n) of scratch.  ids /
-// scores [kk], count, argmax as the merge writes them.
+// The kk best of logits[0, n) (kk > BFP8_TOPK_MAX): kk <= 512 of n <= 65,536
+// from sorted 64-row tiles by one workgroup; beyond, 2048-key blocks sorted in
+// LDS, then ranked (n <= BFP8_SELECT_RANK_MAX), else all n keys sorted by one
+// workgroup.  keys: bfp8_select_scratch_bytes(n) of scratch.  ids / scores [kk],
+// count, argmax as the merge writes them.
 hipError_t bfp8_launch_select_sort(const float* logits, int n, int kk, uint64_t* keys, int* ids, float* scores,
                                    int* count, int* argmax, hipStream_t s);
+// The main kernel of the selection of kk (any) of n logits.
+const char* bfp8_select_kernel_name(int n, int kk);
 hipError_t bfp8_launch_sample(const Bfp8SampleArgs& a, hipStream_t s);
 
 // ---- bfp8_ieee.hip -------------------------------------------------------

@@ -1546,8 +1546,7 @@ const char* bfp8_plan_kernel_name(void* plan, int stage) {
     if (stage == 2) {
         if (!p->odd_items.empty()) return "bfp8_tail_row_kernel";
         if (!p->float_items.empty()) return "bfp8_gemv_float_kernel";
-        if (p->gen_head >= 0)
-            return p->gen_out.topk <= BFP8_TOPK_MAX ? "bfp8_select_partials_kernel" : "bfp8_select_sort_kernel";
+        if (p->gen_head >= 0) return bfp8_select_kernel_name(p->gen_out.M, p->gen_out.topk);
         return "";
     }
     return "";

@@ -786,10 +786,28 @@ hipError_t bfp8_launch_select_partials(const float* logits, int n, int topk, uin
     return hipGetLastError();
 }
 
+namespace {
+enum class SelectForm { kLists, kRank, kSort };
+SelectForm select_form(int n, int kk) {
+    if (n <= kThrMaxN && kk <= kThrMaxK) return SelectForm::kLists;
+    return n <= BFP8_SELECT_RANK_MAX ? SelectForm::kRank : SelectForm::kSort;
+}
+}  // namespace
+
+const char* bfp8_select_kernel_name(int n, int kk) {
+    if (kk <= BFP8_TOPK_MAX) return "bfp8_select_partials_kernel";
+    switch (select_form(n, kk)) {
+        case SelectForm::kLists: return "bfp8_select_lists_kernel";
+        case SelectForm::kRank: return "bfp8_select_block_sort_kernel";
+        default: return "bfp8_select_sort_kernel";
+    }
+}
+
 hipError_t bfp8_launch_select_sort(const float* logits, int n, int kk, uint64_t* keys, int* ids, float* scores,
                                    int* count, int* argmax, hipStream_t s) {
     if (n <= 0 || kk < 1 || kk > n || n > BFP8_SELECT_MAX) return hipErrorInvalidValue;
-    if (n <= kThrMaxN && kk <= kThrMaxK) {
+    const SelectForm form = select_form(n, kk);
+    if (form == SelectForm::kLists) {
         hipLaunchKernelGGL(bfp8_select_partials_kernel, dim3(select_grid(bfp8_ntiles(n), 4)), dim3(256), 0, s, logits, n, 64,
                            keys, (size_t)n);
         hipError_t e = hipGetLastError();
@@ -798,7 +816,7 @@ hipError_t bfp8_launch_select_sort(const float* logits, int n, int kk, uint64_t*
                            argmax);
         return hipGetLastError();
     }
-    if (n <= BFP8_SELECT_RANK_MAX) {
+    if (form == SelectForm::kRank) {
         const int nblk = (n + kSelBlock - 1) / kSelBlock;
         uint32_t* valid = reinterpret_cast<uint32_t*>(keys + n);
         hipLaunchKernelGGL(bfp8_select_block_sort_kernel, dim3(nblk), dim3(kBlkThreads), 0, s, logits, n, keys,

@@ -307,6 +307,19 @@ def test_bf16_device_lm_head_k_above_64(gpu, layout):
     assert int(cnt[1].item()) == ol.argmax(logits)
 
 
+@pytest.mark.parametrize("V,k,name", [(4096, 65, "lists"), (4096, 512, "lists"), (4096, 513, "block_sort"),
+                                      (65536, 512, "lists"), (65538, 512, "block_sort"), (65536, 65536, "block_sort")])
+def test_plan_names_its_selection(gpu, V, k, name):
+    """bfp8_plan_kernel_name on both sides of the lines between the selections
+    for k > 64."""
+    import torch
+
+    mat = gpu.DeviceMatrix.synth(V, 64, 5, 124, 130)
+    plan = gpu.SweepPlan([{"mat": mat, "x": torch.zeros(64, device="cuda"), "topk": k}])
+    assert plan.kernel_name(2) == f"bfp8_select_{name}_kernel"
+    plan.close()
+
+
 @pytest.mark.parametrize("n,k", [(65, 65), (513, 512), (1000, 300), (1025, 500), (2049, 65), (4096, 400),
                                  (8193, 512), (20000, 500), (33000, 512), (65535, 512), (65536, 70)])
 @pytest.mark.parametrize("kind", ["random", "equal", "rising", "falling", "three", "few"])
