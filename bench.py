@@ -424,14 +424,10 @@ def main():
 
 
 def batch_kernel(M, K):
-    """The kernel the library's batch launch picks for B = 16 (M rows, K
-    columns): many tiles, a workgroup per four 64-row tiles (K <= 1024) or
-    per tile; below that a workgroup per half tile and group of vectors with
-    each residue's blocks split over four wavefronts."""
-    nt, nb = (M + 63) // 64, K // 64
-    if nb <= 16:
-        return "bfp8_gemv_batch_cu_kernel" if nt >= 304 else "bfp8_gemv_batch_span_kernel"
-    return "bfp8_gemv_batch_mfma_kernel" if nt >= (192 if nb > 32 else 352) else "bfp8_gemv_batch_span_kernel"
+    """The kernel the library's batch launch takes for B = 16 (M rows, K columns)."""
+    import qwen_kernels_gpu as qk
+
+    return qk.load().bfp8_dev_gemv_batch_kernel_name(M, K, 16).decode()
 
 
 def bench_batch16(args, qk, torch, np):

@@ -327,6 +327,9 @@ int bfp8_dev_gemv_fallback(float* y, const float* x, const int8_t* mant_gpu, con
 int bfp8_dev_gemv_batch(float* Y, const uint32_t* xsplit, const float* xscale,
                         const int8_t* mant_gpu, const uint8_t* exps_gpu, int M, int K, int B,
                         void* stream);
+/* Name of the kernel that bfp8_dev_gemv_batch launches for these sizes ("" if
+ * it takes none). */
+const char* bfp8_dev_gemv_batch_kernel_name(int M, int K, int B);
 
 /* The BFP8 lm_head on quantized activations (hidden <= 4096): outputs on the
  * device (ids[min(k, vocab)], scores[min(k, vocab)], count, argmax), any

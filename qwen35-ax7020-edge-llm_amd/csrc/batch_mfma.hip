@@ -666,7 +666,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
     mf_body(L, Y, xsplit, xscale, mant, exps, M, K, B, (int)blockIdx.x, w & 1, w >> 1);
 }
 
+// The form that a call takes.  One vector is a plain GEMV: 2.8 us against the span
+// kernel's 3.4 at 3584 x 1024, 3.7 against 6.6 at 2048 x 3584, 11.7 against 12.2
+// (a workgroup per four tiles) at 65536 x 1024.
+// Many tiles fill the chip with the weight stream and take the forms that
+// read the weights once for all vectors; fewer take the span kernel.  The
+// lines lie where the two cross (us at a number of tiles, span first):
+// K = 1024, B = 2 6.8 / 9.0 at 469, 9.9 / 9.2 at 625; B = 8 7.9 / 8.7 at
+// 352, 9.8 / 9.1 at 469; B = 16 9.6 / 11.3 at 256, 12.6 / 11.2 at 352.
+// K = 2048, B = 8 25.2 / 25.8 at 782, 30.9 / 27.9 at 1024; B = 16 9.6 /
+// 16.2 at 128, 20.9 / 19.5 at 375.  K = 3584, B = 4 41.6 / 44.8 at 1024; B = 8
+// 26.6 / 29.7 at 375, 63.3 / 48.3 at 1024; B = 16 20.1 / 26.7 at 128, 33.5 /
+// 27.4 at 256.
+enum class BatchForm { kPlain, kCu, kTile, kSpan };
+BatchForm batch_form(int nt, int nb, int B) {
+    if (B == 1) return BatchForm::kPlain;
+    if (nb <= kCuMaxNb) return nt >= (B > 8 ? 304 : B > 4 ? 448 : 544) ? BatchForm::kCu : BatchForm::kSpan;
+    return B > 4 && nt >= (B > 8 ? (nb > 32 ? 192 : 352) : (nb > 32 ? 416 : 832)) ? BatchForm::kTile : BatchForm::kSpan;
+}
+
 }  // namespace
+
+const char* bfp8_batch_kernel_name(int M, int K, int B) {
+    switch (batch_form(bfp8_ntiles(M), K >> 6, B)) {
+        case BatchForm::kPlain: return bfp8_gemv_kernel_name(M, K);
+        case BatchForm::kCu: return "bfp8_gemv_batch_cu_kernel";
+        case BatchForm::kTile: return "bfp8_gemv_batch_mfma_kernel";
+        default: return "bfp8_gemv_batch_span_kernel";
+    }
+}
 
 hipError_t bfp8_launch_gemv_batch(float* Y, const uint32_t* xsplit, const float* xscale, const uint8_t* mant,
                                   const uint8_t* exps, int M, int K, int B, hipStream_t s) {
@@ -676,43 +704,31 @@ hipError_t bfp8_launch_gemv_batch(float* Y, const uint32_t* xsplit, const float*
     // (nb = K / 64 blocks; the split activation's stride is nb blocks)
     if (B < 1 || B > kMfVec || K < 64 || K > 64 * kSpanMaxNb) return hipErrorInvalidValue;
     const int nb = K >> 6;
-    if (B == 1) {
-        // one vector is a plain GEMV: 2.8 us against the span kernel's 3.4 at
-        // 3584 x 1024, 3.7 against 6.6 at 2048 x 3584, 11.7 against 12.2 (a
-        // workgroup per four tiles) at 65536 x 1024
-        Bfp8GemvDesc d{};
-        d.mant = mant;
-        d.exps = exps;
-        d.xsplit = xsplit;
-        d.xscale = xscale;
-        d.y = Y;
-        d.M = M;
-        d.K = K;
-        d.pair_rows = M & ~1;
-        return bfp8_launch_gemv(d, s);
-    }
-    // Many tiles fill the chip with the weight stream and take the forms that
-    // read the weights once for all vectors; fewer take the span kernel.  The
-    // lines lie where the two cross (us at a number of tiles, span first):
-    // K = 1024, B = 2 6.8 / 9.0 at 469, 9.9 / 9.2 at 625; B = 8 7.9 / 8.7 at
-    // 352, 9.8 / 9.1 at 469; B = 16 9.6 / 11.3 at 256, 12.6 / 11.2 at 352.
-    // K = 2048, B = 8 25.2 / 25.8 at 782, 30.9 / 27.9 at 1024; B = 16 9.6 /
-    // 16.2 at 128, 20.9 / 19.5 at 375.  K = 3584, B = 4 41.6 / 44.8 at 1024; B = 8
-    // 26.6 / 29.7 at 375, 63.3 / 48.3 at 1024; B = 16 20.1 / 26.7 at 128, 33.5 /
-    // 27.4 at 256.
-    if (nb <= kCuMaxNb) {
-        const dim3 grid((nt + kCuWaves / 2 - 1) / (kCuWaves / 2)), block(64 * kCuWaves);
-        if (B > 8 && nt >= 304) {
-            hipLaunchKernelGGL((bfp8_gemv_batch_cu_kernel<2, 8>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
+    switch (batch_form(nt, nb, B)) {
+        case BatchForm::kPlain: {
+            Bfp8GemvDesc d{};
+            d.mant = mant;
+            d.exps = exps;
+            d.xsplit = xsplit;
+            d.xscale = xscale;
+            d.y = Y;
+            d.M = M;
+            d.K = K;
+            d.pair_rows = M & ~1;
+            return bfp8_launch_gemv(d, s);
+        }
+        case BatchForm::kCu: {
+            const dim3 grid((nt + kCuWaves / 2 - 1) / (kCuWaves / 2)), block(64 * kCuWaves);
+            if (B > 8)
+                hipLaunchKernelGGL((bfp8_gemv_batch_cu_kernel<2, 8>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
+            else
+                hipLaunchKernelGGL((bfp8_gemv_batch_cu_kernel<2, 4>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
             return hipGetLastError();
         }
-        if (B <= 8 && nt >= (B > 4 ? 448 : 544)) {
-            hipLaunchKernelGGL((bfp8_gemv_batch_cu_kernel<2, 4>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
+        case BatchForm::kTile:
+            hipLaunchKernelGGL(bfp8_gemv_batch_mfma_kernel, dim3(nt), dim3(256), 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
             return hipGetLastError();
-        }
-    } else if (B > 4 && nt >= (B > 8 ? (nb > 32 ? 192 : 352) : (nb > 32 ? 416 : 832))) {
-        hipLaunchKernelGGL(bfp8_gemv_batch_mfma_kernel, dim3(nt), dim3(256), 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
-        return hipGetLastError();
+        case BatchForm::kSpan: break;
     }
     // The fewest vectors per workgroup that still leave at most one workgroup
     // per CU; beyond that every vector in as few workgroups as hold them, but

@@ -728,6 +728,11 @@ hipError_t bfp8_launch_gemv(const Bfp8GemvDesc& d, hipStream_t s) {
     return bfp8_launch_topk_merge(d, s);
 }
 
+const char* bfp8_gemv_kernel_name(int M, int K) {
+    if (bfp8_ntiles(M) > BFP8_WIDE_MAX_TILES) return "bfp8_gemv_kernel";
+    return K <= RT_ROWS_MAX_K ? "rt_rows_gemv_kernel" : "bfp8_gemv_wide_kernel";
+}
+
 const char* bfp8_topk_merge_kernel_name(int M) {
     return bfp8_ntiles(M) <= kMergeLists ? "bfp8_topk_merge_kernel" : "bfp8_topk_merge_wide_kernel";
 }

@@ -107,6 +107,8 @@ hipError_t bfp8_launch_gemv_wide_grouped(const Bfp8GemvDesc* descs_dev, const Bf
 hipError_t bfp8_launch_topk_merge(const Bfp8GemvDesc& d, hipStream_t s);
 // Name of the stand-alone merge kernel bfp8_launch_topk_merge runs for an M-row lm_head.
 const char* bfp8_topk_merge_kernel_name(int M);
+// The kernel of a plain GEMV without per-lane sums or top-k.
+const char* bfp8_gemv_kernel_name(int M, int K);
 // Persistent grouped launch: workgroup w walks tiles_dev[wg_off_dev[w] ..
 // wg_off_dev[w+1]); nwg <= bfp8_stream_grid().  merge_desc >= 0: workgroup 0
 // first merges the top-k partials of descs_dev[merge_desc] (written by an
@@ -210,6 +212,8 @@ hipError_t bfp8_launch_sweep(const Bfp8SweepArgs& a, int nwg, hipStream_t s);
 hipError_t bfp8_launch_gemv_batch(float* Y, const uint32_t* xsplit, const float* xscale,
                                   const uint8_t* mant, const uint8_t* exps, int M, int K, int B,
                                   hipStream_t s);
+// The kernel that it launches.
+const char* bfp8_batch_kernel_name(int M, int K, int B);
 int bfp8_cu_count();
 
 // ---- bf16_head.hip --------------------------------------------------------

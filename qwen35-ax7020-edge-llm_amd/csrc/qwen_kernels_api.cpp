@@ -940,6 +940,10 @@ int bfp8_dev_gemv_batch(float* Y, const uint32_t* xsplit, const float* xscale, c
     return BFP8_OK;
 }
 
+const char* bfp8_dev_gemv_batch_kernel_name(int M, int K, int B) {
+    return M > 0 && K >= 64 && K <= 4096 && B >= 1 && B <= 16 ? bfp8_batch_kernel_name(M, K, B) : "";
+}
+
 int bfp8_dev_lm_head_topk(int* out_ids, float* out_scores, int* out_count, int* out_argmax,
                           const uint32_t* xsplit, const float* xscale, const int8_t* mant_gpu,
                           const uint8_t* exps_gpu, int vocab, int hidden, int k, void* stream) {

@@ -171,6 +171,8 @@ def bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.bfp8_dev_gemv.argtypes = [vp, vp, vp, vp, vp, i, i, vp, vp]
     lib.bfp8_dev_gemv_float.argtypes = [vp, vp, vp, vp, i, i, vp]
     lib.bfp8_dev_gemv_batch.argtypes = [vp, vp, vp, vp, vp, i, i, i, vp]
+    lib.bfp8_dev_gemv_batch_kernel_name.argtypes = [i, i, i]
+    lib.bfp8_dev_gemv_batch_kernel_name.restype = ctypes.c_char_p
     lib.bfp8_dev_lm_head_topk.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i, i, i, vp]
     lib.bfp8_dev_lm_head_topk_noalloc.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i, i, i, vp]
     lib.bfp8_dev_synth_planes.argtypes = [vp, vp, i, i, c_uint64, i, i, vp]

@@ -113,6 +113,25 @@ def test_synthetic_activation_statistics():
     assert np.array_equal(qk.synth_normal(64, 5), qk.synth_normal(64, 5))
 
 
+@pytest.mark.parametrize("M,K,B,name", [(64, 64, 1, "rt_rows_gemv_kernel"), (24577, 1024, 1, "bfp8_gemv_kernel"),
+                                        (3584, 1024, 16, "bfp8_gemv_batch_span_kernel"),
+                                        (19392, 1024, 16, "bfp8_gemv_batch_span_kernel"),
+                                        (19393, 1024, 16, "bfp8_gemv_batch_cu_kernel"),
+                                        (28608, 1024, 8, "bfp8_gemv_batch_span_kernel"),
+                                        (28609, 1024, 8, "bfp8_gemv_batch_cu_kernel"),
+                                        (34752, 64, 4, "bfp8_gemv_batch_span_kernel"),
+                                        (34753, 64, 4, "bfp8_gemv_batch_cu_kernel"),
+                                        (12225, 3584, 16, "bfp8_gemv_batch_mfma_kernel"),
+                                        (12225, 2048, 16, "bfp8_gemv_batch_span_kernel"),
+                                        (200000, 3584, 4, "bfp8_gemv_batch_span_kernel"),
+                                        (64, 63, 4, ""), (64, 4097, 4, ""), (64, 64, 17, ""), (0, 64, 4, "")])
+def test_batch_kernel_names(M, K, B, name):
+    """The batched GEMV's forms on both sides of the lines between them."""
+    import qwen_kernels_gpu as qk
+
+    assert qk.load().bfp8_dev_gemv_batch_kernel_name(M, K, B).decode() == name
+
+
 def test_device_call_without_gpu_reports_error():
     """On a host without a GPU the int entry points return an error code with
     a message; nothing falls back to the CPU."""
