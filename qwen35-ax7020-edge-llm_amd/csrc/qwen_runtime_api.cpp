@@ -79,6 +79,7 @@ struct HostCall {
 // ---- the forward -----------------------------------------------------------------------
 constexpr int kHidden = RT_HIDDEN, kConv = RT_CONV_CH, kHD = RT_HEADS * RT_HEAD_DIM, kMlp = 3584;
 constexpr int kVocab = 65536, kLayers = 24;
+constexpr size_t kTapsLen = (size_t)3 * kConv, kStateLen = (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM;
 
 // Device copies of parameters the forward reads (float vectors, bf16 tables,
 // writable BFP8 planes), keyed by host address and size, kept until
@@ -94,7 +95,6 @@ struct DevState {
     // and rec[rcur] (the separate launches update rec in place; rec[1] is there
     // where the device has room for it: the layer can run in a chain)
     DevBuf buf;                              // conv[0], conv[1], rec[0]
-    DevBuf spare;                            // rec[1]
     float *conv[2], *rec[2] = {nullptr, nullptr};
     int cur = 0, rcur = 0;
     float* host_conv;     // the caller's buffers
@@ -131,10 +131,13 @@ struct FwdLayer {
 // with a wait of 0.25 s and a rest of 256, 6.1 and 506.
 constexpr uint64_t kChainWait = 200000;
 constexpr int kChainRest = 4, kChainRestMax = 65536;
+constexpr int kSeconds = 6;  // second state buffers in one allocation (one each costs a cold token 2 ms of 48)
 struct Chain {
     std::vector<RtChainLayer> host;  // the layer table
     DevBuf layers;                   // ... its device copy, the first `uploaded` entries
     size_t uploaded = 0;
+    std::vector<DevBuf> seconds;     // the states' rec[1], kSeconds each
+    int second_left = 0;             // free places of the last one
     DevBuf xch;                      // two sets of exchange words; each launch takes the other one and clears its predecessor's
     int set = 0;                     // the clean set
     int used[2] = {0, 0};            // words of each that are not clean
@@ -254,6 +257,19 @@ bool mlp_shapes_ok(const MlpPlan& p) {
            p.K_down == kMlp;
 }
 
+// A second state buffer, or null (no chain here, no room).
+float* second_state() {
+    Chain& c = F.chain;
+    if (!rt_chain_fits() || c.off) return nullptr;
+    if (c.second_left == 0) {
+        DevBuf b;
+        if (b.reserve(kSeconds * kStateLen * 4, true)) return nullptr;
+        c.seconds.push_back(b);
+        c.second_left = kSeconds;
+    }
+    return c.seconds.back().as<float>() + kStateLen * (kSeconds - c.second_left--);
+}
+
 // Device state of a layer, keyed by the caller's conv-state buffer.  A new
 // one starts from the caller's buffers.
 int fwd_state(float* conv_s, float* state, DevState** out) {
@@ -264,17 +280,16 @@ int fwd_state(float* conv_s, float* state, DevState** out) {
         return BFP8_OK;
     }
     std::unique_ptr<DevState> st(new DevState());
-    constexpr size_t nc = (size_t)3 * kConv, nr = (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM;
-    if (int rc = st->buf.reserve((2 * nc + nr) * 4)) return rc;
+    if (int rc = st->buf.reserve((2 * kTapsLen + kStateLen) * 4)) return rc;
     float* p = st->buf.as<float>();
     st->rec[0] = p;
-    st->conv[0] = p + nr;
-    st->conv[1] = p + nr + nc;
-    if (rt_chain_fits() && !F.chain.off && st->spare.reserve(nr * 4, true) == BFP8_OK) st->rec[1] = st->spare.as<float>();
+    st->conv[0] = p + kStateLen;
+    st->conv[1] = p + kStateLen + kTapsLen;
+    st->rec[1] = second_state();
     st->host_conv = conv_s;
     st->host_rec = state;
-    HIP_OK(hipMemcpy(st->conv[0], conv_s, (size_t)3 * kConv * 4, hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(st->rec[0], state, (size_t)RT_HEADS * RT_HEAD_DIM * RT_HEAD_DIM * 4, hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(st->conv[0], conv_s, kTapsLen * 4, hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(st->rec[0], state, kStateLen * 4, hipMemcpyHostToDevice));
     *out = st.get();
     F.states[key] = std::move(st);
     return BFP8_OK;
@@ -851,6 +866,9 @@ void drop_chain() {
     F.chain.uploaded = 0;
     F.chain.layers.release();
     F.chain.xch.release();
+    for (DevBuf& b : F.chain.seconds) b.release();
+    F.chain.seconds.clear();
+    F.chain.second_left = 0;
 }
 
 void drop_forward() {
@@ -864,7 +882,6 @@ void drop_forward() {
     F.planes.clear();
     for (auto& kv : F.states) {
         kv.second->buf.release();
-        kv.second->spare.release();
     }
     F.states.clear();
     drop_chain();
@@ -873,12 +890,12 @@ void drop_forward() {
 
 }  // namespace
 
-// The chain's memory and the states' second buffers: about 1 MB a layer, without
-// which the layers run as separate launches.
+// The chain's memory: the states' second buffers (1 MiB a layer) and the exchange
+// words (3.9 MB), without which the layers run as separate launches.
 bool release_spare(size_t bytes) {
     Chain& c = F.chain;
     size_t held = c.xch.n + c.layers.n;
-    for (auto& kv : F.states) held += kv.second->spare.n;
+    for (const DevBuf& b : c.seconds) held += b.n;
     if (!held || c.in_flight) return false;
     size_t room = 0, total = 0;
     if (g_dev_limit)
@@ -888,7 +905,7 @@ bool release_spare(size_t bytes) {
     if (room + held < bytes) return false;
     for (auto& kv : F.states) {  // a state in its second buffer moves to the first
         DevState* st = kv.second.get();
-        if (st->rcur && hipMemcpyAsync(st->rec[0], st->rec[1], st->spare.n, hipMemcpyDeviceToDevice, g.stream) != hipSuccess)
+        if (st->rcur && hipMemcpyAsync(st->rec[0], st->rec[1], kStateLen * 4, hipMemcpyDeviceToDevice, g.stream) != hipSuccess)
             return false;
     }
     if (hipStreamSynchronize(g.stream) != hipSuccess) return false;
@@ -896,7 +913,6 @@ bool release_spare(size_t bytes) {
         DevState* st = kv.second.get();
         st->rcur = 0;
         st->rec[1] = nullptr;
-        st->spare.release();
     }
     for (auto& kv : F.layers) kv.second->slot = -1;
     drop_chain();
