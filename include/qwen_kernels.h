@@ -88,7 +88,10 @@ int lm_head_argmax(const float* h, const uint16_t* embed_table, int vocab_size, 
  * forward's fused linear-attention kernel (conv1d, q/k norm, gates, recurrent
  * step, gated norm) is booked to gdn_recurrent_step; the norms, residual adds
  * and swiglu computed inside the GEMV launches to bfp8_gemv; the final norm
- * to rmsnorm. */
+ * to rmsnorm.  While profiling is on the forward runs each step as a launch of
+ * its own; otherwise runs of layers are one launch, so the slots add up to
+ * more than such a call takes (a token: about 700 microseconds of separate
+ * launches, 470 in one). */
 void qwen_prof_enable(int on);
 void qwen_prof_reset(void);
 int qwen_prof_count(void);
