@@ -29,12 +29,13 @@
 // and takes the two products otherwise; e < 8 (es = 0) and zero, infinite or
 // NaN scales give the same result either way.
 //
-// Work split: GEMVs with many tiles and K <= 1024, a workgroup per four tiles,
-// a wavefront per 32-row half with all 4 residues (bfp8_gemv_batch_cu_kernel);
-// with larger K, a workgroup per tile, a wavefront per half and two residues
-// (bfp8_gemv_batch_mfma_kernel); otherwise a workgroup of 16 wavefronts per half
-// and group of vectors, a wavefront per residue and quarter of the blocks
-// (bfp8_gemv_batch_span_kernel).
+// Work split, by what batch_form at the end picks for the sizes: a workgroup of 16
+// wavefronts per 32-row half and group of vectors, a wavefront per residue and
+// quarter of the blocks (bfp8_gemv_batch_span_kernel); a workgroup per tile, a
+// wavefront per half and two residues, or per half, a wavefront per residue
+// (bfp8_gemv_batch_mfma_kernel); a workgroup per four tiles, a wavefront per half
+// with all 4 residues (bfp8_gemv_batch_cu_kernel); for two vectors also without
+// the matrix cores (bfp8_gemv_batch_dot_kernel).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -61,8 +62,8 @@ struct MfLds {
     uint64_t xa[CH][4][64];
     float xs[CH][kMfVec];      // [block][vector] block scales
     int lo[CH], hi[CH];        // per block: e range of the one-product epilogue
-    // the end's exchange: 2 halves x 2 residues x 8 values x 64 lanes
-    static_assert(CH * 4 * 64 * sizeof(uint64_t) >= 2 * 2 * 8 * 64 * sizeof(float),
+    // the end's exchange: 3 residue groups x 2 halves x 8 values x 64 lanes at most
+    static_assert(CH * 4 * 64 * sizeof(uint64_t) >= 3 * 2 * 8 * 64 * sizeof(float),
                   "the fs exchange fits in the staging area");
 };
 
@@ -142,34 +143,41 @@ __device__ __forceinline__ void mf_stage_store(MfLds<CH>& L, const MfStaged<NT, 
     if (kSync) __syncthreads();
 }
 
-constexpr int kMfRes = 2;    // residues per wavefront of the workgroup-per-tile kernel
-constexpr int kMfDepth = 2;  // its weight-load groups in flight per wavefront
-constexpr int kMfChunk = 8;  // its blocks per staging
-
 // A lane's result slots: register i of the MFMA result (and i + 8, the low
-// parts) is vector 8(i/4) + 4*kh + i%4 of the lane's row, i = 0..7.
-struct MfState {
-    float fs[kMfRes][8];  // [residue of the group][slot]
+// parts) is vector 8(i/4) + 4*kh + i%4 of the lane's row; every vector: slots
+// i = 0..7; vector half kVH: slots i = 4 kVH .. 4 kVH + 3.
+template <int kVH>
+struct MfSlots {
+    static constexpr int n = kVH < 0 ? 8 : 4;
+    static constexpr int i0 = kVH < 0 ? 0 : 4 * kVH;
 };
 
+template <int kRes, int kVH>
+struct MfState {
+    float fs[kRes][MfSlots<kVH>::n];  // [residue of the group][slot]
+};
+
+template <int kRes>
 struct MfLoads {
-    uint64_t w[kMfGroup][kMfRes];  // [block][residue of the group]
+    uint64_t w[kMfGroup][kRes];  // [block][residue of the group]
     uint32_t e;
 };
 
 // One block: an MFMA per residue of the group and the epilogue.
-__device__ __forceinline__ void mf_block(MfState& st, const MfLds<kMfChunk>& L, const uint64_t (&w)[kMfRes], uint32_t e,
+template <int kRes, int kVH, int CH>
+__device__ __forceinline__ void mf_block(MfState<kRes, kVH>& st, const MfLds<CH>& L, const uint64_t (&w)[kRes], uint32_t e,
                                          int u, int q0, int lane) {
-    i32x16 d[kMfRes];
+    constexpr int NS = MfSlots<kVH>::n, I0 = MfSlots<kVH>::i0;
+    i32x16 d[kRes];
     const i32x16 zero = {};
 #pragma unroll
-    for (int r = 0; r < kMfRes; ++r)
+    for (int r = 0; r < kRes; ++r)
         d[r] = __builtin_amdgcn_mfma_i32_32x32x16_i8((long)L.xa[u][q0 + r][lane], (long)w[r], zero, 0, 0, 0);
     const int kh = lane >> 5;
-    float xs[8];
+    float xs[NS];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {  // slots 4h..4h+3: vectors 8h + 4 kh ..
-        const f32x4 x4 = *reinterpret_cast<const f32x4*>(&L.xs[u][8 * h + 4 * kh]);
+    for (int h = 0; h < NS / 4; ++h) {  // slots 4h..4h+3: vectors 8 (I0 / 4 + h) + 4 kh ..
+        const f32x4 x4 = *reinterpret_cast<const f32x4*>(&L.xs[u][8 * (I0 / 4 + h) + 4 * kh]);
 #pragma unroll
         for (int m = 0; m < 4; ++m) xs[4 * h + m] = x4[m];
     }
@@ -177,22 +185,22 @@ __device__ __forceinline__ void mf_block(MfState& st, const MfLds<kMfChunk>& L, 
     const int lo = L.lo[u], hi = L.hi[u];
     const bool one_product = (e < 8u) | ((uint32_t)((int)e - lo) <= (uint32_t)(hi - lo));
     if (__builtin_amdgcn_ballot_w64(!one_product) == 0) {
-        float c[8];
+        float c[NS];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) c[k] = es * xs[k];
+        for (int k = 0; k < NS; ++k) c[k] = es * xs[k];
 #pragma unroll
-        for (int r = 0; r < kMfRes; ++r)
+        for (int r = 0; r < kRes; ++r)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int S = (int)((uint32_t)d[r][k] << 8) + d[r][k + 8];
+            for (int k = 0; k < NS; ++k) {
+                const int S = (int)((uint32_t)d[r][I0 + k] << 8) + d[r][I0 + k + 8];
                 st.fs[r][k] = st.fs[r][k] + (float)S * c[k];
             }
     } else {
 #pragma unroll
-        for (int r = 0; r < kMfRes; ++r)
+        for (int r = 0; r < kRes; ++r)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int S = (int)((uint32_t)d[r][k] << 8) + d[r][k + 8];
+            for (int k = 0; k < NS; ++k) {
+                const int S = (int)((uint32_t)d[r][I0 + k] << 8) + d[r][I0 + k + 8];
                 const float t1 = (float)S * es;
                 st.fs[r][k] = st.fs[r][k] + t1 * xs[k];
             }
@@ -204,12 +212,13 @@ __device__ __forceinline__ void mf_block(MfState& st, const MfLds<kMfChunk>& L, 
 // per dword).  The whole offset goes in the per-lane offset, which the buffer
 // range check covers: groups past the tile read zeros without touching memory.
 static_assert(4 % kMfGroup == 0, "a group's exponents share one dword");
-__device__ __forceinline__ void mf_issue(MfLoads& ld, __amdgpu_buffer_rsrc_t wrs, __amdgpu_buffer_rsrc_t ers, int wv,
+template <int kRes>
+__device__ __forceinline__ void mf_issue(MfLoads<kRes>& ld, __amdgpu_buffer_rsrc_t wrs, __amdgpu_buffer_rsrc_t ers, int wv,
                                          int ev, int gi) {
 #pragma unroll
     for (int uu = 0; uu < kMfGroup; ++uu)
 #pragma unroll
-        for (int r = 0; r < kMfRes; ++r) {
+        for (int r = 0; r < kRes; ++r) {
             const u32x2 v = __builtin_bit_cast(
                 u32x2, __builtin_amdgcn_raw_buffer_load_b64(wrs, wv + (gi * kMfGroup + uu) * 4096 + r * 1024, 0,
                                                             kNonTemporal));
@@ -218,82 +227,94 @@ __device__ __forceinline__ void mf_issue(MfLoads& ld, __amdgpu_buffer_rsrc_t wrs
     ld.e = load_e(ers, ev + (gi * kMfGroup / 4) * 256, 0);
 }
 
-constexpr int kMfThreads = 256;
-
-__device__ __forceinline__ void mf_group(MfState& st, MfLds<kMfChunk>& L, const MfLoads& ld, int gi, int nb,
+template <int kRes, int NT, int kVH, int CH>
+__device__ __forceinline__ void mf_group(MfState<kRes, kVH>& st, MfLds<CH>& L, const MfLoads<kRes>& ld, int gi, int nb,
                                          const uint32_t* __restrict__ xsplit, const float* __restrict__ xscale, int B,
                                          int q0, int lane) {
     const int b0 = gi * kMfGroup;
-    if (b0 % kMfChunk == 0 && b0 > 0) {  // the first chunk is staged before the loop
+    if (b0 % CH == 0 && b0 > 0) {  // the first chunk is staged before the loop
         __syncthreads();  // every wavefront is done with the previous chunk
-        MfStaged<kMfThreads, kMfChunk> S;
-        mf_stage_load<kMfThreads, -1, kMfChunk>(S, xsplit, xscale, nb, B, b0, min(kMfChunk, nb - b0));
-        mf_stage_store<kMfThreads, kMfChunk>(L, S);
+        MfStaged<NT, CH> S;
+        mf_stage_load<NT, kVH, CH>(S, xsplit, xscale, nb, B, b0, min(CH, nb - b0));
+        mf_stage_store<NT, CH>(L, S);
     }
 #pragma unroll
     for (int uu = 0; uu < kMfGroup; ++uu) {
         if (b0 + uu >= nb) break;
-        mf_block(st, L, ld.w[uu], (ld.e >> (8 * ((b0 + uu) & 3))) & 0xffu, (b0 + uu) % kMfChunk, q0, lane);
+        mf_block<kRes, kVH, CH>(st, L, ld.w[uu], (ld.e >> (8 * ((b0 + uu) & 3))) & 0xffu, (b0 + uu) % CH, q0, lane);
     }
 }
 
-// The work of one wavefront: tile t, its 32-row half s, the residues of group
-// grp (two of them), all vectors.
-__device__ __forceinline__ void mf_body(MfLds<kMfChunk>& L, float* __restrict__ Y, const uint32_t* __restrict__ xsplit,
+// The work of one workgroup: tile t, its 32-row half s (kHalves == 1) or both
+// (kHalves == 2, wavefront w takes half w & 1), the residues of group grp,
+// the vectors of kVH (every vector, or one half of them).
+// kDepth: weight-load groups in flight per wavefront (2: one group computed
+// while the next loads; CH / kMfGroup: a chunk's every weight load issued at
+// once, for GEMVs with too few tiles to fill the memory system otherwise).
+template <int kRes, int kHalves, int kDepth, int kVH, int CH>
+__device__ __forceinline__ void mf_body(MfLds<CH>& L, float* __restrict__ Y, const uint32_t* __restrict__ xsplit,
                                         const float* __restrict__ xscale, const uint8_t* __restrict__ mant,
                                         const uint8_t* __restrict__ exps, int M, int K, int B, int t, int s, int grp) {
+    constexpr int NS = MfSlots<kVH>::n, I0 = MfSlots<kVH>::i0;
     const int lane = threadIdx.x & 63;
-    const int q0 = grp * kMfRes;
+    const int q0 = grp * kRes;
     const int col = lane & 31, kh = lane >> 5;
     const int nb = K >> 6, nb4 = (nb + 3) >> 2;
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(mant + (size_t)t * nb * 4096u, (uint32_t)nb * 4096u);
     const __amdgpu_buffer_rsrc_t ers = make_rsrc(exps + (size_t)t * nb4 * 256u, (uint32_t)nb4 * 256u);
     const int wv = q0 * 1024 + (32 * s + col) * 16 + kh * 8;
     const int ev = (32 * s + col) * 4;
-    MfState st;
+    MfState<kRes, kVH> st;
 #pragma unroll
-    for (int r = 0; r < kMfRes; ++r)
+    for (int r = 0; r < kRes; ++r)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) st.fs[r][k] = 0.0f;
+        for (int k = 0; k < NS; ++k) st.fs[r][k] = 0.0f;
     const int ng = (nb + kMfGroup - 1) / kMfGroup;
     // the first chunk's activation loads go out first, then the first
     // weight groups: the staging then waits for its own loads only (a
     // wavefront's loads complete in the order issued)
-    MfStaged<kMfThreads, kMfChunk> S0;
-    mf_stage_load<kMfThreads, -1, kMfChunk>(S0, xsplit, xscale, nb, B, 0, min(kMfChunk, nb));
-    MfLoads ld[kMfDepth];
+    constexpr int NT = 64 * kHalves * (4 / kRes);
+    MfStaged<NT, CH> S0;
+    mf_stage_load<NT, kVH, CH>(S0, xsplit, xscale, nb, B, 0, min(CH, nb));
+    MfLoads<kRes> ld[kDepth];
 #pragma unroll
-    for (int d = 0; d < kMfDepth; ++d) mf_issue(ld[d], wrs, ers, wv, ev, d);
-    mf_stage_store<kMfThreads, kMfChunk>(L, S0);
-    for (int gi = 0; gi < ng; gi += kMfDepth) {
-        // kMfDepth load sets in turn: set d holds group gi + d, then gi + d + kMfDepth
+    for (int d = 0; d < kDepth; ++d) mf_issue<kRes>(ld[d], wrs, ers, wv, ev, d);
+    mf_stage_store<NT, CH>(L, S0);
+    for (int gi = 0; gi < ng; gi += kDepth) {
+        // kDepth load sets in turn: set d holds group gi + d, then gi + d + kDepth
 #pragma unroll
-        for (int d = 0; d < kMfDepth; ++d) {
-            if (gi + d < ng) mf_group(st, L, ld[d], gi + d, nb, xsplit, xscale, B, q0, lane);
-            mf_issue(ld[d], wrs, ers, wv, ev, gi + d + kMfDepth);
+        for (int d = 0; d < kDepth; ++d) {
+            if (gi + d < ng) mf_group<kRes, NT, kVH, CH>(st, L, ld[d], gi + d, nb, xsplit, xscale, B, q0, lane);
+            mf_issue<kRes>(ld[d], wrs, ers, wv, ev, gi + d + kDepth);
         }
     }
-    float (&fs)[kMfRes][8] = st.fs;
+    float (&fs)[kRes][NS] = st.fs;
 
-    // y = (fs_0 + fs_2) + (fs_1 + fs_3): the second residue group of the half
-    // hands its sums to the first through the (no longer needed) staging area
+    // y = (fs_0 + fs_2) + (fs_1 + fs_3): the other residue groups of the half
+    // hand their sums to group 0 through the (no longer needed) staging area
     __syncthreads();
-    float* xch = reinterpret_cast<float*>(&L.xa[0][0][0]);  // [half][residue][slot][lane]
+    float* xch = reinterpret_cast<float*>(&L.xa[0][0][0]);  // [group - 1][half][residue][slot][lane]
     if (grp > 0) {
 #pragma unroll
-        for (int r = 0; r < kMfRes; ++r)
+        for (int r = 0; r < kRes; ++r)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) xch[((s * kMfRes + r) * 8 + k) * 64 + lane] = fs[r][k];
+            for (int k = 0; k < NS; ++k) xch[((((grp - 1) * 2 + s) * kRes + r) * NS + k) * 64 + lane] = fs[r][k];
     }
     __syncthreads();
     if (grp == 0) {
         const int row = t * 64 + 32 * s + col;
         const int pair_rows = M & ~1;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const float f2 = xch[((s * kMfRes + 0) * 8 + k) * 64 + lane], f3 = xch[((s * kMfRes + 1) * 8 + k) * 64 + lane];
-            const int v = 8 * (k / 4) + 4 * kh + (k % 4);
-            const float y = (fs[0][k] + f2) + (fs[1][k] + f3);
+        for (int k = 0; k < NS; ++k) {
+            float f[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int gq = q / kRes, rq = q % kRes;
+                f[q] = gq == 0 ? fs[rq][k] : xch[((((gq - 1) * 2 + s) * kRes + rq) * NS + k) * 64 + lane];
+            }
+            const int i = I0 + k;
+            const int v = 8 * (i / 4) + 4 * kh + (i % 4);
+            const float y = (f[0] + f[2]) + (f[1] + f[3]);
             if (v < B && row < pair_rows) Y[(size_t)v * M + row] = y;
         }
     }
@@ -657,32 +678,218 @@ hipError_t launch_span(float* Y, const uint32_t* xsplit, const float* xscale, co
     return hipGetLastError();
 }
 
-// ---- many tiles, K > 1024: a workgroup per tile ---------------------------------
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void bfp8_gemv_batch_mfma_kernel(
-    float* __restrict__ Y, const uint32_t* __restrict__ xsplit, const float* __restrict__ xscale,
-    const uint8_t* __restrict__ mant, const uint8_t* __restrict__ exps, int M, int K, int B) {
-    __shared__ MfLds<kMfChunk> L;
+// ---- a workgroup per tile, or per 32-row half of one --------------------------------
+// kHalves: halves of a tile per workgroup (2: both, workgroup per tile; 1:
+// workgroup per 32-row half, twice the workgroups for GEMVs with few tiles).
+// kSplit: 1, every vector in each workgroup; 2, a workgroup per half of the
+// vectors, each wavefront then finishing 4 of the 8 result slots of its
+// lanes -- half the epilogue per wavefront, on twice the wavefronts, for
+// GEMVs whose wavefronts are too few to hide the epilogue's latencies.  The
+// two workgroups of a unit are blocks 16a + x and 16a + 8 + x (x < 8), which
+// go to the same XCD (blocks are dealt to the 8 XCDs in turn), so the second
+// reads the unit's weights from that XCD's L2; unit 8a + x, blocks past the
+// last unit exit at once.
+template <int kRes, int kHalves, int kDepth, int kSplit, int CH>
+__global__ __launch_bounds__(64 * kHalves * (4 / kRes)) __attribute__((amdgpu_waves_per_eu(kSplit == 2 ? 2 : 4))) void
+bfp8_gemv_batch_mfma_kernel(float* __restrict__ Y, const uint32_t* __restrict__ xsplit,
+                            const float* __restrict__ xscale, const uint8_t* __restrict__ mant,
+                            const uint8_t* __restrict__ exps, int M, int K, int B) {
+    __shared__ MfLds<CH> L;
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    mf_body(L, Y, xsplit, xscale, mant, exps, M, K, B, (int)blockIdx.x, w & 1, w >> 1);
+    const int b = (int)blockIdx.x;
+    const int bid = kSplit == 2 ? 8 * (b >> 4) + (b & 7) : b;
+    const int nunits = kHalves == 2 ? bfp8_ntiles(M) : 2 * bfp8_ntiles(M);
+    if (kSplit == 2 && bid >= nunits) return;  // the grid's last 16 blocks may hold fewer units
+    // 32-row half, residue group, tile
+    const int s = kHalves == 2 ? (w & 1) : (bid & 1), grp = kHalves == 2 ? (w >> 1) : w;
+    const int t = kHalves == 2 ? bid : (bid >> 1);
+    if (kSplit == 1)
+        mf_body<kRes, kHalves, kDepth, -1, CH>(L, Y, xsplit, xscale, mant, exps, M, K, B, t, s, grp);
+    else if (((b >> 3) & 1) == 0)
+        mf_body<kRes, kHalves, kDepth, 0, CH>(L, Y, xsplit, xscale, mant, exps, M, K, B, t, s, grp);
+    else
+        mf_body<kRes, kHalves, kDepth, 1, CH>(L, Y, xsplit, xscale, mant, exps, M, K, B, t, s, grp);
+}
+
+// ---- two vectors (four with K <= 128), many tiles: dot products ------------------
+// A workgroup per tile, wavefront = residue, lane = row: the residue sums by
+// v_dot4_i32_i8.  Activations of a chunk of 8 blocks for all B vectors are
+// staged in LDS (wave-uniform broadcast reads); each lane keeps B residue
+// accumulators.  Its VALU work grows with B, and the matrix-core forms work for
+// 8 or 16 vectors whatever B is, so it stands where two vectors (or few blocks)
+// leave it the least to do: us by span / four tiles or one a workgroup / this,
+// weights from HBM: 20480 x 256, B = 2 5.8 / 4.7 / 4.2; 32768 x 512, B = 2 7.7 /
+// 6.3 / 6.3; 65536 x 1088, B = 2 21.5 / 17.2 / 16.3; 81920 x 128, B = 4 24 / 6.6 /
+// 5.4.
+constexpr int kBatchChunk = 8;  // blocks per LDS-staged step
+template <int B>
+__global__ __launch_bounds__(256) void bfp8_gemv_batch_dot_kernel(
+    float* __restrict__ Y, const uint32_t* __restrict__ xsplit, const float* __restrict__ xscale,
+    const uint8_t* __restrict__ mant, const uint8_t* __restrict__ exps, int M, int K) {
+    __shared__ uint32_t xl[B * kBatchChunk * 32];
+    __shared__ float xsl[B * kBatchChunk];  // the chunk's block scales (LDS, like the split words: no scalar loads,
+                                            // whose out-of-order returns would make every LDS wait a full wait)
+    float* red = reinterpret_cast<float*>(xl);  // the cross-wave sums reuse the staging space (4 * 64 * B floats)
+    static_assert(kBatchChunk * 32 >= 4 * 64, "red fits in xl");
+    const int q = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int r = threadIdx.x & 63;
+    const int t = blockIdx.x;
+    const int nb = K >> 6;
+    const int nb4 = (nb + 3) >> 2;
+    const uint8_t* mtile = mant + (size_t)t * nb * 4096u;
+    const uint8_t* etile = exps + (size_t)t * nb4 * 256u;
+    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(mtile, (uint32_t)nb * 4096u);
+    const __amdgpu_buffer_rsrc_t ers = make_rsrc(etile, (uint32_t)nb4 * 256u);
+    const int wv = q * 1024 + r * 16;
+    const int xwords = nb * 32;
+    float fs[B];
+#pragma unroll
+    for (int v = 0; v < B; ++v) fs[v] = 0.0f;
+
+    for (int b0 = 0; b0 < nb; b0 += kBatchChunk) {
+        const int nbc = min(kBatchChunk, nb - b0);
+        u32x4 w[kBatchChunk];
+        uint32_t ew[kBatchChunk / 4] = {};
+#pragma unroll
+        for (int u = 0; u < kBatchChunk; ++u)
+            if (u < nbc) w[u] = load_w(wrs, wv, (b0 + u) * 4096);
+#pragma unroll
+        for (int m = 0; m < kBatchChunk / 4; ++m)
+            if (4 * m < nbc) ew[m] = load_e(ers, r * 4, ((b0 >> 2) + m) * 256);
+        __syncthreads();  // previous chunk's LDS reads are done
+        for (int i = threadIdx.x; i < B * nbc * 32; i += 256) {
+            int v = i / (nbc * 32), o = i - v * nbc * 32;
+            xl[v * kBatchChunk * 32 + o] = xsplit[(size_t)v * xwords + b0 * 32 + o];
+        }
+        for (int i = threadIdx.x; i < B * nbc; i += 256) {
+            const int v = i / nbc, u = i - v * nbc;
+            xsl[v * kBatchChunk + u] = xscale[(size_t)v * nb + b0 + u];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < kBatchChunk; ++u) {
+            if (u >= nbc) break;
+            const uint32_t e = (ew[u >> 2] >> (8 * (u & 3))) & 0xffu;
+            const float sc = exp_scale_ftz(e);
+            // vectors in groups of four: the group's LDS reads go out together,
+            // then its four dot-product chains interleave
+            constexpr int kG = B < 4 ? B : 4;
+#pragma unroll
+            for (int v0 = 0; v0 < B; v0 += kG) {
+                uint4 h[kG], l[kG];
+                float xs[kG];
+#pragma unroll
+                for (int j = 0; j < kG; ++j) {
+                    const uint32_t* xb = xl + ((v0 + j) * kBatchChunk + u) * 32 + q * 8;
+                    h[j] = *reinterpret_cast<const uint4*>(xb);
+                    l[j] = *reinterpret_cast<const uint4*>(xb + 4);
+                    xs[j] = xsl[(v0 + j) * kBatchChunk + u];
+                }
+                int acc[kG];
+#pragma unroll
+                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].x, (int)h[j].x, 0, false);
+#pragma unroll
+                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].y, (int)h[j].y, acc[j], false);
+#pragma unroll
+                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].z, (int)h[j].z, acc[j], false);
+#pragma unroll
+                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].w, (int)h[j].w, acc[j], false);
+#pragma unroll
+                for (int j = 0; j < kG; ++j) {
+                    acc[j] = (int)((uint32_t)acc[j] << 8);
+                    acc[j] = __builtin_amdgcn_sdot4((int)w[u].x, (int)l[j].x, acc[j], false);
+                }
+#pragma unroll
+                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].y, (int)l[j].y, acc[j], false);
+#pragma unroll
+                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].z, (int)l[j].z, acc[j], false);
+#pragma unroll
+                for (int j = 0; j < kG; ++j) acc[j] = __builtin_amdgcn_sdot4((int)w[u].w, (int)l[j].w, acc[j], false);
+#pragma unroll
+                for (int j = 0; j < kG; ++j) {
+                    const float t1 = (float)acc[j] * sc;
+                    const float t2 = t1 * xs[j];
+                    fs[v0 + j] = fs[v0 + j] + t2;
+                }
+            }
+        }
+    }
+    __syncthreads();  // every wavefront is done with the staged activations
+#pragma unroll
+    for (int v = 0; v < B; ++v) red[(v * 4 + q) * 64 + r] = fs[v];
+    __syncthreads();
+    const int pair_rows = M & ~1;
+    for (int i = threadIdx.x; i < B * 64; i += 256) {
+        int v = i >> 6, rr = i & 63;
+        int row = t * 64 + rr;
+        const float* p = red + v * 256;
+        float y = (p[rr] + p[128 + rr]) + (p[64 + rr] + p[192 + rr]);
+        if (row < pair_rows) Y[(size_t)v * M + row] = y;
+    }
 }
 
 // The form that a call takes.  One vector is a plain GEMV: 2.8 us against the span
 // kernel's 3.4 at 3584 x 1024, 3.7 against 6.6 at 2048 x 3584, 11.7 against 12.2
 // (a workgroup per four tiles) at 65536 x 1024.
-// Many tiles fill the chip with the weight stream and take the forms that
-// read the weights once for all vectors; fewer take the span kernel.  The
-// lines lie where the two cross (us at a number of tiles, span first):
-// K = 1024, B = 2 6.8 / 9.0 at 469, 9.9 / 9.2 at 625; B = 8 7.9 / 8.7 at
-// 352, 9.8 / 9.1 at 469; B = 16 9.6 / 11.3 at 256, 12.6 / 11.2 at 352.
-// K = 2048, B = 8 25.2 / 25.8 at 782, 30.9 / 27.9 at 1024; B = 16 9.6 /
-// 16.2 at 128, 20.9 / 19.5 at 375.  K = 3584, B = 4 41.6 / 44.8 at 1024; B = 8
-// 26.6 / 29.7 at 375, 63.3 / 48.3 at 1024; B = 16 20.1 / 26.7 at 128, 33.5 /
-// 27.4 at 256.
-enum class BatchForm { kPlain, kCu, kTile, kSpan };
+//
+// The span kernel's time goes up in steps of the workgroups that run at once (512,
+// 256 with four slots) and with K rounded up to a multiple of 1024; the forms
+// that read the weights once for all vectors cost more to start and then grow
+// with the bytes.  The lines lie where the two cross, by the geometric mean of
+// weights from HBM and weights from the cache (the span kernel is up to a
+// quarter faster there: its weight loads are not non-temporal).  Each with both
+// sides, us from HBM (from cache), lower side of the line first:
+//   B <= 4, K <= 256: 128 tiles, B = 4 span 3.9, tile 4.1; 144 span 4.3 (4.4), tile 4.0 (4.1)
+//   B = 2, K = 512: 256 span 4.7, dot 4.8; 320 span 6.0 (5.0), dot 5.6 (4.2); 1024 dot 9.2, four tiles 8.6
+//   B = 4, K = 512: 256 span 4.9 (4.4), tile 5.1 (4.8); 400 span 7.8, tile 6.3; 640 tile 7.8, four tiles 7.4
+//   B = 4, K = 1024: 512 span 9.6 (7.1), four tiles 9.2 (8.8); 576 10.9 (9.6), 9.5 (9.0)
+//   B = 4, K = 768: 448 span 8.5 (6.8), four tiles 7.8 (7.5); 512 8.9 (7.0), 8.0 (7.6)
+//   B = 2, K = 1088: 384 span 10.1 (7.4), dot 10.0 (9.3); 512 12.3 (9.5), 11.3 (10.1); 1024 21.5, 16.3
+//   B = 4, K = 2048: 1024 span 27.9 (24.1), tile 27.4 (26.2); K = 2112: 832 tile 8 % faster, 1024 17 %
+//   B = 8, K = 512: 128 span 4.2, tile 4.9; 144 6.9 (6.4), 5.0 (5.0); 512 tile 6.5, four tiles 7.2; 640 7.9, 7.5
+//   B = 8, K = 768: 144 span 7.7, tile 7.0; 272 tile 8.4, four tiles 7.5
+//   B = 8, K = 1024: 256 span 8.9 (7.2), four tiles 8.6 (8.3); 272 11.5 (9.8), 8.7 (8.4)
+//   B = 8, K = 1088: 256 span 9.3, tile 9.6; 384 12.9 (10.5), 11.5 (11.1); 512 15.9, 11.9
+//   B = 8, K = 3584: 320 span 26.8 (21.9), half 27.0 (26.3); 352 half 27.2, tile 30; 384 span 30.8, half 27.3;
+//     448 half 33.2, tile 30.3
+//   B = 16, K = 512: 64 span 4.0, tile 5.2; 128 6.9, 5.3; 1024 tile 10.1, four tiles 9.1
+//   B = 16, K = 1024: 64 span 4.5; 128 span 8.1 (7.1), half 7.3 (6.7), tile 8.8; 192 tile 8.9, four tiles 11.0;
+//     512 10.8, 11.2; 640 13.2, 11.4; 1088 tile 5 % faster, 1536 four tiles 10 %
+//   B = 16, K = 1088: 128 span 8.7, tile 9.8; 160 11.5, 9.9; K = 2048: 256 span 16.5 (14.5), tile 16.4 (16.1);
+//     384 22.9, 19.3
+//   B = 16, K = 3584: 128 span 20.3 (18.0), half 19.0 (18.8); 192 span 28.1, half 23.0, tile 27.0; 224 half 33.9, tile 27.2
+// (four tiles: bfp8_gemv_batch_cu_kernel; tile, half: bfp8_gemv_batch_mfma_kernel,
+// whose half form runs 768 workgroups at once: 384 tiles, 192 above 8 vectors)
+enum class BatchForm { kPlain, kDot, kSpan, kCu, kTile, kHalf };
 BatchForm batch_form(int nt, int nb, int B) {
     if (B == 1) return BatchForm::kPlain;
-    if (nb <= kCuMaxNb) return nt >= (B > 8 ? 304 : B > 4 ? 448 : 544) ? BatchForm::kCu : BatchForm::kSpan;
-    return B > 4 && nt >= (B > 8 ? (nb > 32 ? 192 : 352) : (nb > 32 ? 416 : 832)) ? BatchForm::kTile : BatchForm::kSpan;
+    const int up = (nb + 15) & ~15, pad = up - nb;  // the span kernel's blocks, those past K
+    if (nb <= kCuMaxNb) {
+        const bool one_round = nt <= 1024;  // of the four-tile kernel
+        if (nb <= 8) {
+            if (nt <= (B > 8 ? 64 : B > 4 || (B > 2 && nb <= 4) ? 128 : 256)) return BatchForm::kSpan;
+            if (nb > 4 && one_round && nt > (B == 2 || B > 8 ? 768 : 512)) return BatchForm::kCu;
+            return B == 2 || (B == 4 && nb <= 2) ? BatchForm::kDot : BatchForm::kTile;
+        }
+        if (B <= 4) {
+            if (nt < (nb <= 12 && B > 2 ? 480 : 544)) return BatchForm::kSpan;
+            return B == 2 && !one_round && (nt < 1600 || nb <= 10) ? BatchForm::kDot : BatchForm::kCu;
+        }
+        if (B <= 8) return nt > 256 ? BatchForm::kCu : nt <= 128 || nb > 12 ? BatchForm::kSpan : BatchForm::kTile;
+        if (nt <= 128) return nt <= 64 ? BatchForm::kSpan : BatchForm::kHalf;
+        return nt <= 512 || (!one_round && nt <= 1280) ? BatchForm::kTile : BatchForm::kCu;
+    }
+    if (B <= 4) {
+        if (nt * pad < 240 * up - 1100) return BatchForm::kSpan;
+        return B == 2 ? BatchForm::kDot : BatchForm::kTile;
+    }
+    if (nb <= 32) {
+        const int line = B <= 8 ? (pad >= 12 ? 340 : pad >= 6 ? 430 : pad >= 2 ? 520 : 900) : (pad >= 12 ? 128 : pad >= 6 ? 208 : 310);
+        return nt <= line ? BatchForm::kSpan : BatchForm::kTile;
+    }
+    if (B <= 8) return nt <= 320 ? BatchForm::kSpan : nt <= 384 ? BatchForm::kHalf : BatchForm::kTile;
+    if (B <= 12) return nt <= (nb <= 37 ? 176 : 208) ? BatchForm::kSpan : BatchForm::kTile;
+    return nt <= (pad >= 8 ? 112 : 128) ? BatchForm::kSpan : nt <= 192 ? BatchForm::kHalf : BatchForm::kTile;
 }
 
 }  // namespace
@@ -690,8 +897,10 @@ BatchForm batch_form(int nt, int nb, int B) {
 const char* bfp8_batch_kernel_name(int M, int K, int B) {
     switch (batch_form(bfp8_ntiles(M), K >> 6, B)) {
         case BatchForm::kPlain: return bfp8_gemv_kernel_name(M, K);
+        case BatchForm::kDot: return "bfp8_gemv_batch_dot_kernel";
         case BatchForm::kCu: return "bfp8_gemv_batch_cu_kernel";
-        case BatchForm::kTile: return "bfp8_gemv_batch_mfma_kernel";
+        case BatchForm::kTile:
+        case BatchForm::kHalf: return "bfp8_gemv_batch_mfma_kernel";
         default: return "bfp8_gemv_batch_span_kernel";
     }
 }
@@ -725,8 +934,23 @@ hipError_t bfp8_launch_gemv_batch(float* Y, const uint32_t* xsplit, const float*
                 hipLaunchKernelGGL((bfp8_gemv_batch_cu_kernel<2, 4>), grid, block, 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
             return hipGetLastError();
         }
+        case BatchForm::kDot:
+            if (B == 2)
+                hipLaunchKernelGGL(bfp8_gemv_batch_dot_kernel<2>, dim3(nt), dim3(256), 0, s, Y, xsplit, xscale, mant, exps, M, K);
+            else
+                hipLaunchKernelGGL(bfp8_gemv_batch_dot_kernel<4>, dim3(nt), dim3(256), 0, s, Y, xsplit, xscale, mant, exps, M, K);
+            return hipGetLastError();
         case BatchForm::kTile:
-            hipLaunchKernelGGL(bfp8_gemv_batch_mfma_kernel, dim3(nt), dim3(256), 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
+            hipLaunchKernelGGL((bfp8_gemv_batch_mfma_kernel<2, 2, 2, 1, 8>), dim3(nt), dim3(256), 0, s, Y, xsplit, xscale,
+                               mant, exps, M, K, B);
+            return hipGetLastError();
+        case BatchForm::kHalf:
+            if (B > 8)  // a workgroup per half of the vectors too: 2 nt units, 16 blocks per 8
+                hipLaunchKernelGGL((bfp8_gemv_batch_mfma_kernel<1, 1, 16 / kMfGroup, 2, 16>), dim3(16 * ((2 * nt + 7) / 8)),
+                                   dim3(256), 0, s, Y, xsplit, xscale, mant, exps, M, K, B);
+            else
+                hipLaunchKernelGGL((bfp8_gemv_batch_mfma_kernel<1, 1, 16 / kMfGroup, 1, 16>), dim3(2 * nt), dim3(256), 0, s,
+                                   Y, xsplit, xscale, mant, exps, M, K, B);
             return hipGetLastError();
         case BatchForm::kSpan: break;
     }

@@ -113,23 +113,27 @@ def test_synthetic_activation_statistics():
     assert np.array_equal(qk.synth_normal(64, 5), qk.synth_normal(64, 5))
 
 
-@pytest.mark.parametrize("M,K,B,name", [(64, 64, 1, "rt_rows_gemv_kernel"), (24577, 1024, 1, "bfp8_gemv_kernel"),
-                                        (3584, 1024, 16, "bfp8_gemv_batch_span_kernel"),
-                                        (19392, 1024, 16, "bfp8_gemv_batch_span_kernel"),
-                                        (19393, 1024, 16, "bfp8_gemv_batch_cu_kernel"),
-                                        (28608, 1024, 8, "bfp8_gemv_batch_span_kernel"),
-                                        (28609, 1024, 8, "bfp8_gemv_batch_cu_kernel"),
-                                        (34752, 64, 4, "bfp8_gemv_batch_span_kernel"),
-                                        (34753, 64, 4, "bfp8_gemv_batch_cu_kernel"),
-                                        (12225, 3584, 16, "bfp8_gemv_batch_mfma_kernel"),
-                                        (12225, 2048, 16, "bfp8_gemv_batch_span_kernel"),
-                                        (200000, 3584, 4, "bfp8_gemv_batch_span_kernel"),
-                                        (64, 63, 4, ""), (64, 4097, 4, ""), (64, 64, 17, ""), (0, 64, 4, "")])
-def test_batch_kernel_names(M, K, B, name):
+@pytest.mark.parametrize("tiles,K,B,name", [
+    (1, 64, 1, "rt_rows_gemv_kernel"), (385, 1024, 1, "bfp8_gemv_kernel"),
+    (256, 512, 2, "span"), (257, 512, 2, "dot"), (768, 512, 2, "dot"), (769, 512, 2, "cu"), (1025, 512, 2, "dot"),
+    (128, 256, 3, "span"), (129, 256, 3, "mfma"), (256, 320, 4, "span"), (512, 320, 4, "mfma"), (513, 320, 4, "cu"),
+    (129, 128, 4, "dot"), (479, 768, 4, "span"), (480, 768, 4, "cu"), (543, 1024, 4, "span"), (544, 1024, 4, "cu"),
+    (1025, 1024, 2, "dot"), (1600, 1024, 2, "cu"), (438, 1088, 2, "span"), (439, 1088, 2, "dot"), (439, 1088, 4, "mfma"),
+    (100000, 2048, 4, "span"), (128, 768, 8, "span"), (129, 768, 8, "mfma"), (256, 1024, 8, "span"), (257, 768, 8, "cu"),
+    (340, 1088, 5, "span"), (341, 1088, 5, "mfma"), (900, 2048, 8, "span"), (901, 2048, 8, "mfma"),
+    (320, 3584, 8, "span"), (321, 3584, 8, "mfma"), (64, 1024, 16, "span"), (65, 1024, 16, "mfma"),
+    (512, 1024, 16, "mfma"), (513, 1024, 16, "cu"), (1024, 1024, 16, "cu"), (1025, 1024, 16, "mfma"), (1281, 1024, 16, "cu"),
+    (128, 1088, 16, "span"), (129, 1088, 16, "mfma"), (128, 4096, 16, "span"), (129, 4096, 16, "mfma"),
+    (208, 4096, 9, "span"), (209, 4096, 9, "mfma"),
+    (1, 63, 4, ""), (1, 4097, 4, ""), (1, 64, 17, ""), (0, 64, 4, "")])
+def test_batch_kernel_names(tiles, K, B, name):
     """The batched GEMV's forms on both sides of the lines between them."""
     import qwen_kernels_gpu as qk
 
-    assert qk.load().bfp8_dev_gemv_batch_kernel_name(M, K, B).decode() == name
+    if name in ("span", "cu", "mfma", "dot"):
+        name = f"bfp8_gemv_batch_{name}_kernel"
+    for M in {64 * tiles, max(64 * tiles - 63, 0)}:
+        assert qk.load().bfp8_dev_gemv_batch_kernel_name(M, K, B).decode() == name
 
 
 def test_device_call_without_gpu_reports_error():

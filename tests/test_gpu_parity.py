@@ -905,13 +905,18 @@ def test_batch_odd_sizes(gpu, torch_mod):
 
 @pytest.mark.parametrize("B,M,K", [(2, 65, 64), (5, 2049, 3584), (7, 100, 1088), (4, 33, 4096), (3, 200, 2112),
                                    (16, 97, 3136), (9, 4100, 2049), (6, 28674, 320), (2, 34815, 128), (16, 19460, 64),
-                                   (5, 26623, 2112), (16, 12290, 2112), (1, 131, 1000)])
+                                   (5, 26623, 2112), (16, 12290, 2112), (1, 131, 1000),
+                                   (2, 16449, 320), (2, 69697, 704), (2, 28673, 1088), (4, 20481, 128),
+                                   (3, 8257, 192), (8, 8257, 512), (8, 8257, 768), (16, 8257, 1024), (13, 65601, 576),
+                                   (5, 21825, 1088), (7, 20545, 2112), (16, 7233, 2112), (14, 8257, 3072),
+                                   (9, 4161, 576), (16, 8191, 1024)])
 def test_batch_dispatch_edges(gpu, torch_mod, B, M, K):
     """Each form of the batched GEMV at the edges of its range: spans of 4, 8,
     12 and 16 blocks per wavefront with the last span partly or wholly empty,
     1, 2 and 4 result slots with idle vectors, row counts just past a tile and
     a half tile, odd last rows, the first tile counts of the many-tile
-    kernels, and one vector (the plain GEMV).  Every exponent byte and block
+    kernels (four tiles, one, half a tile a workgroup; dot products for two and
+    four vectors), and one vector (the plain GEMV).  Every exponent byte and block
     scales from subnormal to huge (no value depends on how the work is split:
     bit-exact against the restatement)."""
     qk = gpu
