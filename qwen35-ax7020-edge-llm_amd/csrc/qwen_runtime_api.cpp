@@ -731,11 +731,13 @@ int chain_launch(const std::vector<FwdLayer*>& layers, int l, int e, const uint1
 }
 
 // After the stream is synchronized: the run's states become the current ones
-// (*ok), or it gave up, and nothing of it counts (!*ok).
+// (*ok), or it gave up or was not to be made (!*ok on entry), and nothing of it
+// counts (!*ok).
 int chain_done(const std::vector<FwdLayer*>& layers, int l, int e, bool* ok) {
     Chain& c = F.chain;
     c.in_flight = false;
-    *ok = __atomic_load_n(&chain_io().status, __ATOMIC_ACQUIRE) == 0;
+    const bool gave_up = __atomic_load_n(&chain_io().status, __ATOMIC_ACQUIRE) != 0;
+    *ok = *ok && !gave_up;
     if (*ok) {
         ++c.done;
         c.next_rest = std::max(c.next_rest - 1, kChainRest);
@@ -746,6 +748,7 @@ int chain_done(const std::vector<FwdLayer*>& layers, int l, int e, bool* ok) {
         }
         return BFP8_OK;
     }
+    if (!gave_up) return BFP8_OK;
     ++c.gave_up;
     HIP_OK(hipMemsetAsync(c.xch.p, 0xff, 2 * (size_t)RT_CHAIN_SET_WORDS * 8, g.stream));
     c.used[0] = c.used[1] = 0;
@@ -758,12 +761,12 @@ int layer_call(const FwdLayer& L, float* h, int slot) {
     const double t0 = g_prof_on ? now_ms() : 0.0;
     int rc;
     const std::vector<FwdLayer*> one{const_cast<FwdLayer*>(&L)};
-    if (chain_ok(one) && chain_takes(h)) {
+    if (chain_ok(one)) {
         if ((rc = states_in(one))) return rc;
         memcpy(chain_io().h_in, h, (size_t)kHidden * 4);
         if ((rc = chain_launch(one, 0, 1, nullptr, 0, 0, nullptr))) return rc;
+        bool ok = chain_takes(h);  // (while the run is under way)
         HIP_OK(hipStreamSynchronize(g.stream));
-        bool ok;
         if ((rc = chain_done(one, 0, 1, &ok))) return rc;
         if (ok) {
             if ((rc = states_out(one))) return rc;
@@ -833,11 +836,12 @@ int token_chain(std::unique_lock<std::mutex>& lk, const std::vector<FwdLayer*>& 
                                     tiled, kVocab, kHidden, 1, 0, g.stream);
         };
         // (an earlier run of the token may have given up, a callback's calls may have changed the table)
-        bool ok = F.chain.rest == 0 && chain_has(layers, l, e) && (embed || chain_takes(h));
+        bool ok = F.chain.rest == 0 && chain_has(layers, l, e);
         if (ok) {
             if (!embed) memcpy(io.h_in, h, hb);
             if ((rc = chain_launch(layers, l, e, embed ? table : nullptr, ntiles, row, last ? fnorm : nullptr))) return rc;
             if (last && (rc = head())) return rc;
+            ok = embed || chain_takes(h);  // (while the run is under way)
             HIP_OK(hipStreamSynchronize(g.stream));
             if ((rc = chain_done(layers, l, e, &ok))) return rc;
         }
