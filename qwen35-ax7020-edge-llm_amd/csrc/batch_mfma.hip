@@ -719,7 +719,7 @@ bfp8_gemv_batch_mfma_kernel(float* __restrict__ Y, const uint32_t* __restrict__ 
 // 8 or 16 vectors whatever B is, so it stands where two vectors (or few blocks)
 // leave it the least to do: us by span / four tiles or one a workgroup / this,
 // weights from HBM: 20480 x 256, B = 2 5.8 / 4.7 / 4.2; 32768 x 512, B = 2 7.7 /
-// 6.3 / 6.3; 65536 x 1088, B = 2 21.5 / 17.2 / 16.3; 81920 x 128, B = 4 24 / 6.6 /
+// 6.3 / 6.3; 65536 x 1088, B = 2 21.5 / 17.2 / 16.3; 81920 x 128, B = 4 15.7 / 6.6 /
 // 5.4.
 constexpr int kBatchChunk = 8;  // blocks per LDS-staged step
 template <int B>
